@@ -216,22 +216,23 @@ struct BuildGeo {
     uint32_t hw, th, bs, log;  // tile half width (AXC: hbs), tile height, COM block size, header shift
 };
 struct BuildOut {
-    double *ax;        // interleaved values / x values (zero filled beforehand)
+    double *ax;        // interleaved values / x values
     uint32_t *plane;   // column of every value slot (AXC: mapx)
     uint32_t *sec;     // AXT row / header words (unused by AXC)
     uint32_t *con;     // AXT con, AXC brp
 };
-// cnt[r] = ceil(rl_r / div) for r < nrows
 // the offsets / column checks of check_kernel OR-ed into *flag (bits 1, 2,
-// 4, 8; the caller clears it first)
-hipError_t build_check(const DevCsr &a, uint32_t *flag, hipStream_t s);
-hipError_t build_count(const DevCsr &a, uint32_t div, uint64_t *cnt, hipStream_t s);
+// 4, 8; the caller clears it first); with cnt, also cnt[r] = ceil(rl_r /
+// div) for r < nrows and cnt[nrows] = 0
+hipError_t build_check(const DevCsr &a, uint32_t div, uint64_t *cnt, uint32_t *flag, hipStream_t s);
 // rocPRIM exclusive scan; tmp == nullptr queries tmp_bytes
 hipError_t build_scan(const uint64_t *in, uint64_t *out, size_t n, void *tmp, size_t &tmp_bytes, hipStream_t s);
 // kind 0: AXC / AXT UNC th == 1, 1: AXT UNC th > 1, 2: COM th == 1, 3: COM th > 1;
-// start = scanned counts (nrows + 1 entries) for kinds 0 and 1
+// start = scanned counts (nrows + 1 entries) for kinds 0 and 1.  Writes every
+// entry of ax (2 nslots), plane (nplane >= nslots), con (nrows + 1) and, where
+// given, sec (nsec).
 hipError_t build_fill(const DevCsr &a, int kind, const uint64_t *start, const BuildGeo &g, const double *x,
-                      const BuildOut &o, hipStream_t s);
+                      const BuildOut &o, uint32_t nslots, uint32_t nplane, uint32_t nsec, hipStream_t s);
 
 hipError_t copy_f64(const double *src, double *dst, size_t n, hipStream_t s);
 hipError_t fill_f64(double *dst, size_t n, double v, hipStream_t s);

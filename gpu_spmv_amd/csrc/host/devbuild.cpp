@@ -12,7 +12,9 @@ using namespace axspmv;
 
 namespace axspmv {
 // Scratch of one device build: the CSR check flag; for the counted layouts
-// the per-row counts, their exclusive scan and rocPRIM's temporary storage.
+// the per-row counts, their exclusive scan (nrows + 2 words: the flag lies
+// in the one after the total, so both come back in one copy) and rocPRIM's
+// temporary storage.
 struct BuildScratch {
     uint32_t *flag = nullptr;
     uint64_t *cnt = nullptr, *start = nullptr;
@@ -69,7 +71,7 @@ struct Scratch {
 // w: the build's scratch (the check flag; for kinds 0 and 1 the counts, their
 // scan and the scan's temporary storage).  own = true allocates the output
 // arrays into f; own = false fills the caller's arrays in f, whose lengths
-// must be the layout's.  Device memory is cleared with fill kernels.
+// must be the layout's.  The fill writes every entry of the outputs.
 int run_build(const axspmv_dcsr *a, const double *d_x, int kind, const launch::BuildGeo &g, bool axc,
               hipStream_t s, axspmv_dfmt *f, const BuildScratch &w, bool own) {
     const uint32_t n = a->nrows;
@@ -77,25 +79,24 @@ int run_build(const axspmv_dcsr *a, const double *d_x, int kind, const launch::B
     const uint64_t ths = uint64_t(g.hw) * g.th;
     Events ev;
     HIP_TRY(ev.create(), "dev build: events");
-    uint64_t total = 0;
-    float ms_scan = 0.0f;
     // the CSR is checked on the device; its flag comes back with the scan
     // total, before anything reads col / val through the offsets
-    uint32_t flag = 0;
+    uint64_t back[2] = {0, 0};  // total, flag (low half)
+    float ms_scan = 0.0f;
     HIP_TRY(launch::fill_u32(w.flag, 1, 0u, s), "dev build: clear");
-    HIP_TRY(launch::build_check(dc, w.flag, s), "dev build: check");
+    HIP_TRY(hipEventRecord(ev.e[0], s), "dev build: event");
+    HIP_TRY(launch::build_check(dc, kind == 0 ? g.hw : g.th, kind <= 1 ? w.cnt : nullptr, w.flag, s), "dev build: check");
     if (kind <= 1) {
         size_t tmp_bytes = w.tmp_bytes;
-        // counts of rows 0 .. n-1; the scan's n + 1st input is 0
-        HIP_TRY(launch::fill_u32(reinterpret_cast<uint32_t *>(w.cnt + n), 2, 0u, s), "dev build: clear");
-        HIP_TRY(hipEventRecord(ev.e[0], s), "dev build: event");
-        HIP_TRY(launch::build_count(dc, kind == 0 ? g.hw : g.th, w.cnt, s), "dev build: count");
         HIP_TRY(launch::build_scan(w.cnt, w.start, size_t(n) + 1, w.tmp, tmp_bytes, s), "dev build: scan");
         HIP_TRY(hipEventRecord(ev.e[1], s), "dev build: event");
-        HIP_TRY(hipMemcpyAsync(&total, w.start + n, 8, hipMemcpyDeviceToHost, s), "dev build: total");
+        HIP_TRY(hipMemcpyAsync(back, w.start + n, 16, hipMemcpyDeviceToHost, s), "dev build: total");
+    } else {
+        HIP_TRY(hipMemcpyAsync(back + 1, w.flag, 4, hipMemcpyDeviceToHost, s), "dev build: check flag");
     }
-    HIP_TRY(hipMemcpyAsync(&flag, w.flag, 4, hipMemcpyDeviceToHost, s), "dev build: check flag");
     HIP_TRY(hipStreamSynchronize(s), "dev build: sync");
+    const uint64_t total = back[0];
+    const uint32_t flag = uint32_t(back[1]);
     if (flag)
         return fail(AXSPMV_E_INVALID, "dev build: invalid device CSR:%s%s%s%s", flag & 1 ? " row offsets decrease;" : "",
                     flag & 2 ? " row[0] != 0;" : "", flag & 4 ? " row[nrows] != nnz;" : "",
@@ -141,14 +142,10 @@ int run_build(const axspmv_dcsr *a, const double *d_x, int kind, const launch::B
                 hipMalloc(&f->con, 4ull * (n + 1)) != hipSuccess ||
                 (!axc && hipMalloc(&f->sec, 4 * (lenSEC ? lenSEC : 1)) != hipSuccess)))
         return fail(AXSPMV_E_NOMEM, "dev build: device allocation failed");
-    // zero fill: padding slots, headers and con[nrows] of the th > 1 layouts
-    HIP_TRY(launch::fill_f64(f->ax, lenAX, 0.0, s), "dev build: clear");
-    HIP_TRY(launch::fill_u32(f->plane, nplane, 0u, s), "dev build: clear");
-    HIP_TRY(launch::fill_u32(f->con, size_t(n) + 1, 0u, s), "dev build: clear");
-    if (!axc) HIP_TRY(launch::fill_u32(f->sec, lenSEC, 0u, s), "dev build: clear");
     HIP_TRY(hipEventRecord(ev.e[2], s), "dev build: event");
     const launch::BuildOut o{f->ax, f->plane, axc ? nullptr : f->sec, f->con};
-    HIP_TRY(launch::build_fill(dc, kind, w.start, g, d_x, o, s), "dev build: fill");
+    HIP_TRY(launch::build_fill(dc, kind, w.start, g, d_x, o, uint32_t(lenAX / 2), uint32_t(nplane), uint32_t(lenSEC), s),
+            "dev build: fill");
     HIP_TRY(hipEventRecord(ev.e[3], s), "dev build: event");
     HIP_TRY(hipStreamSynchronize(s), "dev build: sync");
     float ms_fill = 0.0f;
@@ -229,13 +226,15 @@ extern "C" int axspmv_dev_build_axt(const axspmv_dcsr *a, const double *d_x, uin
     hipStream_t s = static_cast<hipStream_t>(stream);
     Scratch scratch;
     BuildScratch w;
-    w.flag = static_cast<uint32_t *>(scratch.alloc(4));
     if (kind <= 1) {
         AX_TRY(scan_tmp_bytes(a->nrows, s, &w.tmp_bytes));
-        w.cnt = static_cast<uint64_t *>(scratch.alloc(8ull * (a->nrows + 1)));
-        w.start = static_cast<uint64_t *>(scratch.alloc(8ull * (a->nrows + 1)));
+        w.cnt = static_cast<uint64_t *>(scratch.alloc(8 * (size_t(a->nrows) + 1)));
+        w.start = static_cast<uint64_t *>(scratch.alloc(8 * (size_t(a->nrows) + 2)));
         w.tmp = scratch.alloc(w.tmp_bytes);
         if (!w.cnt || !w.start || !w.tmp) return fail(AXSPMV_E_NOMEM, "dev build: scratch allocation failed");
+        w.flag = reinterpret_cast<uint32_t *>(w.start + a->nrows + 1);
+    } else {
+        w.flag = static_cast<uint32_t *>(scratch.alloc(4));
     }
     if (!w.flag) return fail(AXSPMV_E_NOMEM, "dev build: scratch allocation failed");
     auto *f = host_calloc<axspmv_dfmt>(1);
@@ -259,11 +258,11 @@ extern "C" int axspmv_dev_build_axc(const axspmv_dcsr *a, const double *d_x, uin
     Scratch scratch;
     BuildScratch w;
     AX_TRY(scan_tmp_bytes(a->nrows, s, &w.tmp_bytes));
-    w.flag = static_cast<uint32_t *>(scratch.alloc(4));
-    w.cnt = static_cast<uint64_t *>(scratch.alloc(8ull * (a->nrows + 1)));
-    w.start = static_cast<uint64_t *>(scratch.alloc(8ull * (a->nrows + 1)));
+    w.cnt = static_cast<uint64_t *>(scratch.alloc(8 * (size_t(a->nrows) + 1)));
+    w.start = static_cast<uint64_t *>(scratch.alloc(8 * (size_t(a->nrows) + 2)));
     w.tmp = scratch.alloc(w.tmp_bytes);
-    if (!w.flag || !w.cnt || !w.start || !w.tmp) return fail(AXSPMV_E_NOMEM, "dev build: scratch allocation failed");
+    if (!w.cnt || !w.start || !w.tmp) return fail(AXSPMV_E_NOMEM, "dev build: scratch allocation failed");
+    w.flag = reinterpret_cast<uint32_t *>(w.start + a->nrows + 1);
     auto *f = host_calloc<axspmv_dfmt>(1);
     if (!f) return AXSPMV_E_NOMEM;
     f->format = AXSPMV_FMT_AXC;
@@ -289,24 +288,26 @@ int dev_build_axt_into(const axspmv_dcsr *a, const double *d_x, uint32_t bs, uin
     uint32_t log = 0;
     char name[48];
     AX_TRY(axt_params(a, bs, thw, th, mode, &kind, &log, name, sizeof name));
-    // flag | counts | starts | scan storage, each at a 256-byte boundary
+    // counts | starts and flag | scan storage, each at a 256-byte boundary
+    // (COM layouts: the flag alone)
     auto up = [](size_t v) { return (v + 255) & ~size_t(255); };
     BuildScratch w;
+    w.flag = reinterpret_cast<uint32_t *>(scratch);
     size_t need = 256;
     if (kind <= 1) {
         AX_TRY(scan_tmp_bytes(a->nrows, s, &w.tmp_bytes));
-        const size_t cnt_bytes = up(8 * (size_t(a->nrows) + 1));
-        w.cnt = reinterpret_cast<uint64_t *>(scratch + need);
-        w.start = reinterpret_cast<uint64_t *>(scratch + need + cnt_bytes);
-        w.tmp = scratch + need + 2 * cnt_bytes;
-        need += 2 * cnt_bytes + up(w.tmp_bytes);
+        const size_t cnt_bytes = up(8 * (size_t(a->nrows) + 1)), start_bytes = up(8 * (size_t(a->nrows) + 2));
+        w.cnt = reinterpret_cast<uint64_t *>(scratch);
+        w.start = reinterpret_cast<uint64_t *>(scratch + cnt_bytes);
+        w.tmp = scratch + cnt_bytes + start_bytes;
+        w.flag = reinterpret_cast<uint32_t *>(w.start + a->nrows + 1);
+        need += 2 * cnt_bytes + up(w.tmp_bytes);  // start_bytes <= cnt_bytes + 256
     }
     if (need > cap)
         return fail(AXSPMV_E_UNSUPPORTED,
                     "dev_build_axt_noalloc: %u rows need %zu bytes of scratch, the static workspace holds %zu "
                     "(axspmv_dev_build_axt has no such limit)",
                     a->nrows, need, cap);
-    w.flag = reinterpret_cast<uint32_t *>(scratch);
     // *f changes only when the build succeeds
     axspmv_dfmt g = *f;
     set_axt_header(&g, name, bs, thw, th, mode, log);

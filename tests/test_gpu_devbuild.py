@@ -6,10 +6,13 @@ cudaSpmv.cu:1004-1062) with kernels.  Bar: every array equal, bit for bit,
 to the host builder's (which test_builders.py pins to the reference's own
 builders compiled from its sources, and to the oracle's restatement).
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import gpu_spmv_amd as ax
+from gpu_spmv_amd import _lib as L
 from conftest import FIXTURES, FixtureMatrix
 
 pytestmark = pytest.mark.gpu
@@ -98,3 +101,57 @@ def test_dev_build_checks_the_device_csr(case, row, col, ncols, msg):
         ax.dev_build_axt(m, None, 256, 64, 1, ax.AXT_COM)
     with pytest.raises(ax.AxspmvError, match="invalid device CSR:.*" + msg):
         ax.dev_build_axc(m, None, 4)
+
+
+def _edge_matrix(extra):
+    """A long row, a run of empty rows longer than two 64-wide search steps,
+    short rows, a last row that ends the slots at 256 k + extra."""
+    lens = [700, 0, 3] + [0] * 5000 + [1, 2, 5, 4, 1] * 13 + [0] * 70 + [2600]
+    total = sum(lens)
+    lens.append((-total) % 256 + 256 + extra)
+    lens += [0] * 3
+    rng = np.random.default_rng(17)
+    row = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    col = np.concatenate([np.sort(rng.choice(6001, n, replace=False)) for n in lens]).astype(np.uint32)
+    return ax.CsrMatrix(row, col, rng.standard_normal(col.size), ncols=6001)
+
+
+@pytest.mark.parametrize("extra", [-1, 0, 1])
+@pytest.mark.parametrize("bs,thw,th,mode", [(256, 1, 1, ax.AXT_UNC), (256, 7, 1, ax.AXT_UNC), (256, 16, 5, ax.AXT_UNC),
+                                            (16, 64, 1, ax.AXT_COM), (256, 24, 8, ax.AXT_COM), (0, 32, 0, None), (0, 7, 0, None)])
+def test_fill_slot_edges(extra, bs, thw, th, mode):
+    """One lane per slot: slot counts around a wave's 256, rows found by
+    search across long empty runs, hw that is and is not a power of two."""
+    m = _edge_matrix(extra)
+    x = ax.uniform(44, m.ncols)
+    if mode is None:
+        h, d = ax.build_axc(m, x, thw), ax.dev_build_axc(m, x, thw)
+        pairs = (("ax", "ax"), ("con", "brp"), ("plane", "mapx"))
+    else:
+        h, d = ax.build_axt(m, x, bs, thw, th, mode), ax.dev_build_axt(m, x, bs, thw, th, mode)
+        pairs = (("ax", "ax"), ("con", "con"), ("sec", "sec"), ("plane", "cplane"))
+    for a, b in pairs:
+        assert d[a].tobytes() == h[b].tobytes(), a
+
+
+def test_dev_build_with_columns_off_16_bytes():
+    """The column check's plain loads (a device CSR whose col is 4-byte aligned)."""
+    m = MATS["plaw512"]
+    shifted = np.concatenate([np.zeros(1, np.uint32), m.col])
+    dcol = ax.DeviceBuffer.from_array(shifted)
+    drow, dval = ax.DeviceBuffer.from_array(m.row), ax.DeviceBuffer.from_array(m.val)
+    for bad in (False, True):
+        if bad:
+            shifted[-1] = m.ncols
+            dcol.upload(shifted)
+        a = L.Dcsr(m.nrows, m.ncols, m.nnz, 0, drow.ptr, dcol.ptr + 4, dval.ptr)
+        out = C.POINTER(L.Dfmt)()
+        if bad:
+            with pytest.raises(ax.AxspmvError, match="column >= ncols"):
+                L.call("axspmv_dev_build_axt", C.byref(a), None, 256, 4, 1, ax.AXT_UNC, None, C.byref(out))
+            continue
+        L.call("axspmv_dev_build_axt", C.byref(a), None, 256, 4, 1, ax.AXT_UNC, None, C.byref(out))
+        plane = np.empty(out.contents.lenMAPX, np.uint32)
+        L.call("axspmv_memcpy_d2h", plane.ctypes.data, out.contents.plane, plane.nbytes, None)
+        L.load().axspmv_dfmt_free(out)
+        assert np.array_equal(plane, ax.build_axt(m, ax.uniform(1, m.ncols), 256, 4, 1, ax.AXT_UNC)["cplane"])
