@@ -79,6 +79,8 @@ struct SpmmArgs {
     const uint32_t *col;
     const uint32_t *longrows;
     uint32_t nlong;
+    uint32_t ncols;
+    uint32_t xcd;  // 1: XCD i takes the i-th eighth of the rows
 };
 // kt (k-tile) in {8, 16, 32, 64}
 hipError_t spmm(const SpmmArgs &a, uint32_t k, uint32_t kt, const double *X, double *Y, hipStream_t s);

@@ -44,6 +44,8 @@ enum : int {
     DPP_ROW_HALF_MIRROR = 0x141,
     DPP_QUAD_1032 = 0xB1,  // quad_perm [1,0,3,2]
     DPP_QUAD_2301 = 0x4E,  // quad_perm [2,3,0,1]
+    DPP_QUAD_BCAST0 = 0x00,  // quad_perm [j,j,j,j] = j * 0x55
+    DPP_ROW_NEWBCAST0 = 0x150,  // lane j of each 16-lane row = 0x150 + j
 };
 
 // Lanes whose DPP source is out of range or whose row is masked keep `old`.
@@ -57,6 +59,43 @@ __device__ __forceinline__ double dpp_f64(double old, double v) {
     const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(v), CTRL, ROWMASK, 0xf, false);
     const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(v), CTRL, ROWMASK, 0xf, false);
     return __hiloint2double(hi, lo);
+}
+
+// f(integral constant 0), ..., f(integral constant N - 1): the DPP control of
+// step j is a constant
+template <int J>
+struct StaticInt {
+    static constexpr int value = J;
+};
+template <int N, int J = 0, class F>
+__device__ __forceinline__ void static_for(F &&f) {
+    if constexpr (J < N) {
+        f(StaticInt<J>{});
+        static_for<N, J + 1>(f);
+    }
+}
+
+// The value of lane J of the lane's aligned group of G lanes (G = 4, 8 or
+// 16), in every lane of the group.
+template <int G, int J>
+__device__ __forceinline__ uint32_t group_bcast_u32(uint32_t v) {
+    static_assert((G == 4 || G == 8 || G == 16) && J < G, "group_bcast");
+    const int x = int(v);
+    if constexpr (G == 4) return uint32_t(__builtin_amdgcn_update_dpp(x, x, DPP_QUAD_BCAST0 + J * 0x55, 0xf, 0xf, false));
+    else if constexpr (G == 16) return uint32_t(__builtin_amdgcn_update_dpp(x, x, DPP_ROW_NEWBCAST0 + J, 0xf, 0xf, false));
+    else {  // lanes 0-7 of a row (banks 0, 1) take lane J, lanes 8-15 lane 8 + J
+        const int lo = __builtin_amdgcn_update_dpp(x, x, DPP_ROW_NEWBCAST0 + J, 0xf, 0x3, false);
+        return uint32_t(__builtin_amdgcn_update_dpp(lo, x, DPP_ROW_NEWBCAST0 + 8 + J, 0xf, 0xc, false));
+    }
+}
+template <int G, int J>
+__device__ __forceinline__ float group_bcast(float v) {
+    return __uint_as_float(group_bcast_u32<G, J>(__float_as_uint(v)));
+}
+template <int G, int J>
+__device__ __forceinline__ double group_bcast(double v) {
+    return __hiloint2double(int(group_bcast_u32<G, J>(uint32_t(__double2hiint(v)))),
+                            int(group_bcast_u32<G, J>(uint32_t(__double2loint(v)))));
 }
 
 __device__ __forceinline__ uint32_t lane_id() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }

@@ -122,6 +122,17 @@ namespace {
 // Rows longer than this many slots are done one wave per row by SpMM.
 constexpr uint32_t SPMM_LONG = 256;
 
+// SpMM gives XCD i the i-th eighth of the rows (neighbouring rows of a mesh
+// read the same X rows: one L2 instead of eight) where no eighth holds much
+// more than its share of the entries; rows sorted by length, say, are dealt
+// out round-robin instead.
+uint32_t spmm_by_eighths(const axspmv_csr *a) {
+    const uint64_t n = a->nrows;
+    uint64_t most = 0;
+    for (uint64_t i = 0; i < 8; ++i) most = std::max<uint64_t>(most, a->row[(i + 1) * n / 8] - a->row[i * n / 8]);
+    return 8 * most <= uint64_t(a->nnz) + a->nnz / 8 ? 1 : 0;
+}
+
 // Row-contiguous layouts: record where each row starts (device array
 // `first`, uploaded here unless it is the CSR row pointer itself) for SpMM
 // and the value gradient.
@@ -144,7 +155,7 @@ int setup_rowwise(Plan &p, const axspmv_csr *a, const uint32_t *d_first, const v
     if (!lr) return AXSPMV_E_NOMEM;
     AX_TRY(p.upload(lr, longrows.data(), 4 * longrows.size(), s));
     p.spmm = launch::SpmmArgs{a->nrows, p.o.vtype, SPMM_LONG, p.d_first, p.d_rowptr, d_val, d_col, lr,
-                              uint32_t(longrows.size())};
+                              uint32_t(longrows.size()), a->ncols, spmm_by_eighths(a)};
     p.rowwise = true;
     return AXSPMV_OK;
 }

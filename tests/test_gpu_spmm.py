@@ -1,0 +1,80 @@
+"""GPU: SpMM kernels at the sizes where they can go wrong -- row lengths
+around a batch of entries and around the long-row limit, odd and even numbers
+of right-hand sides, operands off 16 bytes, X beyond 32-bit byte offsets --
+against the oracle's spmm.  Tolerance: FP64 sums of at most 2600 products,
+1e-12 of the largest entry as in the other parity tests."""
+import numpy as np
+import pytest
+
+import gpu_spmv_amd as ax
+from conftest import rel_err
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-12
+
+
+def edge_rows():
+    lens = [0, 1, 7, 8, 9, 15, 16, 17, 0, 31, 32, 33, 255, 256, 257, 271, 272, 273, 2600, 0, 4] + [3, 5, 8, 16, 2] * 20
+    rng = np.random.default_rng(3)
+    row = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    n = 3001
+    col = np.concatenate([np.sort(rng.choice(n, k, replace=False)) for k in lens]).astype(np.uint32)
+    return ax.CsrMatrix(row, col, rng.standard_normal(col.size), ncols=n)
+
+
+EDGE = edge_rows()
+ROWWISE = [(ax.FMT_AXT, dict(thw=4)), (ax.FMT_CSR, {}), (ax.FMT_AXC, dict(hbs=2, vtype=ax.F32))]
+
+
+def spmm(plan, m, X, off=0):
+    """Y of one call with X and Y `off` doubles past their buffers' start;
+    the words before and after Y must stay untouched."""
+    k = X.shape[1]
+    n = m.nrows * k
+    dX = ax.DeviceBuffer.from_array(np.concatenate([np.full(off, np.nan), X.ravel()]))
+    dY = ax.DeviceBuffer.from_array(np.full(n + off + 1, np.nan))
+    plan.spmm(k, dX.ptr + 8 * off, dY.ptr + 8 * off)
+    ax._lib.call("axspmv_device_sync")
+    Y = dY.download(np.float64, n + off + 1)
+    assert np.isnan(Y[-1]) and np.all(np.isnan(Y[:off]))
+    return Y[off:-1].reshape(m.nrows, k)
+
+
+def f32_values(m, kw):
+    if kw.get("vtype") != ax.F32:
+        return m
+    return ax.CsrMatrix(m.row, m.col, m.val.astype(np.float32).astype(np.float64), ncols=m.ncols)
+
+
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("k,kt", [(1, 0), (2, 0), (7, 0), (8, 0), (16, 0), (17, 16), (18, 16), (32, 0), (33, 32), (64, 0), (66, 64)])
+@pytest.mark.parametrize("fmt,kw", ROWWISE, ids=["axt", "csr", "axc_f32"])
+def test_rowwise_edges(fmt, kw, k, kt, off):
+    X = ax.uniform(70 + k, EDGE.ncols * k).reshape(EDGE.ncols, k)
+    Y = spmm(ax.Plan(EDGE, fmt, ktile=kt, **kw), EDGE, X, off)
+    assert rel_err(orc.spmm(f32_values(EDGE, kw), X), Y) <= TOL
+
+
+@pytest.mark.parametrize("fmt,kw", ROWWISE, ids=["axt", "csr", "axc_f32"])
+def test_x_of_4_gb(fmt, kw):
+    """X of 4.3 GB: row offsets beyond 32 bits."""
+    ncols, k = (1 << 23) + 5, 64
+    rng = np.random.default_rng(8)
+    lens = np.array([0, 5, 300, 40, 17])
+    row = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    col = np.concatenate([np.sort(rng.choice(ncols, n, replace=False)) for n in lens]).astype(np.uint32)
+    col[-1] = ncols - 1
+    m = ax.CsrMatrix(row, col, rng.standard_normal(col.size), ncols=ncols)
+    # only the X rows that the matrix reads are filled
+    used = np.unique(col)
+    X = ax.uniform(9, used.size * k).reshape(used.size, k)
+    dX = ax.DeviceBuffer(8 * ncols * k)
+    for c, xr in zip(used, X):
+        ax._lib.call("axspmv_memcpy_h2d", dX.ptr + 8 * k * int(c), xr.ctypes.data, xr.nbytes, None)
+    ax._lib.call("axspmv_device_sync")
+    dY = ax.DeviceBuffer.from_array(np.full(m.nrows * k, np.nan))
+    ax.Plan(m, fmt, **kw).spmm(k, dX, dY)
+    xs, val = X[np.searchsorted(used, col)], f32_values(m, kw).val
+    ref = np.stack([val[a:b] @ xs[a:b] for a, b in zip(row[:-1].astype(int), row[1:].astype(int))])
+    assert rel_err(ref, dY.download(np.float64, m.nrows * k).reshape(m.nrows, k)) <= TOL
