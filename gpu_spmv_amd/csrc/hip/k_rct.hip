@@ -24,6 +24,8 @@
 // LDS adds (ds_add_f64) make the order of the additions inside a row
 // nondeterministic; the result stays within the FP64 tolerance of the
 // left-to-right CPU sum.
+#include <type_traits>
+
 #include "launch.hpp"
 #include "wave64.hpp"
 
@@ -343,14 +345,56 @@ __global__ void __launch_bounds__(1024) rct_vbar_kernel(RctArgs a, const double 
     }
 }
 
-// SpMM: Y[:, k0 .. k0 + KT) (+)= A X[:, k0 .. k0 + KT) over one tile.  KT
-// lanes serve one entry (one coalesced KT x 8-byte gather of the entry's X
-// row); the tile's rows x KT sums stay in LDS (ds_add_f64) and go to Y at
+// SpMM: Y[:, k0 .. k0 + KT) (+)= A X[:, k0 .. k0 + KT) over one tile.  A
+// group of GL lanes serves one entry at a time, V neighbouring right-hand
+// sides per lane (KT = GL * V; one contiguous KT x 8-byte read of the entry's
+// X row); the tile's rows x KT sums stay in LDS (ds_add_f64) and go to Y at
 // the end: stored with one slice, added with FP64 atomics (Y cleared first)
 // with several.
-template <class VT, int KEY, int KT>
+//
+// Values and keys are loaded and decoded a batch at a time, one entry per
+// lane, and handed to the group by DPP: with every lane of a group loading
+// its entry's value, key and base, the vector L1 spent three of its four
+// requests per entry on them.  Power-law matrices, FP64: 600,000 rows, k = 8,
+// 1024-row tiles 259 -> 222 us (4 slices 209 -> 184); 400,003 rows, k = 32,
+// 256-row tiles 468 -> 323 us; the 64^3 stencil, k = 16, 512-row tiles 169 ->
+// 57 us.  What is left on the power-law ones are the X rows that miss L2 (one
+// 128-byte line per entry, 5.5 TB/s from the Infinity Cache).  A batch's X
+// loads go out together; the next batch's values and keys are in flight
+// behind them.  X rows are addressed by 32-bit byte offsets, or (WIDE: X of
+// 4 GB and more) by their column.
+//
+// LDS layout: sum (row, right-hand side l V + v) sits at row KT + v GL + l,
+// and odd groups add their second right-hand side first, so the groups of
+// one ds_add_f64 spread over both halves of their rows' banks.
+template <class VT, int KEY, int GL, bool WIDE>
+struct SpmmBatch {
+    static constexpr int ROW = GL < 16 ? GL : 16;  // lanes that share a batch: wider groups load it once per 16
+    static constexpr int E = ROW == 4 ? 2 : 1;     // entries per lane
+    static constexpr int B = ROW * E;
+    VT v[E];
+    uint32_t c[E], r[E];  // X row (byte offset, or column), tile row
+    __device__ __forceinline__ void load(const RctEntries<VT, KEY> &ent, uint32_t e0, uint32_t end, uint32_t k) {
+        const uint32_t i = e0 + threadIdx.x % ROW;
+#pragma unroll
+        for (int u = 0; u < E; ++u)
+            if (i + u * ROW < end) {
+                v[u] = ent.val[i + u * ROW];
+                uint32_t cc;
+                ent.at(i + u * ROW, cc, r[u]);
+                c[u] = WIDE ? cc : cc * k * 8;
+            }
+    }
+};
+
+template <class VT, int KEY, int GL, int V, bool WIDE>
 __global__ void __launch_bounds__(1024) rct_spmm_kernel(RctArgs a, uint32_t k, uint32_t k0,
                                                         const double *__restrict__ X, double *__restrict__ Y) {
+    using namespace axspmv::dev;
+    using Batch = SpmmBatch<VT, KEY, GL, WIDE>;
+    typedef double vec __attribute__((ext_vector_type(V)));
+    using XV = std::conditional_t<V == 1, double, vec>;
+    constexpr uint32_t KT = GL * V, B = Batch::B, ROW = Batch::ROW, STEP = 8;
     extern __shared__ double acc[];
     TileOf tile;
     if (!tile.from(a, blockIdx.x)) return;
@@ -361,57 +405,100 @@ __global__ void __launch_bounds__(1024) rct_spmm_kernel(RctArgs a, uint32_t k, u
     const uint32_t t = tile.rb * a.S + tile.s;
     const uint32_t beg = a.tile_ptr[t], end = a.tile_ptr[t + 1];
     const RctEntries<VT, KEY> ent(a, row0);
-    const uint32_t j = tid % KT, nsub = nt / KT;  // nt is a multiple of 64
-    const bool live = k0 + j < k;                 // the last k-tile may be partial
-    const double *__restrict__ xj = X + k0 + j;
-    constexpr int U = 4;
-    uint32_t e = beg + tid / KT;
-    for (; e + (U - 1) * nsub < end; e += U * nsub) {
-        uint32_t c[U], r[U];
-        double v[U], xv[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) ent.load(e + u * nsub, c[u], r[u], v[u]);
-#pragma unroll
-        for (int u = 0; u < U; ++u) xv[u] = live ? xj[size_t(c[u]) * k] : 0.0;
-#pragma unroll
-        for (int u = 0; u < U; ++u) atomicAdd(&acc[r[u] * KT + j], v[u] * xv[u]);
-    }
-    for (; e < end; e += nsub) {
-        uint32_t c, r;
-        double v;
-        ent.load(e, c, r, v);
-        const double xv = live ? xj[size_t(c) * k] : 0.0;
-        atomicAdd(&acc[r * KT + j], v * xv);
+    const uint32_t l = tid % GL, g = tid / GL, chunk = nt / GL * B;  // nt is a multiple of 64
+    // a lane past the last right-hand side (a partial k-tile) works on the
+    // first one's X and on sums of its own that are not stored
+    const uint32_t kx = k0 + l * V < k ? k0 + l * V : 0;
+    double *const al = acc + l;
+    auto work = [&](const Batch &b, uint32_t left) {
+        static_for<B / STEP ? B / STEP : 1>([&](auto H) {
+            constexpr int N = B < STEP ? B : STEP, j0 = H.value * N;
+            XV xv[N];
+            static_for<N>([&](auto J) {
+                constexpr int j = j0 + J.value;
+                const uint32_t c = group_bcast_u32<ROW, j % ROW>(b.c[j / ROW]);
+                if (uint32_t(j) < left) {
+                    if constexpr (WIDE) xv[J.value] = *reinterpret_cast<const XV *>(X + size_t(c) * k + kx);
+                    else xv[J.value] = *reinterpret_cast<const XV *>(reinterpret_cast<const char *>(X) + (c + kx * 8));
+                }
+            });
+            __builtin_amdgcn_sched_barrier(0);
+            static_for<N>([&](auto J) {
+                constexpr int j = j0 + J.value;
+                const double v = double(group_bcast<ROW, j % ROW>(b.v[j / ROW]));
+                const uint32_t r = group_bcast_u32<ROW, j % ROW>(b.r[j / ROW]) * KT;
+                if (uint32_t(j) < left) {
+                    if constexpr (V == 1) {
+                        atomicAdd(al + r, v * xv[J.value]);
+                    } else {
+                        const double p0 = v * xv[J.value].x, p1 = v * xv[J.value].y;
+                        const uint32_t o = g & 1 ? GL : 0;
+                        atomicAdd(al + r + o, g & 1 ? p1 : p0);
+                        atomicAdd(al + r + (GL - o), g & 1 ? p0 : p1);
+                    }
+                }
+            });
+        });
+    };
+    uint32_t e = beg + g * B;
+    if (e < end) {
+        Batch b;
+        b.load(ent, e, end, k);
+        for (; e + chunk < end; e += chunk) {
+            Batch n;
+            n.load(ent, e + chunk, end, k);
+            work(b, B);  // every batch but a group's last is whole
+            b = n;
+        }
+        work(b, end - e);
     }
     __syncthreads();
-    for (uint32_t q = tid; q < rows * KT; q += nt) {
-        const uint32_t rr = q / KT, jj = q % KT;
-        if (k0 + jj >= k) continue;
-        double *out = Y + size_t(row0 + rr) * k + k0 + jj;
-        if (a.S == 1)
-            *out = acc[q];
-        else
-            unsafeAtomicAdd(out, acc[q]);
+    if (a.S == 1) {
+        for (uint32_t q = tid; q < rows * GL; q += nt) {
+            const uint32_t rr = q / GL, ll = q % GL;
+            if (k0 + ll * V >= k) continue;
+            const double *s = acc + rr * KT + ll;
+            double *out = Y + size_t(row0 + rr) * k + k0 + ll * V;
+            if constexpr (V == 1) *out = *s;
+            else *reinterpret_cast<XV *>(out) = XV{s[0], s[GL]};
+        }
+    } else {
+        // one sum per lane, so that the lanes' atomics fall side by side (two
+        // per lane made 4 slices 25 % slower)
+        for (uint32_t q = tid; q < rows * KT; q += nt) {
+            const uint32_t rr = q / KT, jj = q % KT;
+            if (k0 + jj < k) unsafeAtomicAdd(Y + size_t(row0 + rr) * k + k0 + jj, acc[rr * KT + jj % V * GL + jj / V]);
+        }
     }
 }
 
-template <class VT, int KEY>
-hipError_t rct_spmm_vt(const RctArgs &a, uint32_t k, uint32_t kt, const double *X, double *Y, hipStream_t s) {
+template <class VT, int KEY, int V, bool WIDE>
+hipError_t rct_spmm_run(const RctArgs &a, uint32_t k, uint32_t kt, const double *X, double *Y, hipStream_t s) {
     const size_t lds = size_t(a.R) * kt * sizeof(double);
     const uint32_t per = 8 / a.S;
     const unsigned grid = (a.nrb + per - 1) / per * 8;
     for (uint32_t k0 = 0; k0 < k; k0 += kt) {
         switch (kt) {
-            case 8: rct_spmm_kernel<VT, KEY, 8><<<grid, a.block, lds, s>>>(a, k, k0, X, Y); break;
-            case 16: rct_spmm_kernel<VT, KEY, 16><<<grid, a.block, lds, s>>>(a, k, k0, X, Y); break;
-            case 32: rct_spmm_kernel<VT, KEY, 32><<<grid, a.block, lds, s>>>(a, k, k0, X, Y); break;
-            case 64: rct_spmm_kernel<VT, KEY, 64><<<grid, a.block, lds, s>>>(a, k, k0, X, Y); break;
+            case 8: rct_spmm_kernel<VT, KEY, 8 / V, V, WIDE><<<grid, a.block, lds, s>>>(a, k, k0, X, Y); break;
+            case 16: rct_spmm_kernel<VT, KEY, 16 / V, V, WIDE><<<grid, a.block, lds, s>>>(a, k, k0, X, Y); break;
+            case 32: rct_spmm_kernel<VT, KEY, 32 / V, V, WIDE><<<grid, a.block, lds, s>>>(a, k, k0, X, Y); break;
+            case 64: rct_spmm_kernel<VT, KEY, 64 / V, V, WIDE><<<grid, a.block, lds, s>>>(a, k, k0, X, Y); break;
             default: return hipErrorInvalidValue;
         }
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
+}
+
+// Two right-hand sides per lane where every 16-byte access is aligned: k
+// even, X and Y 16-byte aligned (k0 is a multiple of 8).
+template <class VT, int KEY>
+hipError_t rct_spmm_vt(const RctArgs &a, uint32_t k, uint32_t kt, const double *X, double *Y, hipStream_t s) {
+    const bool two = k % 2 == 0 && (reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(Y)) % 16 == 0;
+    const bool wide = uint64_t(a.ncols) * k * 8 >= (1ull << 32);
+    if (wide) return two ? rct_spmm_run<VT, KEY, 2, true>(a, k, kt, X, Y, s) : rct_spmm_run<VT, KEY, 1, true>(a, k, kt, X, Y, s);
+    return two ? rct_spmm_run<VT, KEY, 2, false>(a, k, kt, X, Y, s) : rct_spmm_run<VT, KEY, 1, false>(a, k, kt, X, Y, s);
 }
 
 }  // namespace

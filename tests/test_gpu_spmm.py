@@ -24,6 +24,10 @@ def edge_rows():
 
 
 EDGE = edge_rows()
+BAND = ax.banded(3001, 3, 0.5, seed=6)  # narrow band: 16-bit keys
+RCT = [("packed", EDGE, dict(tile_rows=256)), ("s4", EDGE, dict(tile_rows=200, slices=4)),
+       ("split_f32", EDGE, dict(tile_rows=300, flags=ax.PLAN_RCT_SPLIT, vtype=ax.F32)), ("k16", BAND, dict(tile_rows=128)),
+       ("block64", EDGE, dict(tile_rows=64, block=64))]
 ROWWISE = [(ax.FMT_AXT, dict(thw=4)), (ax.FMT_CSR, {}), (ax.FMT_AXC, dict(hbs=2, vtype=ax.F32))]
 
 
@@ -56,7 +60,16 @@ def test_rowwise_edges(fmt, kw, k, kt, off):
     assert rel_err(orc.spmm(f32_values(EDGE, kw), X), Y) <= TOL
 
 
-@pytest.mark.parametrize("fmt,kw", ROWWISE, ids=["axt", "csr", "axc_f32"])
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("k,kt", [(1, 0), (2, 8), (7, 8), (8, 8), (16, 16), (17, 16), (18, 16), (32, 32), (33, 32), (64, 64), (66, 64)])
+@pytest.mark.parametrize("m,kw", [r[1:] for r in RCT], ids=[r[0] for r in RCT])
+def test_rct_edges(m, kw, k, kt, off):
+    X = ax.uniform(90 + k, m.ncols * k).reshape(m.ncols, k)
+    Y = spmm(ax.Plan(m, ax.FMT_RCT, ktile=kt, **kw), m, X, off)
+    assert rel_err(orc.spmm(f32_values(m, kw), X), Y) <= TOL
+
+
+@pytest.mark.parametrize("fmt,kw", ROWWISE + [(ax.FMT_RCT, dict(tile_rows=4, slices=2))], ids=["axt", "csr", "axc_f32", "rct"])
 def test_x_of_4_gb(fmt, kw):
     """X of 4.3 GB: row offsets beyond 32 bits."""
     ncols, k = (1 << 23) + 5, 64
