@@ -144,40 +144,74 @@ struct RctEntries {
 int key_mode(const RctArgs &a) { return a.key16 ? KEY_DIAG : a.key ? KEY_PACKED : KEY_SPLIT; }
 
 // Tile w of the grid: XCD w % 8 takes slice (w % 8) % S; false for the
-// workgroups past the last row block.
+// workgroups past the last row block.  HV: the heavy rows' tiles come first,
+// block w / 8 and slice w % 8 for the XCD w % 8.
+template <bool HV = false>
 struct TileOf {
-    uint32_t s, rb;
+    uint32_t s, rb, t;  // t: index in storage order
+    uint32_t row0, rows;
+    bool heavy;
     __device__ __forceinline__ bool from(const RctArgs &a, uint32_t w) {
+        heavy = false;
+        if constexpr (HV) {
+            if (w < axspmv::launch::HEAVY_SLICES * a.nhb) {
+                heavy = true;
+                s = w % axspmv::launch::HEAVY_SLICES;
+                rb = w / axspmv::launch::HEAVY_SLICES;
+                t = a.nrb * a.S + w;
+                row0 = a.hb_start[rb];
+                rows = a.hb_start[rb + 1] - row0;
+                return true;
+            }
+            w -= axspmv::launch::HEAVY_SLICES * a.nhb;
+        }
         const uint32_t xcd = w % 8, i = w / 8;
         const uint32_t per = 8 / a.S;  // row-block groups per slice
         s = xcd % a.S;
         rb = i * per + xcd / a.S;
-        return rb < a.nrb;
+        if (rb >= a.nrb) return false;
+        t = rb * a.S + s;
+        row0 = a.rb_start[rb];
+        rows = a.rb_start[rb + 1] - row0;  // <= a.R
+        return true;
+    }
+    // the row of y that the tile's row k adds to or is stored in; false: a
+    // heavy row's place in a row block, nothing to write
+    __device__ __forceinline__ bool out_row(const RctArgs &a, uint32_t k, uint32_t &r) const {
+        r = row0 + k;
+        if constexpr (HV) {
+            if (heavy) r = a.hrows[r];
+            else return !((a.hmask[r >> 5] >> (r & 31)) & 1);
+        }
+        return true;
     }
 };
+
+unsigned rct_grid(const RctArgs &a) {
+    const uint32_t per = 8 / a.S;
+    return (a.nrb + per - 1) / per * 8 + axspmv::launch::HEAVY_SLICES * a.nhb;
+}
 
 // VB: the same product on the plan of A^T, fused with the value gradient of
 // A: vb[e] = xr[row(e)] * x[col(e)] for every entry, in entry order (the
 // tile's xr values sit in LDS after its sums).  With x = r and xr = the
 // forward x, y = A^T r and vb holds r[i] * x[j] for every nonzero A(i, j).
-template <class VT, int KEY, bool VB, bool NT>
+template <class VT, int KEY, bool VB, bool NT, bool HV = false>
 __global__ void __launch_bounds__(1024) rct_kernel(RctArgs a, const double *__restrict__ x, double *__restrict__ y,
                                                    const double *__restrict__ xr, double *__restrict__ vb,
                                                    const double *__restrict__ bvec, double *__restrict__ res) {
     extern __shared__ double yl[];
-    TileOf tile;
+    TileOf<HV> tile;
     if (!tile.from(a, blockIdx.x)) return;  // the whole workgroup leaves together
-    const uint32_t s = tile.s, rb = tile.rb;
     const uint32_t tid = threadIdx.x, nt = blockDim.x;
-    const uint32_t row0 = a.rb_start[rb], rows = a.rb_start[rb + 1] - row0;  // rows <= a.R
+    const uint32_t row0 = tile.row0, rows = tile.rows;
     double *xs = yl + a.R;  // VB: xr of the tile's rows
     for (uint32_t k = tid; k < rows; k += nt) {
         yl[k] = 0.0;
         if constexpr (VB) xs[k] = xr[row0 + k];
     }
     __syncthreads();
-    const uint32_t t = rb * a.S + s;  // tile index in storage order
-    const uint32_t beg = a.tile_ptr[t], end = a.tile_ptr[t + 1];
+    const uint32_t beg = a.tile_ptr[tile.t], end = a.tile_ptr[tile.t + 1];
     const RctEntries<VT, KEY, NT> ent(a, row0);
     // Each lane takes entries in aligned pairs (2q, 2q + 1): a value load
     // moves 16 bytes and a key load 8, and the value gradient (VB) goes out
@@ -294,7 +328,16 @@ __global__ void __launch_bounds__(1024) rct_kernel(RctArgs a, const double *__re
     }
     __syncthreads();
     double *out = y + row0;
-    if (a.S == 1) {
+    if constexpr (HV) {
+        // heavy rows add their slices' sums into y (cleared there, or
+        // everywhere with S > 1); the others as below
+        for (uint32_t k = tid; k < rows; k += nt) {
+            uint32_t r;
+            if (!tile.out_row(a, k, r)) continue;
+            if (tile.heavy || a.S > 1) unsafeAtomicAdd(y + r, yl[k]);
+            else __builtin_nontemporal_store(yl[k], y + r);
+        }
+    } else if (a.S == 1) {
         // non-temporal: y kept in the L2s would take room from the next
         // SpMV's x (the 1024^2 Laplacian: 14.6 -> 13.9 us)
         for (uint32_t k = tid; k < rows; k += nt) {
@@ -303,7 +346,7 @@ __global__ void __launch_bounds__(1024) rct_kernel(RctArgs a, const double *__re
         }
     } else if (a.part && !VB) {
         // the slice's partial vector, read once by the merge: non-temporal
-        double *ps = a.part + size_t(s) * a.nrows + row0;
+        double *ps = a.part + size_t(tile.s) * a.nrows + row0;
         for (uint32_t k = tid; k < rows; k += nt) __builtin_nontemporal_store(yl[k], ps + k);
     } else {
         for (uint32_t k = tid; k < rows; k += nt) unsafeAtomicAdd(out + k, yl[k]);
@@ -317,14 +360,13 @@ template <int KEY>
 __global__ void __launch_bounds__(1024) rct_vbar_kernel(RctArgs a, const double *__restrict__ ybar,
                                                         const double *__restrict__ x, double *__restrict__ vbar) {
     extern __shared__ double yb[];
-    TileOf tile;
+    TileOf<> tile;
     if (!tile.from(a, blockIdx.x)) return;
     const uint32_t tid = threadIdx.x, nt = blockDim.x;
-    const uint32_t row0 = a.rb_start[tile.rb], rows = a.rb_start[tile.rb + 1] - row0;
+    const uint32_t row0 = tile.row0, rows = tile.rows;
     for (uint32_t k = tid; k < rows; k += nt) yb[k] = ybar[row0 + k];
     __syncthreads();
-    const uint32_t t = tile.rb * a.S + tile.s;
-    const uint32_t beg = a.tile_ptr[t], end = a.tile_ptr[t + 1];
+    const uint32_t beg = a.tile_ptr[tile.t], end = a.tile_ptr[tile.t + 1];
     const RctEntries<double, KEY> ent(a, row0);  // columns and rows only
     constexpr int U = 4;
     uint32_t e = beg + tid;
@@ -387,7 +429,7 @@ struct SpmmBatch {
     }
 };
 
-template <class VT, int KEY, int GL, int V, bool WIDE>
+template <class VT, int KEY, int GL, int V, bool WIDE, bool HV>
 __global__ void __launch_bounds__(1024) rct_spmm_kernel(RctArgs a, uint32_t k, uint32_t k0,
                                                         const double *__restrict__ X, double *__restrict__ Y) {
     using namespace axspmv::dev;
@@ -396,19 +438,18 @@ __global__ void __launch_bounds__(1024) rct_spmm_kernel(RctArgs a, uint32_t k, u
     using XV = std::conditional_t<V == 1, double, vec>;
     constexpr uint32_t KT = GL * V, B = Batch::B, ROW = Batch::ROW, STEP = 8;
     extern __shared__ double acc[];
-    TileOf tile;
+    TileOf<HV> tile;
     if (!tile.from(a, blockIdx.x)) return;
     const uint32_t tid = threadIdx.x, nt = blockDim.x;
-    const uint32_t row0 = a.rb_start[tile.rb], rows = a.rb_start[tile.rb + 1] - row0;
+    const uint32_t row0 = tile.row0, rows = tile.rows;
     for (uint32_t q = tid; q < rows * KT; q += nt) acc[q] = 0.0;
     __syncthreads();
-    const uint32_t t = tile.rb * a.S + tile.s;
-    const uint32_t beg = a.tile_ptr[t], end = a.tile_ptr[t + 1];
+    const uint32_t beg = a.tile_ptr[tile.t], end = a.tile_ptr[tile.t + 1];
     const RctEntries<VT, KEY> ent(a, row0);
     const uint32_t l = tid % GL, g = tid / GL, chunk = nt / GL * B;  // nt is a multiple of 64
     // a lane past the last right-hand side (a partial k-tile) works on the
-    // first one's X and on sums of its own that are not stored
-    const uint32_t kx = k0 + l * V < k ? k0 + l * V : 0;
+    // k-tile's first X and on sums of its own that are not stored
+    const uint32_t kx = k0 + l * V < k ? k0 + l * V : k0;
     double *const al = acc + l;
     auto work = [&](const Batch &b, uint32_t left) {
         static_for<B / STEP ? B / STEP : 1>([&](auto H) {
@@ -453,12 +494,13 @@ __global__ void __launch_bounds__(1024) rct_spmm_kernel(RctArgs a, uint32_t k, u
         work(b, end - e);
     }
     __syncthreads();
-    if (a.S == 1) {
+    if (a.S == 1 && !tile.heavy) {
         for (uint32_t q = tid; q < rows * GL; q += nt) {
             const uint32_t rr = q / GL, ll = q % GL;
-            if (k0 + ll * V >= k) continue;
+            uint32_t r;
+            if (k0 + ll * V >= k || !tile.out_row(a, rr, r)) continue;
             const double *s = acc + rr * KT + ll;
-            double *out = Y + size_t(row0 + rr) * k + k0 + ll * V;
+            double *out = Y + size_t(r) * k + k0 + ll * V;
             if constexpr (V == 1) *out = *s;
             else *reinterpret_cast<XV *>(out) = XV{s[0], s[GL]};
         }
@@ -467,22 +509,31 @@ __global__ void __launch_bounds__(1024) rct_spmm_kernel(RctArgs a, uint32_t k, u
         // per lane made 4 slices 25 % slower)
         for (uint32_t q = tid; q < rows * KT; q += nt) {
             const uint32_t rr = q / KT, jj = q % KT;
-            if (k0 + jj < k) unsafeAtomicAdd(Y + size_t(row0 + rr) * k + k0 + jj, acc[rr * KT + jj % V * GL + jj / V]);
+            uint32_t r;
+            if (k0 + jj < k && tile.out_row(a, rr, r))
+                unsafeAtomicAdd(Y + size_t(r) * k + k0 + jj, acc[rr * KT + jj % V * GL + jj / V]);
         }
     }
 }
 
-template <class VT, int KEY, int V, bool WIDE>
+// Y[rows[i], :] = 0: the heavy rows' place before their slices' adds
+__global__ void __launch_bounds__(256) clear_rows_kernel(const uint32_t *__restrict__ rows, uint64_t total, uint32_t k,
+                                                         double *__restrict__ Y) {
+    const uint64_t t = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (t < total) Y[size_t(rows[t / k]) * k + t % k] = 0.0;
+}
+
+template <class VT, int KEY, int V, bool WIDE, bool HV>
 hipError_t rct_spmm_run(const RctArgs &a, uint32_t k, uint32_t kt, const double *X, double *Y, hipStream_t s) {
-    const size_t lds = size_t(a.R) * kt * sizeof(double);
-    const uint32_t per = 8 / a.S;
-    const unsigned grid = (a.nrb + per - 1) / per * 8;
+    const unsigned grid = rct_grid(a);
     for (uint32_t k0 = 0; k0 < k; k0 += kt) {
+        while (kt > 8 && k - k0 <= kt / 2) kt /= 2;  // the last right-hand sides: no wider than they need
+        const size_t lds = size_t(a.R) * kt * sizeof(double);
         switch (kt) {
-            case 8: rct_spmm_kernel<VT, KEY, 8 / V, V, WIDE><<<grid, a.block, lds, s>>>(a, k, k0, X, Y); break;
-            case 16: rct_spmm_kernel<VT, KEY, 16 / V, V, WIDE><<<grid, a.block, lds, s>>>(a, k, k0, X, Y); break;
-            case 32: rct_spmm_kernel<VT, KEY, 32 / V, V, WIDE><<<grid, a.block, lds, s>>>(a, k, k0, X, Y); break;
-            case 64: rct_spmm_kernel<VT, KEY, 64 / V, V, WIDE><<<grid, a.block, lds, s>>>(a, k, k0, X, Y); break;
+            case 8: rct_spmm_kernel<VT, KEY, 8 / V, V, WIDE, HV><<<grid, a.block, lds, s>>>(a, k, k0, X, Y); break;
+            case 16: rct_spmm_kernel<VT, KEY, 16 / V, V, WIDE, HV><<<grid, a.block, lds, s>>>(a, k, k0, X, Y); break;
+            case 32: rct_spmm_kernel<VT, KEY, 32 / V, V, WIDE, HV><<<grid, a.block, lds, s>>>(a, k, k0, X, Y); break;
+            case 64: rct_spmm_kernel<VT, KEY, 64 / V, V, WIDE, HV><<<grid, a.block, lds, s>>>(a, k, k0, X, Y); break;
             default: return hipErrorInvalidValue;
         }
         const hipError_t e = hipGetLastError();
@@ -493,12 +544,21 @@ hipError_t rct_spmm_run(const RctArgs &a, uint32_t k, uint32_t kt, const double 
 
 // Two right-hand sides per lane where every 16-byte access is aligned: k
 // even, X and Y 16-byte aligned (k0 is a multiple of 8).
-template <class VT, int KEY>
-hipError_t rct_spmm_vt(const RctArgs &a, uint32_t k, uint32_t kt, const double *X, double *Y, hipStream_t s) {
+template <class VT, int KEY, bool HV>
+hipError_t rct_spmm_hv(const RctArgs &a, uint32_t k, uint32_t kt, const double *X, double *Y, hipStream_t s) {
     const bool two = k % 2 == 0 && (reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(Y)) % 16 == 0;
     const bool wide = uint64_t(a.ncols) * k * 8 >= (1ull << 32);
-    if (wide) return two ? rct_spmm_run<VT, KEY, 2, true>(a, k, kt, X, Y, s) : rct_spmm_run<VT, KEY, 1, true>(a, k, kt, X, Y, s);
-    return two ? rct_spmm_run<VT, KEY, 2, false>(a, k, kt, X, Y, s) : rct_spmm_run<VT, KEY, 1, false>(a, k, kt, X, Y, s);
+    if (wide)
+        return two ? rct_spmm_run<VT, KEY, 2, true, HV>(a, k, kt, X, Y, s)
+                   : rct_spmm_run<VT, KEY, 1, true, HV>(a, k, kt, X, Y, s);
+    return two ? rct_spmm_run<VT, KEY, 2, false, HV>(a, k, kt, X, Y, s)
+               : rct_spmm_run<VT, KEY, 1, false, HV>(a, k, kt, X, Y, s);
+}
+template <class VT, int KEY>
+hipError_t rct_spmm_vt(const RctArgs &a, uint32_t k, uint32_t kt, const double *X, double *Y, hipStream_t s) {
+    if constexpr (KEY != KEY_DIAG)
+        if (a.nhb) return rct_spmm_hv<VT, KEY, true>(a, k, kt, X, Y, s);
+    return rct_spmm_hv<VT, KEY, false>(a, k, kt, X, Y, s);
 }
 
 }  // namespace
@@ -510,6 +570,11 @@ hipError_t rct_spmm(const RctArgs &a, uint32_t k, uint32_t kt, const double *X, 
     if (!a.nrows || !k) return hipSuccess;
     if (a.S > 1) {
         const hipError_t e = clear_f64(Y, size_t(a.nrows) * k, s);
+        if (e != hipSuccess) return e;
+    } else if (a.nhb) {
+        const uint64_t total = uint64_t(a.nheavy) * k;
+        clear_rows_kernel<<<unsigned((total + 255) / 256), 256, 0, s>>>(a.hrows, total, k, Y);
+        const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
     const int km = key_mode(a);
@@ -524,8 +589,7 @@ hipError_t rct_spmm(const RctArgs &a, uint32_t k, uint32_t kt, const double *X, 
 
 hipError_t rct_vbar(const RctArgs &a, const double *ybar, const double *x, double *vbar, hipStream_t s) {
     if (!a.nrows) return hipSuccess;
-    const uint32_t per = 8 / a.S;
-    const unsigned grid = (a.nrb + per - 1) / per * 8;
+    const unsigned grid = rct_grid(a);
     const size_t lds = size_t(a.R) * sizeof(double);
     switch (key_mode(a)) {
         case KEY_DIAG: rct_vbar_kernel<KEY_DIAG><<<grid, a.block, lds, s>>>(a, ybar, x, vbar); break;
@@ -539,9 +603,7 @@ hipError_t rct(const RctArgs &a, const double *x, double *y, hipStream_t s, hipE
                double *vbar, const double *rb, double *res) {
     if (!a.nrows) return hipSuccess;
     if (vbar) rb = res = nullptr;  // the residual belongs to a forward pass
-    const uint32_t per = 8 / a.S;
-    const uint32_t groups = (a.nrb + per - 1) / per;
-    const unsigned grid = groups * 8;
+    const unsigned grid = rct_grid(a);
     const bool vb = vbar != nullptr;
     const size_t lds = size_t(a.R) * sizeof(double) * (vb ? 2 : 1);
     const bool partials = a.S > 1 && a.part && !vb;
@@ -552,6 +614,9 @@ hipError_t rct(const RctArgs &a, const double *x, double *y, hipStream_t s, hipE
             const hipError_t e = hipEventRecord(mid, s);
             if (e != hipSuccess) return e;
         }
+    } else if (a.nhb) {
+        const hipError_t e = fill_rows(a.hrows, a.nheavy, y, s);
+        if (e != hipSuccess) return e;
     }
     const int km = key_mode(a);
     // the value-gradient sweep too streams with non-temporal loads where the
@@ -560,7 +625,10 @@ hipError_t rct(const RctArgs &a, const double *x, double *y, hipStream_t s, hipE
     // us, one box
 #define AX_RCT_LAUNCH(VT, P)                                                                         \
     do {                                                                                             \
-        if (vb && a.nt_stream)                                                                       \
+        if (P != KEY_DIAG && a.nhb)                                                                  \
+            rct_kernel<VT, P == KEY_DIAG ? KEY_SPLIT : P, false, false, true><<<grid, a.block, lds, s>>>( \
+                a, x, y, xr, vbar, rb, res);                                                         \
+        else if (vb && a.nt_stream)                                                                       \
             rct_kernel<VT, P, true, true><<<grid, a.block, lds, s>>>(a, x, y, xr, vbar, rb, res);   \
         else if (vb)                                                                                 \
             rct_kernel<VT, P, true, false><<<grid, a.block, lds, s>>>(a, x, y, xr, vbar, rb, res);  \
@@ -589,7 +657,7 @@ hipError_t rct(const RctArgs &a, const double *x, double *y, hipStream_t s, hipE
     if (partials) {
         if (e == hipSuccess && mid) e = hipEventRecord(mid, s);
         if (e == hipSuccess) e = part_merge(a.part, a.S, a.nrows, y, s, rb, res);
-    } else if (res && a.S > 1 && e == hipSuccess) {
+    } else if (res && (a.S > 1 || a.nhb) && e == hipSuccess) {
         e = residual(a.nrows, y, rb, res, s);  // after the slices' adds
     }
     return e;

@@ -104,7 +104,7 @@ __global__ void __launch_bounds__(256) spmm_rows_kernel(uint32_t nrows, const ui
     const uint32_t len = rowptr[r + 1] - rowptr[r];
     if (len > long_slots) return;
     const bool on = kc < k;
-    const uint32_t kx = on ? kc : 0;  // a lane past the last right-hand side reads the first and stores nothing
+    const uint32_t kx = on ? kc : blockIdx.y * (GL * V);  // past the last right-hand side: a live lane's X, nothing stored
     uint32_t q = first[r], left = len;
     XV acc = XV(0.0);
     Batch<VT, GL, WIDE> b;
@@ -144,7 +144,7 @@ __global__ void __launch_bounds__(256) spmm_long_kernel(const uint32_t *__restri
     const uint32_t r = rows[wave], g = lane / GL;
     const uint32_t kc = blockIdx.y * (GL * V) + lane % GL * V;
     const bool on = kc < k;
-    const uint32_t kx = on ? kc : 0;  // a lane past the last right-hand side reads the first and stores nothing
+    const uint32_t kx = on ? kc : blockIdx.y * (GL * V);  // past the last right-hand side: a live lane's X, nothing stored
     const uint32_t q0 = first[r], len = rowptr[r + 1] - rowptr[r];
     XV acc = XV(0.0);
     uint32_t t = g * B;  // group g takes batches g, g + G, ...

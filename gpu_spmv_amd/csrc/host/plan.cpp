@@ -742,6 +742,35 @@ bool narrow_bands(const axspmv_csr *a, uint32_t rows, uint64_t cols) {
     return wide * 8 <= a->nnz;
 }
 
+// The rows of an RCT plan for SpMM that get blocks of their own, in column
+// slices (one per XCD), or none.  On random columns every entry reads its own
+// line of X past the L2; rows of many entries are the exception, if they are
+// worked on together: the tiles that an XCD holds in LDS at once (64 of them)
+// then read each X row of their slice several times while it is in L2.  A
+// heavy row costs an atomic add per slice, as much traffic as a few lines, so
+// it needs at least 32 entries; the split is made where such rows are few (at
+// most 1/8 of the rows) but hold a good part of the entries (1/4, and at
+// least 4 per column), and the rows reach over more than 65,536 columns (X of
+// 8 right-hand sides and more does not fit an L2).  Power-law matrices, FP64,
+// one box, without / with: 600,000 rows, k = 8, 1024-row tiles 222 / 148 us;
+// 400,003 rows, k = 32, 256-row tiles 323 / 236 us; SpMV on 10^6 rows and
+// 1024-row tiles 195 / 133 us.  (With 4 column slices for the other rows, k =
+// 8: 184 / 185 us.)
+std::vector<uint32_t> heavy_rows(const axspmv_csr *a) {
+    constexpr uint32_t LONG = 32;
+    std::vector<uint32_t> rows;
+    if (a->ncols <= 65536) return rows;
+    uint64_t nnz = 0;
+    for (uint32_t r = 0; r < a->nrows; ++r) {
+        const uint32_t l = a->row[r + 1] - a->row[r];
+        if (l < LONG) continue;
+        rows.push_back(r);
+        nnz += l;
+    }
+    if (8 * rows.size() > a->nrows || 4 * nnz < a->nnz || nnz < 4ull * a->ncols || narrow_bands(a, 1024, 65536)) rows.clear();
+    return rows;
+}
+
 // RCT: row blocks of at most tile_rows rows and about equal nonzeros, column
 // slices, entries of a tile sorted by (column, row).
 int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
@@ -837,13 +866,34 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
     uint32_t R = 1;  // rows of the largest block: the LDS accumulator size
     for (uint32_t k = 0; k < nrb; ++k) R = std::max(R, rbs[k + 1] - rbs[k]);
     const uint32_t C = uint32_t(std::max<uint64_t>(1, ceil_div(a->ncols, S)));
-    const uint64_t ntile = uint64_t(nrb) * S;
+    // Heavy rows (plans that SpMM can use): blocks of their own, in column
+    // slices, their tiles after the others.
+    std::vector<uint32_t> hrows, hbs(1, 0), hmask;
+    if (!p.keep_pos && 64ull * R <= lds_max) hrows = heavy_rows(a);
+    const uint32_t HS = launch::HEAVY_SLICES;
+    const uint32_t HC = uint32_t(std::max<uint64_t>(1, ceil_div(a->ncols, HS)));
+    const uint32_t nhb = uint32_t(ceil_div(hrows.size(), R));
+    if (nhb) {
+        hmask.assign(ceil_div(n, 32), 0);
+        for (uint32_t r : hrows) hmask[r >> 5] |= 1u << (r & 31);
+        for (uint32_t k = 1; k <= nhb; ++k) hbs.push_back(uint32_t(uint64_t(hrows.size()) * k / nhb));
+    }
+    auto heavy = [&](uint32_t r) { return nhb && (hmask[r >> 5] >> (r & 31) & 1); };
+    const uint64_t ntile = uint64_t(nrb) * S, nall = ntile + uint64_t(nhb) * HS;
     // count entries per tile
-    std::vector<uint64_t> cnt(ntile + 1, 0);
+    std::vector<uint64_t> cnt(nall + 1, 0);
 #pragma omp parallel for schedule(dynamic, 1)
     for (uint32_t rb = 0; rb < nrb; ++rb)
-        for (uint32_t j = a->row[rbs[rb]]; j < a->row[rbs[rb + 1]]; ++j) cnt[uint64_t(rb) * S + a->col[j] / C + 1]++;
-    for (uint64_t t = 0; t < ntile; ++t) cnt[t + 1] += cnt[t];
+        for (uint32_t r = rbs[rb]; r < rbs[rb + 1]; ++r) {
+            if (heavy(r)) continue;
+            for (uint32_t j = a->row[r]; j < a->row[r + 1]; ++j) cnt[uint64_t(rb) * S + a->col[j] / C + 1]++;
+        }
+#pragma omp parallel for schedule(dynamic, 1)
+    for (uint32_t hb = 0; hb < nhb; ++hb)
+        for (uint32_t i = hbs[hb]; i < hbs[hb + 1]; ++i)
+            for (uint32_t j = a->row[hrows[i]]; j < a->row[hrows[i] + 1]; ++j)
+                cnt[ntile + uint64_t(hb) * HS + a->col[j] / HC + 1]++;
+    for (uint64_t t = 0; t < nall; ++t) cnt[t + 1] += cnt[t];
     const uint64_t nnz = a->nnz;
     std::vector<uint32_t> col(nnz ? nnz : 1);
     std::vector<uint16_t> lrow(nnz ? nnz : 1);
@@ -855,15 +905,25 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
     {
         std::vector<std::pair<uint64_t, uint32_t>> key;  // (col << 16 | lrow, CSR position)
 #pragma omp for schedule(dynamic, 1)
-        for (uint32_t rb = 0; rb < nrb; ++rb) {
-            const uint32_t r0 = rbs[rb], r1 = rbs[rb + 1];
+        for (uint32_t b = 0; b < nhb + nrb; ++b) {  // the heavy blocks, of the most entries, first
             key.clear();
-            for (uint32_t r = r0; r < r1; ++r)
-                for (uint32_t j = a->row[r]; j < a->row[r + 1]; ++j)
-                    key.emplace_back((uint64_t(a->col[j]) << 16) | (r - r0), j);
+            uint64_t q;
+            if (b < nhb) {
+                for (uint32_t i = hbs[b]; i < hbs[b + 1]; ++i)
+                    for (uint32_t j = a->row[hrows[i]]; j < a->row[hrows[i] + 1]; ++j)
+                        key.emplace_back((uint64_t(a->col[j]) << 16) | (i - hbs[b]), j);
+                q = cnt[ntile + uint64_t(b) * HS];
+            } else {
+                const uint32_t rb = b - nhb, r0 = rbs[rb], r1 = rbs[rb + 1];
+                for (uint32_t r = r0; r < r1; ++r) {
+                    if (heavy(r)) continue;
+                    for (uint32_t j = a->row[r]; j < a->row[r + 1]; ++j)
+                        key.emplace_back((uint64_t(a->col[j]) << 16) | (r - r0), j);
+                }
+                q = cnt[uint64_t(rb) * S];
+            }
             std::sort(key.begin(), key.end());
             // sorted by column, so the slices come out in order
-            uint64_t q = cnt[uint64_t(rb) * S];
             for (const auto &k : key) {
                 col[q] = uint32_t(k.first >> 16);
                 lrow[q] = uint16_t(k.first & 0xffff);
@@ -874,9 +934,9 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
         }
     }
     // the kernel indexes entries in 32 bits with up to 2 * 8 * 1024 past the end
-    if (cnt[ntile] >= (1ull << 32) - (1u << 16)) return fail(AXSPMV_E_OVERFLOW, "RCT: too many entries");
-    std::vector<uint32_t> tptr(ntile + 1);
-    for (uint64_t t = 0; t <= ntile; ++t) tptr[t] = uint32_t(cnt[t]);
+    if (cnt[nall] >= (1ull << 32) - (1u << 16)) return fail(AXSPMV_E_OVERFLOW, "RCT: too many entries");
+    std::vector<uint32_t> tptr(nall + 1);
+    for (uint64_t t = 0; t <= nall; ++t) tptr[t] = uint32_t(cnt[t]);
     const size_t vs = p.o.vtype == AXSPMV_F32 ? 4 : 8;
     // Pack (column offset, row within the tile) into one word when both fit
     // in 32 bits.  The offset is taken from a base column per run of 1024
@@ -920,7 +980,7 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
     std::vector<uint32_t> sbase16;
     int64_t dlo = 0;
     uint32_t cbits16 = 0;
-    bool diag = packed && nnz > 0 && !(p.o.flags & AXSPMV_PLAN_RCT_WIDE_KEY);
+    bool diag = packed && nnz > 0 && !nhb && !(p.o.flags & AXSPMV_PLAN_RCT_WIDE_KEY);
     if (diag) {
         int64_t lo = INT64_MAX, hi = INT64_MIN;
 #pragma omp parallel for schedule(dynamic, 1) reduction(min : lo) reduction(max : hi)
@@ -1002,7 +1062,7 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
     // Laplacian on 256^2, 1.3K per tile, 3.69 -> 3.05 us at 128; a 2^16-row
     // power-law matrix, 5.1K per tile, 9.17 -> 7.83 us at 256).
     if (block == 0) {
-        const uint64_t per_tile = nnz / std::max<uint64_t>(1, ntile);
+        const uint64_t per_tile = nnz / std::max<uint64_t>(1, nall);
         block = per_tile < 2048 ? 128 : per_tile < 16384 ? 256 : 512;
     }
 
@@ -1019,7 +1079,7 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
     // atomics).  The plan of A^T, which adds into x_bar from its fused
     // value-gradient sweep, keeps the atomic adds.
     double *dpart = nullptr;
-    if (S > 1 && p.lds_per_row == 8 && !(p.o.flags & AXSPMV_PLAN_RCT_ATOMIC) && 6ull * S * n >= nnz) {
+    if (S > 1 && !nhb && p.lds_per_row == 8 && !(p.o.flags & AXSPMV_PLAN_RCT_ATOMIC) && 6ull * S * n >= nnz) {
         dpart = static_cast<double *>(p.dalloc(8ull * S * n));
         if (!dpart) return AXSPMV_E_NOMEM;
     }
@@ -1037,13 +1097,27 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
     p.rct.key16 = dk16;
     p.rct.cbits16 = cbits16;
     p.rct.dmin = uint32_t(uint64_t(dlo));
+    if (nhb) {
+        auto *dh = static_cast<uint32_t *>(p.dalloc(4 * hrows.size()));
+        auto *db = static_cast<uint32_t *>(p.dalloc(4 * hbs.size()));
+        auto *dm = static_cast<uint32_t *>(p.dalloc(4 * hmask.size()));
+        if (!dh || !db || !dm) return AXSPMV_E_NOMEM;
+        AX_TRY(p.upload(dh, hrows.data(), 4 * hrows.size(), s));
+        AX_TRY(p.upload(db, hbs.data(), 4 * hbs.size(), s));
+        AX_TRY(p.upload(dm, hmask.data(), 4 * hmask.size(), s));
+        p.rct.nhb = nhb;
+        p.rct.nheavy = uint32_t(hrows.size());
+        p.rct.hrows = dh;
+        p.rct.hb_start = db;
+        p.rct.hmask = dm;
+    }
     p.slots = nnz;
     // matrix stream; with S > 1 the partials written and read back and y
     // written by the merge, or the clear of y and S atomic adds per row
     p.stream_bytes = (vs + kbytes) * nnz + 4 * tptr.size() +
-                     (S == 1 ? 0 : dpart ? 8ull * (2 * S + 1) * n : 8ull * (S + 1) * n);
-    p.launches = S > 1 ? 2 : 1;
-    p.nblocks = uint32_t(ntile);
+                     (S == 1 ? 0 : dpart ? 8ull * (2 * S + 1) * n : 8ull * (S + 1) * n) + 8ull * HS * hrows.size();
+    p.launches = S > 1 || nhb ? 2 : 1;
+    p.nblocks = uint32_t(nall);
     p.kind = Plan::RCT;
     std::snprintf(p.name, sizeof p.name, "rct_r%u_s%u%s%s", Rt, S, diag ? "_k16" : packed ? "" : "_split",
                   S > 1 && !dpart && p.lds_per_row == 8 ? "_atomic" : "");

@@ -458,7 +458,10 @@ int axspmv_fwd_adj(axspmv_plan *p, const double *d_x, const double *d_b, double 
  * ktile sums in LDS, so tile_rows * ktile * 8 bytes must fit one workgroup's
  * LDS -- tile_rows <= 2560 at ktile 8 on 160 KB; the default ktile is cut
  * to fit; with several column slices Y is cleared, then atomically added
- * to; 1024-lane workgroups unless the plan sets block).  No reference
+ * to; rows of 32 entries and more, where they are few but hold a good part
+ * of a matrix of over 65,536 columns, get tiles of their own in plans whose
+ * tile_rows SpMM can use, and their sums are added to Y atomically;
+ * 1024-lane workgroups unless the plan sets block).  No reference
  * counterpart. */
 int axspmv_spmm(axspmv_plan *p, uint32_t k, const double *d_X, double *d_Y, void *stream);
 

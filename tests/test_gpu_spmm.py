@@ -91,3 +91,75 @@ def test_x_of_4_gb(fmt, kw):
     xs, val = X[np.searchsorted(used, col)], f32_values(m, kw).val
     ref = np.stack([val[a:b] @ xs[a:b] for a, b in zip(row[:-1].astype(int), row[1:].astype(int))])
     assert rel_err(ref, dY.download(np.float64, m.nrows * k).reshape(m.nrows, k)) <= TOL
+
+
+# ------------------------------------------- heavy rows (RCT plans for SpMM)
+def heavy_matrix():
+    """70,001 rows, over 65,536 columns, a fifteenth of the rows holding most
+    of the entries, the first and the last row among them."""
+    n = 70001
+    rng = np.random.default_rng(12)
+    lens = rng.integers(0, 6, n)
+    big = np.concatenate([[0, n - 1], rng.choice(np.arange(1, n - 1), n // 15, replace=False)])
+    lens[big] = rng.integers(32, 200, big.size)
+    lens[0] = 2500
+    row = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    col = rng.integers(0, n, int(row[-1])).astype(np.uint32)  # unsorted, repeats: every entry is summed
+    return ax.CsrMatrix(row, col, rng.standard_normal(col.size), ncols=n)
+
+
+HEAVY = heavy_matrix()
+HEAVY_PLANS = [dict(tile_rows=1024), dict(tile_rows=250, slices=4), dict(tile_rows=512, flags=ax.PLAN_RCT_SPLIT),
+               dict(tile_rows=2048, slices=2, vtype=ax.F32, block=256)]
+
+
+def has_heavy(plan, kw):
+    return plan.info()["nblocks"] > -(-HEAVY.nrows // kw["tile_rows"]) * kw.get("slices", 1)
+
+
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("k", [1, 6, 16, 21])
+@pytest.mark.parametrize("kw", HEAVY_PLANS, ids=["r1024", "r250_s4", "split", "f32_s2"])
+def test_heavy_rows_spmm(kw, k, off):
+    X = ax.uniform(110 + k, HEAVY.ncols * k).reshape(HEAVY.ncols, k)
+    p = ax.Plan(HEAVY, ax.FMT_RCT, **kw)
+    assert has_heavy(p, kw)
+    for _ in range(2):  # the second call's heavy rows start from the first one's sums: cleared
+        assert rel_err(orc.spmm(f32_values(HEAVY, kw), X), spmm(p, HEAVY, X, off)) <= TOL
+
+
+@pytest.mark.parametrize("kw", HEAVY_PLANS, ids=["r1024", "r250_s4", "split", "f32_s2"])
+def test_heavy_rows_spmv_and_fwd_adj(kw):
+    m = HEAVY
+    ref_m = f32_values(m, kw)
+    x, b = ax.uniform(5, m.ncols), ax.uniform(6, m.nrows)
+    p = ax.Plan(m, ax.FMT_RCT, **dict(kw, flags=kw.get("flags", 0) | ax.PLAN_TRANSPOSE))
+    assert has_heavy(p, kw)
+    y = orc.ncsr(ref_m, x)
+    for _ in range(2):
+        assert rel_err(y, ax.spmv_host(p, x)) <= TOL
+    dx, db = ax.DeviceBuffer.from_array(x), ax.DeviceBuffer.from_array(b)
+    dy, dr, dxb = (ax.DeviceBuffer.from_array(np.full(m.nrows, np.nan)) for _ in range(3))
+    dv = ax.DeviceBuffer(8 * m.nnz)
+    for fused in (True, False):
+        p.fwd_adj(dx, db, dy, dr, dxb, dv, fused=fused)
+        assert rel_err(y, dy.download(np.float64, m.nrows)) <= TOL
+        r = dr.download(np.float64, m.nrows)
+        assert np.array_equal(r, dy.download(np.float64, m.nrows) - b)
+        assert rel_err(orc.ncsr_t(ref_m, r, m.ncols), dxb.download(np.float64, m.ncols)) <= TOL
+        assert np.array_equal(p.vbar_csr(dv.download(np.float64, m.nnz)), r[m.row_ids()] * x[m.col])
+
+
+def test_heavy_rows_graph():
+    """Replays of a captured SpMM clear the heavy rows each time."""
+    k = 8
+    X = ax.uniform(120, HEAVY.ncols * k).reshape(HEAVY.ncols, k)
+    p = ax.Plan(HEAVY, ax.FMT_RCT, tile_rows=1024)
+    dX, dY = ax.DeviceBuffer.from_array(X), ax.DeviceBuffer(8 * HEAVY.nrows * k)
+    g = ax.Graph.of_plan(p, ax._lib.OP_SPMM, repeats=2, X=dX, Y=dY, k=k)
+    ref = orc.spmm(HEAVY, X)
+    for _ in range(3):
+        dY.upload(np.full(HEAVY.nrows * k, np.nan))
+        g.launch()
+        ax._lib.call("axspmv_device_sync")
+        assert rel_err(ref, dY.download(np.float64, HEAVY.nrows * k).reshape(HEAVY.nrows, k)) <= TOL
