@@ -143,33 +143,39 @@ struct RctEntries {
 
 int key_mode(const RctArgs &a) { return a.key16 ? KEY_DIAG : a.key ? KEY_PACKED : KEY_SPLIT; }
 
-// Tile w of the grid: XCD w % 8 takes slice (w % 8) % S; false for the
-// workgroups past the last row block.  HV: the heavy rows' tiles come first,
-// block w / 8 and slice w % 8 for the XCD w % 8.
+// Tile w of nb row blocks x S slices: XCD w % 8 takes slice (w % 8) % S; false
+// for the workgroups past the last row block.
+__device__ __forceinline__ bool tile_of(uint32_t w, uint32_t nb, uint32_t S, uint32_t &rb, uint32_t &s) {
+    const uint32_t xcd = w % 8, i = w / 8;
+    const uint32_t per = 8 / S;  // row-block groups per slice
+    s = xcd % S;
+    rb = i * per + xcd / S;
+    return rb < nb;
+}
+__host__ __device__ constexpr uint32_t tile_groups(uint32_t nb, uint32_t S) { return (nb + 8 / S - 1) / (8 / S) * 8; }
+
+// The tile of workgroup w.  HV: the heavy rows' tiles come first.
 template <bool HV = false>
 struct TileOf {
-    uint32_t s, rb, t;  // t: index in storage order
+    uint32_t s, t;  // slice; index in storage order
     uint32_t row0, rows;
     bool heavy;
     __device__ __forceinline__ bool from(const RctArgs &a, uint32_t w) {
+        uint32_t rb;
         heavy = false;
         if constexpr (HV) {
-            if (w < axspmv::launch::HEAVY_SLICES * a.nhb) {
+            const uint32_t nh = tile_groups(a.nhb, a.hs);
+            if (w < nh) {
                 heavy = true;
-                s = w % axspmv::launch::HEAVY_SLICES;
-                rb = w / axspmv::launch::HEAVY_SLICES;
-                t = a.nrb * a.S + w;
+                if (!tile_of(w, a.nhb, a.hs, rb, s)) return false;
+                t = a.nrb * a.S + rb * a.hs + s;
                 row0 = a.hb_start[rb];
                 rows = a.hb_start[rb + 1] - row0;
                 return true;
             }
-            w -= axspmv::launch::HEAVY_SLICES * a.nhb;
+            w -= nh;
         }
-        const uint32_t xcd = w % 8, i = w / 8;
-        const uint32_t per = 8 / a.S;  // row-block groups per slice
-        s = xcd % a.S;
-        rb = i * per + xcd / a.S;
-        if (rb >= a.nrb) return false;
+        if (!tile_of(w, a.nrb, a.S, rb, s)) return false;
         t = rb * a.S + s;
         row0 = a.rb_start[rb];
         rows = a.rb_start[rb + 1] - row0;  // <= a.R
@@ -187,10 +193,7 @@ struct TileOf {
     }
 };
 
-unsigned rct_grid(const RctArgs &a) {
-    const uint32_t per = 8 / a.S;
-    return (a.nrb + per - 1) / per * 8 + axspmv::launch::HEAVY_SLICES * a.nhb;
-}
+unsigned rct_grid(const RctArgs &a) { return tile_groups(a.nrb, a.S) + (a.nhb ? tile_groups(a.nhb, a.hs) : 0); }
 
 // VB: the same product on the plan of A^T, fused with the value gradient of
 // A: vb[e] = xr[row(e)] * x[col(e)] for every entry, in entry order (the
@@ -406,25 +409,27 @@ __global__ void __launch_bounds__(1024) rct_vbar_kernel(RctArgs a, const double 
 // behind them.  X rows are addressed by 32-bit byte offsets, or (WIDE: X of
 // 4 GB and more) by their column.
 //
-// LDS layout: sum (row, right-hand side l V + v) sits at row KT + v GL + l,
-// and odd groups add their second right-hand side first, so the groups of
-// one ds_add_f64 spread over both halves of their rows' banks.
-template <class VT, int KEY, int GL, bool WIDE>
+// LDS layout: sum (row, right-hand side l V + v) sits at row KT + l + GL (v
+// xor the row's parity), so the groups of one ds_add_f64 spread over both
+// halves of their rows' banks.
+template <class VT, int KEY, int GL, int V, bool WIDE>
 struct SpmmBatch {
+    static constexpr int KT = GL * V;
     static constexpr int ROW = GL < 16 ? GL : 16;  // lanes that share a batch: wider groups load it once per 16
     static constexpr int E = ROW == 4 ? 2 : 1;     // entries per lane
     static constexpr int B = ROW * E;
     VT v[E];
-    uint32_t c[E], r[E];  // X row (byte offset, or column), tile row
+    uint32_t c[E], r[E];  // X row (byte offset, or column), tile row's first sum
     __device__ __forceinline__ void load(const RctEntries<VT, KEY> &ent, uint32_t e0, uint32_t end, uint32_t k) {
         const uint32_t i = e0 + threadIdx.x % ROW;
 #pragma unroll
         for (int u = 0; u < E; ++u)
             if (i + u * ROW < end) {
                 v[u] = ent.val[i + u * ROW];
-                uint32_t cc;
-                ent.at(i + u * ROW, cc, r[u]);
+                uint32_t cc, rr;
+                ent.at(i + u * ROW, cc, rr);
                 c[u] = WIDE ? cc : cc * k * 8;
+                r[u] = rr * KT + (V == 2 ? (rr & 1) * GL : 0);
             }
     }
 };
@@ -433,7 +438,7 @@ template <class VT, int KEY, int GL, int V, bool WIDE, bool HV>
 __global__ void __launch_bounds__(1024) rct_spmm_kernel(RctArgs a, uint32_t k, uint32_t k0,
                                                         const double *__restrict__ X, double *__restrict__ Y) {
     using namespace axspmv::dev;
-    using Batch = SpmmBatch<VT, KEY, GL, WIDE>;
+    using Batch = SpmmBatch<VT, KEY, GL, V, WIDE>;
     typedef double vec __attribute__((ext_vector_type(V)));
     using XV = std::conditional_t<V == 1, double, vec>;
     constexpr uint32_t KT = GL * V, B = Batch::B, ROW = Batch::ROW, STEP = 8;
@@ -467,15 +472,13 @@ __global__ void __launch_bounds__(1024) rct_spmm_kernel(RctArgs a, uint32_t k, u
             static_for<N>([&](auto J) {
                 constexpr int j = j0 + J.value;
                 const double v = double(group_bcast<ROW, j % ROW>(b.v[j / ROW]));
-                const uint32_t r = group_bcast_u32<ROW, j % ROW>(b.r[j / ROW]) * KT;
+                const uint32_t r = group_bcast_u32<ROW, j % ROW>(b.r[j / ROW]);
                 if (uint32_t(j) < left) {
                     if constexpr (V == 1) {
                         atomicAdd(al + r, v * xv[J.value]);
                     } else {
-                        const double p0 = v * xv[J.value].x, p1 = v * xv[J.value].y;
-                        const uint32_t o = g & 1 ? GL : 0;
-                        atomicAdd(al + r + o, g & 1 ? p1 : p0);
-                        atomicAdd(al + r + (GL - o), g & 1 ? p0 : p1);
+                        atomicAdd(al + r, v * xv[J.value].x);
+                        atomicAdd(al + (r ^ GL), v * xv[J.value].y);
                     }
                 }
             });
@@ -499,10 +502,10 @@ __global__ void __launch_bounds__(1024) rct_spmm_kernel(RctArgs a, uint32_t k, u
             const uint32_t rr = q / GL, ll = q % GL;
             uint32_t r;
             if (k0 + ll * V >= k || !tile.out_row(a, rr, r)) continue;
-            const double *s = acc + rr * KT + ll;
+            const uint32_t i = rr * KT + ll + (V == 2 ? (rr & 1) * GL : 0);
             double *out = Y + size_t(r) * k + k0 + ll * V;
-            if constexpr (V == 1) *out = *s;
-            else *reinterpret_cast<XV *>(out) = XV{s[0], s[GL]};
+            if constexpr (V == 1) *out = acc[i];
+            else *reinterpret_cast<XV *>(out) = XV{acc[i], acc[rr * KT + ll + (~rr & 1) * GL]};
         }
     } else {
         // one sum per lane, so that the lanes' atomics fall side by side (two
@@ -511,7 +514,8 @@ __global__ void __launch_bounds__(1024) rct_spmm_kernel(RctArgs a, uint32_t k, u
             const uint32_t rr = q / KT, jj = q % KT;
             uint32_t r;
             if (k0 + jj < k && tile.out_row(a, rr, r))
-                unsafeAtomicAdd(Y + size_t(r) * k + k0 + jj, acc[rr * KT + jj % V * GL + jj / V]);
+                unsafeAtomicAdd(Y + size_t(r) * k + k0 + jj,
+                                acc[rr * KT + jj / V + (V == 2 ? ((jj ^ rr) & 1) * GL : 0)]);
         }
     }
 }

@@ -109,12 +109,11 @@ struct RctArgs {
     // rows of many entries kept apart (nhb > 0; not with key16 or partials):
     // nheavy rows listed in hrows (and marked in hmask, a bit per row; their
     // rows of the row blocks hold no entries), cut into nhb blocks (hb_start,
-    // nhb + 1 offsets into hrows, at most R rows each) x HEAVY_SLICES column
-    // slices, tiles after the others in tile_ptr
-    uint32_t nhb = 0, nheavy = 0;
+    // nhb + 1 offsets into hrows, at most R rows each) x hs column slices (1,
+    // 2, 4 or 8), tiles after the others in tile_ptr
+    uint32_t nhb = 0, nheavy = 0, hs = 1;
     const uint32_t *hb_start = nullptr, *hrows = nullptr, *hmask = nullptr;
 };
-constexpr uint32_t HEAVY_SLICES = 8;  // one per XCD
 // S > 1 with a.part: the tile kernel stores every slice's row sums in its
 // partial vector, then part_merge adds them in slice order into y; mid
 // (optional) is recorded on s between the two.  S > 1 without a.part: a fill

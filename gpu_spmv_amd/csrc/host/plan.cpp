@@ -870,9 +870,14 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
     // slices, their tiles after the others.
     std::vector<uint32_t> hrows, hbs(1, 0), hmask;
     if (!p.keep_pos && 64ull * R <= lds_max) hrows = heavy_rows(a);
-    const uint32_t HS = launch::HEAVY_SLICES;
+    // One slice per XCD, and blocks of few enough rows that their tiles reach
+    // every CU: 100,000-row power-law matrix, k = 8, blocks as tall as the LDS
+    // allows (64 tiles) 38 us, 256 tiles 26, 512 tiles 29.  4 slices lose where
+    // X is large (k = 32, 400,003 rows: 252 against 237 us) and gain a little
+    // elsewhere (k = 8, 600,000 rows: 144 against 149); 16 cost their adds (266).
+    constexpr uint32_t HS = 8, HTILES = 256;
     const uint32_t HC = uint32_t(std::max<uint64_t>(1, ceil_div(a->ncols, HS)));
-    const uint32_t nhb = uint32_t(ceil_div(hrows.size(), R));
+    const uint32_t nhb = uint32_t(std::max<uint64_t>(ceil_div(hrows.size(), R), std::min<uint64_t>(hrows.size(), HTILES / HS)));
     if (nhb) {
         hmask.assign(ceil_div(n, 32), 0);
         for (uint32_t r : hrows) hmask[r >> 5] |= 1u << (r & 31);
@@ -1106,6 +1111,7 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
         AX_TRY(p.upload(db, hbs.data(), 4 * hbs.size(), s));
         AX_TRY(p.upload(dm, hmask.data(), 4 * hmask.size(), s));
         p.rct.nhb = nhb;
+        p.rct.hs = HS;
         p.rct.nheavy = uint32_t(hrows.size());
         p.rct.hrows = dh;
         p.rct.hb_start = db;
