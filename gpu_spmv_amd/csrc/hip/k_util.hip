@@ -5,6 +5,7 @@
 #include "wave64.hpp"
 
 namespace {
+using axspmv::launch::PermVecs;
 
 __global__ void __launch_bounds__(256) copy_kernel(const double2 *__restrict__ src, double2 *__restrict__ dst, size_t n2) {
     const size_t stride = size_t(gridDim.x) * blockDim.x;
@@ -82,14 +83,18 @@ __global__ void __launch_bounds__(256) fill_u32_kernel(uint32_t *__restrict__ ds
 // first reads a block of the source and writes its values in runs, one run
 // per destination chunk; the second reads a destination chunk's values, now
 // side by side, and writes the chunk in order.  No lane reads memory at
-// random; each lane issues U loads before it waits.
+// random; each lane issues U loads before it waits.  blockIdx.y picks one of
+// the vectors; res (a second pass) takes dst - rb with it.
 template <bool W>
 __global__ void __launch_bounds__(1024) permute_chunk_kernel(const uint32_t *__restrict__ w,
                                                              const uint16_t *__restrict__ b, uint32_t n, uint32_t L,
-                                                             const double *__restrict__ src,
-                                                             double *__restrict__ dst) {
+                                                             PermVecs vecs) {
     constexpr int U = 8;
     extern __shared__ double lds[];
+    const uint32_t vec = blockIdx.y;
+    const double *__restrict__ src = vecs.src[vec];
+    double *__restrict__ dst = vecs.dst[vec];
+    const bool res = !W && vec == 0 && vecs.res;
     const uint64_t base = uint64_t(blockIdx.x) * L;
     const uint32_t len = n - base < L ? uint32_t(n - base) : L, nt = blockDim.x;
     for (uint32_t i0 = threadIdx.x; i0 < len; i0 += U * nt) {
@@ -117,7 +122,11 @@ __global__ void __launch_bounds__(1024) permute_chunk_kernel(const uint32_t *__r
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const uint32_t i = i0 + u * nt;
-            if (i < len) dst[W ? to[u] : base + i] = lds[j[u]];
+            if (i < len) {
+                const double v = lds[j[u]];
+                dst[W ? to[u] : base + i] = v;
+                if (res) vecs.res[base + i] = v - vecs.rb[base + i];
+            }
         }
     }
 }
@@ -186,6 +195,34 @@ __global__ void __launch_bounds__(1024) back_residual_in_kernel(const uint16_t *
             const uint32_t i = i0 + u * nt;
             if (i < len) t2[to[u]] = lr[j[u]];
         }
+    }
+}
+
+// Whole vectors by a plain gather, four elements per lane; blockIdx.y picks
+// the vector.
+__global__ void __launch_bounds__(256) gather_vecs_kernel(uint32_t n, axspmv::launch::GatherVecs g) {
+    constexpr int U = 4;
+    const uint32_t vec = blockIdx.y;
+    const uint32_t *__restrict__ idx = g.idx[vec];
+    const double *__restrict__ src = g.src[vec], *from = g.from[vec];
+    double *dst = g.dst[vec];
+    const bool res = vec == 0 && g.res;
+    const uint32_t i0 = blockIdx.x * (256 * U) + threadIdx.x;
+    uint32_t j[U];
+    double v[U], f[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) j[u] = i0 + u * 256 < n ? idx[i0 + u * 256] : 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        v[u] = src[j[u]];
+        f[u] = i0 + u * 256 < n ? (from ? from[i0 + u * 256] : res ? g.rb[i0 + u * 256] : 0.0) : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const uint32_t i = i0 + u * 256;
+        if (i >= n) continue;
+        dst[i] = from ? f[u] - v[u] : v[u];
+        if (res) g.res[i] = v[u] - f[u];
     }
 }
 
@@ -340,13 +377,17 @@ hipError_t back_residual_in(const uint16_t *b2, const uint32_t *w1, const uint16
     return hipGetLastError();
 }
 
-hipError_t permute_chunks(const uint32_t *w, const uint16_t *b, uint32_t n, uint32_t L, const double *src,
-                          double *dst, hipStream_t s) {
-    const unsigned grid = unsigned((uint64_t(n) + L - 1) / L);
+hipError_t permute_chunks(const uint32_t *w, const uint16_t *b, uint32_t n, uint32_t L, const PermVecs &v, hipStream_t s) {
+    const dim3 grid(unsigned((uint64_t(n) + L - 1) / L), v.count);
     if (n && w)
-        permute_chunk_kernel<true><<<grid, 1024, size_t(L) * 8, s>>>(w, b, n, L, src, dst);
+        permute_chunk_kernel<true><<<grid, 1024, size_t(L) * 8, s>>>(w, b, n, L, v);
     else if (n)
-        permute_chunk_kernel<false><<<grid, 1024, size_t(L) * 8, s>>>(w, b, n, L, src, dst);
+        permute_chunk_kernel<false><<<grid, 1024, size_t(L) * 8, s>>>(w, b, n, L, v);
+    return hipGetLastError();
+}
+
+hipError_t gather_vecs(uint32_t n, const GatherVecs &g, hipStream_t s) {
+    if (n) gather_vecs_kernel<<<dim3((n + 1023) / 1024, g.count), 256, 0, s>>>(n, g);
     return hipGetLastError();
 }
 

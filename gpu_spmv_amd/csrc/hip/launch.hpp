@@ -257,12 +257,20 @@ hipError_t touch(const double *p, size_t n, double *sink, hipStream_t s);
 // the wave64 primitive op (enum axspmv_wave_op) lane by lane; n a multiple of 64
 hipError_t wave_selftest(uint32_t op, const double *v, const uint32_t *h, double *ov, uint32_t *oh, size_t n,
                          hipStream_t s);
-// For every chunk c of L positions of src (n in all; the last chunk may be
-// short; L <= 65536 and L * 8 bytes of LDS): lds[i] = src[c L + i], then
-// dst[w ? w[c L + i] : c L + i] = lds[b[c L + i]] (every w value < the length
-// of dst, every b value < the chunk's length)
-hipError_t permute_chunks(const uint32_t *w, const uint16_t *b, uint32_t n, uint32_t L, const double *src,
-                          double *dst, hipStream_t s);
+// Up to three vectors through one permutation pass: src[v] -> dst[v].  With
+// res, also res[i] = dst[0][i] - rb[i] (a pass without w).
+struct PermVecs {
+    const double *src[3];
+    double *dst[3];
+    uint32_t count;
+    const double *rb;
+    double *res;
+};
+// For every vector v and every chunk c of L positions of src[v] (n in all; the
+// last chunk may be short; L <= 65536 and L * 8 bytes of LDS): lds[i] = src[c
+// L + i], then dst[w ? w[c L + i] : c L + i] = lds[b[c L + i]] (every w value <
+// the length of dst, every b value < the chunk's length)
+hipError_t permute_chunks(const uint32_t *w, const uint16_t *b, uint32_t n, uint32_t L, const PermVecs &v, hipStream_t s);
 // For every chunk c of L positions (n in all; L <= 10240: 2 L * 8 bytes of
 // LDS): y[c L + i] = t[c L + b2[c L + i]], r[c L + i] = y[c L + i] -
 // bv[c L + i], then t2[w1[c L + i]] = r[c L + b1[c L + i]] -- the second pass
@@ -270,6 +278,19 @@ hipError_t permute_chunks(const uint32_t *w, const uint16_t *b, uint32_t n, uint
 // joined by a residual (t2 must not overlap t)
 hipError_t back_residual_in(const uint16_t *b2, const uint32_t *w1, const uint16_t *b1, uint32_t n, uint32_t L,
                             const double *t, const double *bv, double *y, double *r, double *t2, hipStream_t s);
+// Up to three vectors gathered by one launch: dst[v][i] = src[v][idx[v][i]], or
+// from[v][i] minus that (from[v] != nullptr), for i < n (every idx value < the
+// length of its src).  With res, also res[i] = dst[0][i] - rb[i] (no dst lies
+// over rb, but res may be it).
+struct GatherVecs {
+    const uint32_t *idx[3];
+    const double *src[3], *from[3];
+    double *dst[3];
+    uint32_t count;
+    const double *rb;
+    double *res;
+};
+hipError_t gather_vecs(uint32_t n, const GatherVecs &g, hipStream_t s);
 // dst[i k + j] = src[idx[i] k + j] for i < n, j < k (every idx[i] k + k <= the
 // length of src)
 hipError_t gather_rows(const uint32_t *idx, uint32_t n, uint32_t k, const double *src, double *dst, hipStream_t s);

@@ -1196,9 +1196,21 @@ double mean_diagonal_distance(const axspmv_csr *a) {
 // us for two XCD-segmented gathers (each XCD reading an L2-resident eighth
 // of the source at random), 20.5 us with the runs on the reading side and
 // 23.8 us with chunks of 4096.
+//
+// Vectors of up to 2^20 entries (8 MB) are gathered by one launch instead:
+// while the source more or less fits an L2 (4 MB) the gather runs at the
+// L2's rate, and the second launch costs more than the lines read twice.
+// Permuted stencils, AXT UNC SpMV, gather / two passes: 60^3 24.9 / 37.6 us,
+// 90^3 73.5 / 80.3, 116^3 (1.56M entries) 159.2 / 146.8; RCT on 100^3 97.7 /
+// 102.7.
+constexpr uint32_t PERM_DIRECT = 1u << 20;
 int upload_perm(Plan &p, const std::vector<uint32_t> &perm, Plan::Perm &out, hipStream_t s) {
     const uint32_t n = uint32_t(perm.size());
-    const uint32_t L = std::max(1u, std::min<uint32_t>(8192, n));
+    out.idx = static_cast<uint32_t *>(p.dalloc(4ull * n));
+    if (!out.idx) return AXSPMV_E_NOMEM;
+    AX_TRY(p.upload(out.idx, perm.data(), 4ull * n, s));
+    if (n <= PERM_DIRECT) return AXSPMV_OK;
+    const uint32_t L = 8192;
     const uint64_t nch = ceil_div(n, L);
     // t position of every destination: chunk by chunk, sorted by (source block, k)
     std::vector<uint32_t> tp(n ? n : 1);
@@ -1275,11 +1287,6 @@ int plan_reordered(const axspmv_csr *a, const axspmv_opts *o, void *stream, axsp
     hipStream_t s = static_cast<hipStream_t>(stream);
     AX_TRY(upload_perm(*p, q, p->to_b, s));
     AX_TRY(upload_perm(*p, qi, p->from_b, s));
-    p->d_perm = static_cast<uint32_t *>(p->dalloc(4ull * n));
-    p->d_iperm = static_cast<uint32_t *>(p->dalloc(4ull * n));
-    if (!p->d_perm || !p->d_iperm) return AXSPMV_E_NOMEM;
-    AX_TRY(p->upload(p->d_perm, q.data(), 4ull * n, s));
-    AX_TRY(p->upload(p->d_iperm, qi.data(), 4ull * n, s));
     p->nscratch = pi->T ? 6 : 3;
     for (uint32_t k = 0; k < p->nscratch; ++k) {
         p->d_scr[k] = static_cast<double *>(p->dalloc(8ull * n));
@@ -1292,13 +1299,15 @@ int plan_reordered(const axspmv_csr *a, const axspmv_opts *o, void *stream, axsp
     p->device_bytes += pi->device_bytes;
     p->alg_bytes = pi->alg_bytes;
     // the inner plan's bytes, then per vector permuted (x into B's order
-    // before the SpMV, y back after it) two passes of 8 B read and 8 B
-    // written, with 2 + 6 B of indices.  (RCT tiles storing their rows straight into A's
-    // numbering, y[q[k]], measured slower on the permuted 128^3 stencil: the
-    // tile kernel took 38 us more with ordinary scattered stores, 56 us more
-    // with non-temporal ones, against 30 us for the two passes.)
-    p->stream_bytes = pi->stream_bytes + 2ull * 40 * n;  // 2 vectors x (16 + 16 + 8) B
-    p->launches = pi->launches + 4;
+    // before the SpMV, y back after it) 8 B read and 8 B written, by one
+    // gather with 4 B of index or by two passes with 2 + 6 B.  (RCT tiles
+    // storing their rows straight into A's numbering, y[q[k]], measured slower
+    // on the permuted 128^3 stencil: the tile kernel took 38 us more with
+    // ordinary scattered stores, 56 us more with non-temporal ones, against 30
+    // us for the two passes.)
+    const bool direct = !p->to_b.L;
+    p->stream_bytes = pi->stream_bytes + 2ull * (direct ? 20 : 40) * n;
+    p->launches = pi->launches + (direct ? 2 : 4);
     p->nblocks = pi->nblocks;
     p->staged_blocks = pi->staged_blocks;
     p->rowwise = pi->rowwise;
@@ -1393,12 +1402,35 @@ extern "C" int axspmv_plan_get_info(const axspmv_plan *p, axspmv_plan_info *info
 
 namespace axspmv {
 
-// dst = src permuted by q, staged in the plan's last scratch vector
-static hipError_t permute(const Plan *p, const Plan::Perm &q, const double *src, double *dst, hipStream_t s) {
-    double *t = p->d_scr[p->nscratch - 1];
-    hipError_t e = launch::permute_chunks(q.w1, q.b1, p->nrows, q.L, src, t, s);
-    if (e == hipSuccess) e = launch::permute_chunks(nullptr, q.b2, p->nrows, q.L, t, dst, s);
+// v.dst = v.src permuted by q, by a plain gather (q.L == 0) or in two passes,
+// vector i staged in t[i] (no stage is another vector's source)
+static hipError_t permute(const Plan *p, const Plan::Perm &q, const launch::PermVecs &v, double *const *t, hipStream_t s) {
+    if (!q.L) {
+        launch::GatherVecs g{};
+        for (uint32_t i = 0; i < v.count; ++i) {
+            g.idx[i] = q.idx;
+            g.src[i] = v.src[i];
+            g.dst[i] = v.dst[i];
+        }
+        g.count = v.count;
+        g.rb = v.rb;
+        g.res = v.res;
+        return launch::gather_vecs(p->nrows, g, s);
+    }
+    launch::PermVecs one = v, two = v;
+    one.res = nullptr;
+    for (uint32_t i = 0; i < v.count; ++i) {
+        one.dst[i] = t[i];
+        two.src[i] = t[i];
+    }
+    hipError_t e = launch::permute_chunks(q.w1, q.b1, p->nrows, q.L, one, s);
+    if (e == hipSuccess) e = launch::permute_chunks(nullptr, q.b2, p->nrows, q.L, two, s);
     return e;
+}
+static launch::PermVecs perm_vec(const double *src, double *dst) { return {{src}, {dst}, 1, nullptr, nullptr}; }
+// One vector, staged in the plan's last scratch vector
+static hipError_t permute(const Plan *p, const Plan::Perm &q, const double *src, double *dst, hipStream_t s) {
+    return permute(p, q, perm_vec(src, dst), &p->d_scr[p->nscratch - 1], s);
 }
 
 hipError_t plan_launch(axspmv_plan *p, const double *x, double *y, hipStream_t s) {
@@ -1572,6 +1604,16 @@ static hipError_t reordered_op(Plan *p, uint32_t op, const axspmv_operands &o, h
     double *const *w = p->d_scr;
     auto in = [&](const double *v, double *d) { return permute(p, p->to_b, v, d, s); };
     auto back = [&](const double *v, double *d) { return permute(p, p->from_b, v, d, s); };
+    // two vectors into w[0] and w[1], together where there is a second stage
+    auto in2 = [&](const double *u, const double *v) {
+        if (p->nscratch < 4) {
+            const hipError_t e = in(u, w[0]);
+            return e == hipSuccess ? in(v, w[1]) : e;
+        }
+        double *const t[2] = {w[2], w[p->nscratch - 1]};
+        return permute(p, p->to_b, launch::PermVecs{{u, v}, {w[0], w[1]}, 2, nullptr, nullptr}, t, s);
+    };
+    auto apart = [&](const double *u, const double *v) { return u + p->nrows <= v || v + p->nrows <= u; };
     axspmv_operands io{};
     hipError_t e = hipSuccess;
     switch (op) {
@@ -1587,50 +1629,65 @@ static hipError_t reordered_op(Plan *p, uint32_t op, const axspmv_operands &o, h
             io.ybar = w[0];
             io.x = w[1];
             io.vbar = o.vbar;
-            e = in(o.ybar, w[0]);
-            if (e == hipSuccess) e = in(o.x, w[1]);
+            e = in2(o.ybar, o.x);
             if (e == hipSuccess) e = plan_op(p->inner, op, io, s);
             return e;
         case AXSPMV_OP_FWD_ADJ:
         case AXSPMV_OP_FWD_ADJ_SPLIT:
             if (op == AXSPMV_OP_FWD_ADJ && p->inner->kind != Plan::RCT) {
-                // the format's fused sweep takes b: x and b in, y, r and x_bar out
+                // the format's fused sweep takes b: x and b in together, y and
+                // x_bar out together, r = y - b formed again on y's way out
+                // (where an output lies over b: r out as the third vector)
                 io.x = w[0];
                 io.b = w[1];
                 io.y = w[2];
                 io.r = w[3];
                 io.xbar = w[4];
                 io.vbar = o.vbar;
-                e = in(o.x, w[0]);
-                if (e == hipSuccess) e = in(o.b, w[1]);
+                e = in2(o.x, o.b);
                 if (e == hipSuccess) e = plan_op(p->inner, op, io, s);
-                if (e == hipSuccess) e = back(w[2], o.y);
-                if (e == hipSuccess) e = back(w[3], o.r);
-                if (e == hipSuccess) e = back(w[4], o.xbar);
-                return e;
+                if (e != hipSuccess) return e;
+                if (apart(o.b, o.y) && apart(o.b, o.xbar) && apart(o.b, o.r))
+                    return permute(p, p->from_b, launch::PermVecs{{w[2], w[4]}, {o.y, o.xbar}, 2, o.b, o.r}, w, s);
+                double *const t[3] = {w[0], w[1], w[p->nscratch - 1]};
+                return permute(p, p->from_b, launch::PermVecs{{w[2], w[3], w[4]}, {o.y, o.r, o.xbar}, 3, nullptr, nullptr}, t, s);
             }
-            // four permutations instead of five: y comes back, r = y - b in
-            // A's numbering, r goes in; then x_bar and v_bar from B's plan of
-            // B^T (RCT: one sweep; otherwise the adjoint and the value
-            // gradient), x_bar back.  y's way back and r's way in meet in
-            // the same chunks of A's numbering: one kernel does the second
-            // pass of the one, the residual and the first pass of the other
-            // (y~'s vector, spent by then, takes r's runs).  With the
-            // non-temporal v_bar stores of the RCT sweep, on one box: the
-            // permuted 128^3 stencil, RCT, 483.4 -> 470.0 us.
+            // x in, the product, y back and r in, then x_bar and v_bar from
+            // B's plan of B^T (RCT: one sweep; otherwise the adjoint and the
+            // value gradient), x_bar back.  y's way back and r's way in are
+            // one launch of gathers, or, in two passes, meet in the same
+            // chunks of A's numbering: one kernel does the second pass of the
+            // one, the residual and the first pass of the other (y~'s vector,
+            // spent by then, takes r's runs; with the non-temporal v_bar
+            // stores of the RCT sweep, on one box: the permuted 128^3
+            // stencil, RCT, 483.4 -> 470.0 us).
             e = in(o.x, w[0]);
             if (e == hipSuccess) e = plan_launch(p->inner, w[0], w[1], s);
-            if (p->from_b.L == p->to_b.L) {
+            if (!p->to_b.L && !(apart(o.b, o.y) && apart(o.b, o.r))) {  // y or r over b: r from y, then r in
+                if (e == hipSuccess)
+                    e = permute(p, p->from_b, launch::PermVecs{{w[1]}, {o.y}, 1, o.b, o.r}, w, s);
+                if (e == hipSuccess) e = in(o.r, w[2]);
+            } else if (!p->to_b.L) {
+                // one launch: y = y~ back, r = y - b, and r~ = y~ - (b in B's order)
+                launch::GatherVecs g{};
+                g.idx[0] = p->from_b.idx;
+                g.src[0] = w[1];
+                g.dst[0] = o.y;
+                g.rb = o.b;
+                g.res = o.r;
+                g.idx[1] = p->to_b.idx;
+                g.src[1] = o.b;
+                g.from[1] = w[1];
+                g.dst[1] = w[2];
+                g.count = 2;
+                if (e == hipSuccess) e = launch::gather_vecs(p->nrows, g, s);
+            } else {
                 double *t = p->d_scr[p->nscratch - 1];
                 const Plan::Perm &f = p->from_b, &g = p->to_b;
-                if (e == hipSuccess) e = launch::permute_chunks(f.w1, f.b1, p->nrows, f.L, w[1], t, s);
+                if (e == hipSuccess) e = launch::permute_chunks(f.w1, f.b1, p->nrows, f.L, perm_vec(w[1], t), s);
                 if (e == hipSuccess)
                     e = launch::back_residual_in(f.b2, g.w1, g.b1, p->nrows, f.L, t, o.b, o.y, o.r, w[1], s);
-                if (e == hipSuccess) e = launch::permute_chunks(nullptr, g.b2, p->nrows, g.L, w[1], w[2], s);
-            } else {
-                if (e == hipSuccess) e = back(w[1], o.y);
-                if (e == hipSuccess) e = launch::residual(p->nrows, o.y, o.b, o.r, s);
-                if (e == hipSuccess) e = in(o.r, w[2]);
+                if (e == hipSuccess) e = launch::permute_chunks(nullptr, g.b2, p->nrows, g.L, perm_vec(w[1], w[2]), s);
             }
             if (e != hipSuccess) return e;
             if (op == AXSPMV_OP_FWD_ADJ) {  // RCT: x_bar = B^T r~ and v_bar in one sweep over the plan of B^T
@@ -1651,9 +1708,9 @@ static hipError_t reordered_op(Plan *p, uint32_t op, const axspmv_operands &o, h
             io.k = o.k;
             io.X = p->d_mm;
             io.Y = p->d_mm + nk;
-            e = launch::gather_rows(p->d_perm, p->nrows, o.k, o.X, p->d_mm, s);
+            e = launch::gather_rows(p->to_b.idx, p->nrows, o.k, o.X, p->d_mm, s);
             if (e == hipSuccess) e = plan_op(p->inner, op, io, s);
-            if (e == hipSuccess) e = launch::gather_rows(p->d_iperm, p->nrows, o.k, p->d_mm + nk, o.Y, s);
+            if (e == hipSuccess) e = launch::gather_rows(p->from_b.idx, p->nrows, o.k, p->d_mm + nk, o.Y, s);
             return e;
         }
         case AXSPMV_OP_XREFRESH:

@@ -82,8 +82,8 @@ struct axspmv_plan {
         uint16_t *b1 = nullptr, *b2 = nullptr;
         uint32_t *w1 = nullptr;
         uint32_t L = 0;
+        uint32_t *idx = nullptr;  // the permutation itself: small vectors, SpMM's rows of X and Y
     } to_b, from_b;
-    uint32_t *d_perm = nullptr, *d_iperm = nullptr;  // SpMM: rows of X into B's order, rows of Y back
     // SpMM operands in B's order (2 x nrows x k doubles, grown by
     // plan_op_prepare before a call needs them)
     double *d_mm = nullptr;

@@ -205,3 +205,45 @@ def test_reordered_rejects():
         ax.Plan(rect, ax.FMT_CSR, flags=ax.PLAN_REORDER)
     with pytest.raises(ax.AxspmvError):
         ax.Batch([m, m], fmt=ax.FMT_AXT, thw=4, flags=ax.PLAN_REORDER)
+
+
+@pytest.fixture(scope="module")
+def around_the_gather_line():
+    """Shuffled Laplacians just under and just over the 2^20 entries up to
+    which a vector is permuted by one gather."""
+    return {g: shuffled(ax.laplace2d(g), g) for g in (1023, 1025)}
+
+
+@pytest.mark.parametrize("alias", ["apart", "r_over_b", "y_over_b"])
+@pytest.mark.parametrize("fmt,kw", [(ax.FMT_AXT, dict(thw=4)), (ax.FMT_RCT, {})], ids=["axt", "rct"])
+@pytest.mark.parametrize("grid", [1023, 1025])
+def test_reordered_vectors_both_ways(around_the_gather_line, grid, fmt, kw, alias):
+    """Forward + adjoint and the value gradient on either permutation, with
+    the residual or y written over b as well."""
+    m = around_the_gather_line[grid]
+    n = m.nrows
+    p = ax.Plan(m, fmt, flags=ax.PLAN_REORDER | ax.PLAN_TRANSPOSE, **kw)
+    assert p.info()["name"].endswith("_rcm")
+    x, b = ax.uniform(31, n), ax.uniform(32, n)
+    y_ref = orc.ncsr(m, x)
+    for fused in (True, False):
+        dx, db = ax.DeviceBuffer.from_array(x), ax.DeviceBuffer.from_array(b)
+        dy, dr, dxb = (ax.DeviceBuffer.from_array(np.full(n, np.nan)) for _ in range(3))
+        dv = ax.DeviceBuffer(8 * m.nnz)
+        if alias == "r_over_b":
+            dr = db
+        if alias == "y_over_b":
+            dy = db
+        p.fwd_adj(dx, db, dy, dr, dxb, dv, fused=fused)
+        y, r = dy.download(np.float64, n), dr.download(np.float64, n)
+        assert rel_err(y_ref, y) <= TOL
+        assert np.array_equal(r, y - b)
+        assert rel_err(orc.ncsr_t(m, r, n), dxb.download(np.float64, n)) <= TOL
+        assert np.array_equal(p.vbar_csr(dv.download(np.float64, m.nnz)), r[m.row_ids()] * x[m.col])
+    p.vbar(dx, dxb, dv)  # two vectors in at once (x as y_bar, x_bar as x)
+    xb = dxb.download(np.float64, n)
+    assert np.array_equal(p.vbar_csr(dv.download(np.float64, m.nnz)), x[m.row_ids()] * xb[m.col])
+    if fmt == ax.FMT_AXT and alias == "apart":  # no transposed plan: one stage only
+        q = ax.Plan(m, fmt, flags=ax.PLAN_REORDER, **kw)
+        q.vbar(dx, dxb, dv)
+        assert np.array_equal(q.vbar_csr(dv.download(np.float64, m.nnz)), x[m.row_ids()] * xb[m.col])
