@@ -1090,15 +1090,15 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
     }
     p.rct = launch::RctArgs{dv, dc, dl, dk, dcb, dt, drb, n, R, S, nrb, p.o.vtype, block, rbits, a->ncols, dpart};
     // A matrix stream larger than the 256 MB Infinity Cache comes from HBM
-    // on every SpMV whatever the loads do: there tall tiles (one workgroup
-    // per CU) stream it with non-temporal loads (the 128^3 stencil
-    // renumbered by reverse Cuthill-McKee, 8192-row tiles: 184 -> 168 us per
-    // SpMV; the permuted stencil's 16384-row tiles: unchanged).  A smaller
-    // stream stays cached between SpMVs, and non-temporal loads give that up
-    // (the 2^20-row power-law matrix, 252 MB: 58 -> 89 us); short tiles,
-    // several workgroups per CU, measured 1 % slower with them (256 banded
-    // matrices, 2048-row tiles: 1236 -> 1249 us).
-    p.rct.nt_stream = (vs + kbytes) * nnz > (256ull << 20) && R >= 4096 ? 1 : 0;
+    // on every SpMV whatever the loads do: it is streamed with non-temporal
+    // loads, whatever the tile height (permuted 100^3 stencil, renumbered, one
+    // box: 3968-row tiles 98 -> 90 us per SpMV, 1024-row tiles 99 -> 97; the
+    // same in natural order 62 -> 57; 48 banded matrices with 16-bit keys,
+    // 512-row tiles 92.6 -> 90.5, 1.5M banded rows, 5888-row tiles 102 -> 97).
+    // A smaller stream stays cached between SpMVs, and non-temporal loads
+    // give that up (the 2^20-row power-law matrix, 252 MB, back to back: 58 ->
+    // 89 us).
+    p.rct.nt_stream = (vs + kbytes) * nnz > (256ull << 20) ? 1 : 0;
     p.rct.key16 = dk16;
     p.rct.cbits16 = cbits16;
     p.rct.dmin = uint32_t(uint64_t(dlo));
