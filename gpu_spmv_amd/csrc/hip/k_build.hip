@@ -225,7 +225,8 @@ __global__ void __launch_bounds__(256) fill_kernel(DevCsr a, const uint64_t *__r
 // ax -- pass through LDS and leave as 1 KB runs: stored from the lanes'
 // registers, each 16-byte piece was a request of its own (the 2^18-row
 // power-law matrix, 5.2M entries, hw 4: 64 us, against 73 us from registers,
-// 82 with non-temporal stores there, and 70 us one slot per lane).
+// 82 with non-temporal stores there, and 70 us one slot per lane), and now
+// whole lines, non-temporal, so that they leave the L2s to x: 37 us.
 typedef double f64x2 __attribute__((ext_vector_type(2)));
 typedef double f64x2_at8 __attribute__((ext_vector_type(2), aligned(8)));
 typedef uint32_t u32x4_at4 __attribute__((ext_vector_type(4), aligned(4)));
@@ -268,7 +269,7 @@ __global__ void __launch_bounds__(256) fill_quads_kernel(DevCsr a, const uint64_
             if (m > 2) x1.x = x[c.z];
         }
     }
-    if (i < nquads) reinterpret_cast<u32x4 *>(o.plane)[i] = c;
+    if (i < nquads) __builtin_nontemporal_store(c, reinterpret_cast<u32x4 *>(o.plane) + i);
     // slots 4 lane .. 4 lane + 3 of the wave's 256, as pairs of doubles of ax
     f64x2 *w = buf[threadIdx.x >> 6];
     const uint32_t sl = lane * 4, pr = (((sl >> hw_log) << (hw_log + 1)) + (sl & ((1u << hw_log) - 1))) / 2;
@@ -282,7 +283,7 @@ __global__ void __launch_bounds__(256) fill_quads_kernel(DevCsr a, const uint64_
     const uint32_t pairs = first < nquads ? min(nquads - first, 64u) * 4 : 0;
 #pragma unroll
     for (uint32_t j = 0; j < 4; ++j)
-        if (j * 64 + lane < pairs) s[j * 64 + lane] = w[j * 64 + lane];
+        if (j * 64 + lane < pairs) __builtin_nontemporal_store(w[j * 64 + lane], s + j * 64 + lane);
 }
 
 }  // namespace
