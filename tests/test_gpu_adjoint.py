@@ -336,3 +336,32 @@ def test_axt_slices_deterministic(slices):
         xs.append(dxb.download(np.float64, m.ncols))
     assert rel_err(orc.ncsr_t(m, w, m.ncols), xs[0]) <= TOL
     assert all(v.tobytes() == xs[0].tobytes() for v in xs)
+
+
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("thw", [1, 2, 4, 16, 64])
+def test_axt_value_gradient_runs(thw, off):
+    """The wave's value gradients leave as one run: units that are padding
+    only (wide tiles), rows that end inside a unit, empty rows between, rows of
+    more than 64 units, and nothing outside v_bar (at either 8-byte offset)."""
+    lens = [3, 0, 1, 64, 65, 4, 0, 0, 7, 256, 257, 1, 300, 2, 0, 5] + [1, 2, 3] * 40 + [2000, 1, 0]
+    rng = np.random.default_rng(7)
+    row = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    n = 2100
+    col = np.concatenate([np.sort(rng.choice(n, k, replace=False)) for k in lens]).astype(np.uint32)
+    m = ax.CsrMatrix(row, col, rng.standard_normal(col.size), ncols=n)
+    x, b, w = ax.uniform(91, n), ax.uniform(92, m.nrows), ax.uniform(93, m.nrows)
+    p = ax.Plan(m, ax.FMT_AXT, thw=thw, flags=ax.PLAN_TRANSPOSE)
+    dx, db, dw = (ax.DeviceBuffer.from_array(v) for v in (x, b, w))
+    dy, dr, dxb = ax.DeviceBuffer(8 * m.nrows), ax.DeviceBuffer(8 * m.nrows), ax.DeviceBuffer(8 * n)
+
+    def vbar(call, s):
+        dv = ax.DeviceBuffer.from_array(np.full(m.nnz + off + 1, np.nan))
+        call(dv.ptr + 8 * off)
+        ax._lib.call("axspmv_device_sync")
+        v = dv.download(np.float64, m.nnz + off + 1)
+        assert np.all(np.isnan(v[:off])) and np.isnan(v[-1])
+        assert np.array_equal(v[off:-1], s()[m.row_ids()] * x[m.col])
+
+    vbar(lambda d: p.vbar(dw, dx, d), lambda: w)
+    vbar(lambda d: p.fwd_adj(dx, db, dy, dr, dxb, d), lambda: dr.download(np.float64, m.nrows))
