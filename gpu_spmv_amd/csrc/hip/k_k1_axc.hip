@@ -38,23 +38,43 @@ __global__ void __launch_bounds__(256) k1_kernel(const K1Item *__restrict__ item
     const uint32_t r = lane % chunk;
     const uint32_t gid = w.chunk * chunk + r;
     const uint64_t base = uint64_t(w.chp) + r;
+    // Steps U at a time: the values and columns of the next U steps are in
+    // flight while the x gathers of these are waited for (a chunk is one
+    // chain of steps, and a small matrix has few chunks per SIMD to hide it
+    // behind).  Steps past the end re-read the item's last one and add
+    // nothing.  Against 4 steps without prefetch: random rows of 4 to 40
+    // entries, 20,001 rows 14.6 -> 7.8 us, 300,007 rows, FP32 values, 41.3 ->
+    // 37.4 (their x gathers alone take 28); 50,000-row power-law matrix 34.6 ->
+    // 24.3; permuted 80^3 stencil renumbered 61.0 -> 53.6.
+    constexpr uint32_t U = 8;
     double acc = 0.0;
-    uint32_t j = w.j0;
-    for (; j + 4 <= w.j1; j += 4) {
-        const uint64_t q = base + uint64_t(j) * chunk;
-        const VT v0 = stream_load<NT>(val + q), v1 = stream_load<NT>(val + q + chunk),
-                 v2 = stream_load<NT>(val + q + 2 * chunk), v3 = stream_load<NT>(val + q + 3 * chunk);
-        const double x0 = xpad(x, stream_load<NT>(col + q)), x1 = xpad(x, stream_load<NT>(col + q + chunk)),
-                     x2 = xpad(x, stream_load<NT>(col + q + 2 * chunk)),
-                     x3 = xpad(x, stream_load<NT>(col + q + 3 * chunk));
-        acc = fma(double(v0), x0, acc);
-        acc = fma(double(v1), x1, acc);
-        acc = fma(double(v2), x2, acc);
-        acc = fma(double(v3), x3, acc);
-    }
-    for (; j < w.j1; ++j) {
-        const uint64_t q = base + uint64_t(j) * chunk;
-        acc = fma(double(stream_load<NT>(val + q)), xpad(x, stream_load<NT>(col + q)), acc);
+    VT v[U];
+    uint32_t c[U];
+    auto half = [&](uint32_t j, uint32_t u0) {
+#pragma unroll
+        for (uint32_t u = u0; u < u0 + U / 2; ++u) {
+            const uint64_t q = base + uint64_t(min(j + u, w.j1 - 1)) * chunk;
+            v[u] = stream_load<NT>(val + q);
+            c[u] = stream_load<NT>(col + q);
+        }
+    };
+    auto fetch = [&](uint32_t j) {
+        half(j, 0);
+        if (j + U / 2 < w.j1) half(j, U / 2);
+    };
+    if (w.j0 < w.j1) {
+        fetch(w.j0);
+        for (uint32_t j = w.j0; j < w.j1; j += U) {
+            double xv[U], vv[U];
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u) {
+                xv[u] = j + u < w.j1 ? xpad(x, c[u]) : 0.0;
+                vv[u] = j + u < w.j1 ? double(v[u]) : 0.0;
+            }
+            if (j + U < w.j1) fetch(j + U);
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u) acc = fma(vv[u], xv[u], acc);
+        }
     }
     if (w.slot == NOROW) {
         if (gid < nrows) y[permi[gid]] = acc;
