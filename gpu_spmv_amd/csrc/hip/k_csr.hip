@@ -32,9 +32,7 @@ __global__ void __launch_bounds__(256) csr_vector_kernel(uint32_t nrows, const V
     const uint32_t r = uint32_t(gl / G), g = uint32_t(gl % G);
     const uint32_t b = row[r], e = row[r + 1];
     if (e - b > long_len) return;  // csr_long's row
-    double acc = 0.0;
-    for (uint32_t j = b + g; j < e; j += G)
-        acc = fma(double(axspmv::dev::stream_load<NT>(val + j)), x[axspmv::dev::stream_load<NT>(col + j)], acc);
+    double acc = axspmv::dev::strided_dot<NT, false, G <= 16 ? 4 : 1>(val, col, b + g, e, G, x);
     acc = axspmv::dev::group_sum_f64<G>(acc);
     if (g == 0) y[r] = acc;
 }
@@ -47,9 +45,7 @@ __global__ void __launch_bounds__(256) csr_long_kernel(const uint32_t *__restric
     const uint32_t w = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = threadIdx.x & 63;
     if (w >= nlong) return;
     const uint32_t r = rows[w];
-    double acc = 0.0;
-    for (uint32_t j = row[r] + lane; j < row[r + 1]; j += 64)
-        acc = fma(double(axspmv::dev::stream_load<NT>(val + j)), x[axspmv::dev::stream_load<NT>(col + j)], acc);
+    double acc = axspmv::dev::strided_dot<NT, false, 4>(val, col, row[r] + lane, row[r + 1], 64, x);
     acc = axspmv::dev::group_sum_f64<64>(acc);
     if (lane == 0) y[r] = acc;
 }

@@ -109,8 +109,7 @@ __global__ void __launch_bounds__(256) axc_kernel(uint32_t nrows, const uint32_t
     const uint32_t r = uint32_t(gl / G), g = uint32_t(gl % G);
     const uint32_t b = brp[r] >> 1, e = brp[r + 1] >> 1;
     if (e - b > long_slots) return;
-    double acc = 0.0;
-    for (uint32_t q = b + g; q < e; q += G) acc = fma(double(stream_load<NT>(vp + q)), xpad(x, stream_load<NT>(mapx + q)), acc);
+    double acc = strided_dot<NT, true, G <= 16 ? 4 : 1>(vp, mapx, b + g, e, G, x);
     acc = group_sum_f64<G>(acc);
     if (g == 0) y[r] = acc;
 }
@@ -124,9 +123,7 @@ __global__ void __launch_bounds__(256) axc_long(const uint32_t *__restrict__ row
     if (wave >= nlong) return;
     const uint32_t r = rows[wave];
     const uint32_t b = brp[r] >> 1, e = brp[r + 1] >> 1;
-    double acc = 0.0;
-    for (uint32_t q = b + lane; q < e; q += 64)
-        acc = fma(double(stream_load<NT>(vp + q)), xpad(x, stream_load<NT>(mapx + q)), acc);
+    double acc = strided_dot<NT, true, 4>(vp, mapx, b + lane, e, 64, x);
     acc = group_sum_f64<64>(acc);
     if (lane == 0) y[r] = acc;
 }

@@ -30,6 +30,44 @@ __device__ __forceinline__ T stream_load(const T *p) {
     else return *p;
 }
 
+// Sum of val[j] x[col[j]] over j = first, first + stride, ... < end, U terms in
+// flight at a time (PAD: columns may be padding), in the order of j.  The row
+// kernels take U = 4 with up to 16 lanes per row and for the long rows' waves,
+// where one term at a time made a chain of load pairs: CSR vector / AXC on the
+// 50,000-row power-law matrix 25.8 -> 15.6 / 42.8 -> 25.8 us, on 10^6 rows
+// 250 -> 240 / 277 -> 253, the 1000^2 Laplacian 22.1 -> 18.3 / 29.4 -> 25.9; U
+// = 1 with 32 and 64 lanes per row, which a row seldom fills twice (the 80^3
+// stencil, 32 lanes: 67.6 us, 71.7 with U = 4).
+template <bool NT, bool PAD, uint32_t U, class VT>
+__device__ __forceinline__ double strided_dot(const VT *__restrict__ val, const uint32_t *__restrict__ col,
+                                              uint32_t first, uint32_t end, uint32_t stride,
+                                              const double *__restrict__ x) {
+    double acc = 0.0;
+    for (uint32_t j = first; j < end; j += U * stride) {
+        // (CSR positions reach 2^32, where j + u stride would wrap; padded
+        // layouts stay under 2^31, and the plain test is the faster one)
+        const uint32_t left = end - j;
+        auto in = [&](uint32_t u) { return PAD ? j + u * stride < end : u * stride < left; };
+        VT v[U];
+        uint32_t c[U];
+        double xv[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u)
+            if (in(u)) {
+                v[u] = stream_load<NT>(val + j + u * stride);
+                c[u] = stream_load<NT>(col + j + u * stride);
+            }
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u)
+            if (in(u)) xv[u] = PAD ? xpad(x, c[u]) : x[c[u]];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u)
+            if (in(u)) acc = fma(double(v[u]), xv[u], acc);
+        if (!PAD && left <= U * stride) break;
+    }
+    return acc;
+}
+
 // DPP control words (GFX9 encoding).
 enum : int {
     DPP_ROW_SHR1 = 0x111,
