@@ -7,6 +7,7 @@
 #include "wave64.hpp"
 
 namespace {
+using namespace axspmv::dev;
 
 template <class VT>
 __global__ void __launch_bounds__(256) csr_naive_kernel(uint32_t nrows, const VT *__restrict__ val,
@@ -27,14 +28,37 @@ __global__ void __launch_bounds__(256) csr_vector_kernel(uint32_t nrows, const V
                                                          const uint32_t *__restrict__ col,
                                                          const uint32_t *__restrict__ row, uint32_t long_len,
                                                          const double *__restrict__ x, double *__restrict__ y) {
+    constexpr uint32_t R = rows_per_group(G);
     const size_t gl = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (gl / G >= nrows) return;  // whole groups leave together (G divides 64)
-    const uint32_t r = uint32_t(gl / G), g = uint32_t(gl % G);
-    const uint32_t b = row[r], e = row[r + 1];
-    if (e - b > long_len) return;  // csr_long's row
-    double acc = axspmv::dev::strided_dot<NT, false, G <= 16 ? 4 : 1>(val, col, b + g, e, G, x);
-    acc = axspmv::dev::group_sum_f64<G>(acc);
-    if (g == 0) y[r] = acc;
+    if (gl / G * R >= nrows) return;  // whole groups leave together (G divides 64)
+    const uint32_t r = uint32_t(gl / G) * R, g = uint32_t(gl % G);
+    if constexpr (R == 1) {
+        const uint32_t b = row[r], e = row[r + 1];
+        if (e - b > long_len) return;  // csr_long's row
+        double acc = strided_dot<NT, false, G <= 16 ? 4 : 1>(val, col, b + g, e, G, x);
+        acc = group_sum_f64<G>(acc);
+        if (g == 0) y[r] = acc;
+    } else {
+        uint32_t b[R], e[R];
+        double acc[R];
+#pragma unroll
+        for (uint32_t i = 0; i < R; ++i) {
+            b[i] = row[min(r + i, nrows)];
+            e[i] = row[min(r + i + 1, nrows)];
+        }
+        bool mine[R];  // not csr_long's row, not past the last
+#pragma unroll
+        for (uint32_t i = 0; i < R; ++i) {
+            mine[i] = r + i < nrows && e[i] - b[i] <= long_len;
+            if (!mine[i]) e[i] = b[i];
+        }
+        strided_dots<NT, false, R>(val, col, b, e, g, G, x, acc);
+#pragma unroll
+        for (uint32_t i = 0; i < R; ++i) {
+            acc[i] = group_sum_f64<G>(acc[i]);
+            if (g == 0 && mine[i]) y[r + i] = acc[i];
+        }
+    }
 }
 
 template <class VT, bool NT>
@@ -45,8 +69,8 @@ __global__ void __launch_bounds__(256) csr_long_kernel(const uint32_t *__restric
     const uint32_t w = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = threadIdx.x & 63;
     if (w >= nlong) return;
     const uint32_t r = rows[w];
-    double acc = axspmv::dev::strided_dot<NT, false, 4>(val, col, row[r] + lane, row[r + 1], 64, x);
-    acc = axspmv::dev::group_sum_f64<64>(acc);
+    double acc = strided_dot<NT, false, 4>(val, col, row[r] + lane, row[r + 1], 64, x);
+    acc = group_sum_f64<64>(acc);
     if (lane == 0) y[r] = acc;
 }
 
@@ -54,7 +78,8 @@ template <class VT, bool NT>
 hipError_t csr_vector_vt(uint32_t nrows, const VT *val, const uint32_t *col, const uint32_t *row, uint32_t lanes,
                          uint32_t long_len, const uint32_t *longrows, uint32_t nlong, const double *x, double *y,
                          hipStream_t s) {
-    const unsigned grid = unsigned((uint64_t(nrows) * lanes + 255) / 256);
+    const uint32_t rows = rows_per_group(lanes);
+    const unsigned grid = unsigned(((uint64_t(nrows) + rows - 1) / rows * lanes + 255) / 256);
     switch (lanes) {
 #define AX_G_CASE(G) \
     case G: csr_vector_kernel<VT, G, NT><<<grid, 256, 0, s>>>(nrows, val, col, row, long_len, x, y); break;

@@ -104,14 +104,37 @@ __global__ void __launch_bounds__(256) axc_kernel(uint32_t nrows, const uint32_t
                                                   const VT *__restrict__ vp, const uint32_t *__restrict__ mapx,
                                                   uint32_t long_slots, const double *__restrict__ x,
                                                   double *__restrict__ y) {
+    constexpr uint32_t R = rows_per_group(G);
     const size_t gl = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (gl / G >= nrows) return;  // whole groups leave together (G divides 64)
-    const uint32_t r = uint32_t(gl / G), g = uint32_t(gl % G);
-    const uint32_t b = brp[r] >> 1, e = brp[r + 1] >> 1;
-    if (e - b > long_slots) return;
-    double acc = strided_dot<NT, true, G <= 16 ? 4 : 1>(vp, mapx, b + g, e, G, x);
-    acc = group_sum_f64<G>(acc);
-    if (g == 0) y[r] = acc;
+    if (gl / G * R >= nrows) return;  // whole groups leave together (G divides 64)
+    const uint32_t r = uint32_t(gl / G) * R, g = uint32_t(gl % G);
+    if constexpr (R == 1) {
+        const uint32_t b = brp[r] >> 1, e = brp[r + 1] >> 1;
+        if (e - b > long_slots) return;
+        double acc = strided_dot<NT, true, G <= 16 ? 4 : 1>(vp, mapx, b + g, e, G, x);
+        acc = group_sum_f64<G>(acc);
+        if (g == 0) y[r] = acc;
+    } else {
+        uint32_t b[R], e[R];
+        double acc[R];
+#pragma unroll
+        for (uint32_t i = 0; i < R; ++i) {
+            b[i] = brp[min(r + i, nrows)] >> 1;
+            e[i] = brp[min(r + i + 1, nrows)] >> 1;
+        }
+        bool mine[R];  // not axc_long's row, not past the last
+#pragma unroll
+        for (uint32_t i = 0; i < R; ++i) {
+            mine[i] = r + i < nrows && e[i] - b[i] <= long_slots;
+            if (!mine[i]) e[i] = b[i];
+        }
+        strided_dots<NT, true, R>(vp, mapx, b, e, g, G, x, acc);
+#pragma unroll
+        for (uint32_t i = 0; i < R; ++i) {
+            acc[i] = group_sum_f64<G>(acc[i]);
+            if (g == 0 && mine[i]) y[r + i] = acc[i];
+        }
+    }
 }
 
 template <class VT, bool NT>
@@ -148,8 +171,8 @@ hipError_t k1_vt(const axspmv::launch::K1Args &a, const double *x, double *y, hi
 template <class VT, bool NT>
 hipError_t axc_vt(const axspmv::launch::AxcArgs &a, const double *x, double *y, hipStream_t s) {
     const VT *vp = static_cast<const VT *>(a.vplane);
-    const uint64_t th = uint64_t(a.nrows) * a.hbs;
-    const unsigned grid = unsigned((th + 255) / 256);
+    const uint32_t rows = rows_per_group(a.hbs);
+    const unsigned grid = unsigned(((uint64_t(a.nrows) + rows - 1) / rows * a.hbs + 255) / 256);
     if (a.nrows) switch (a.hbs) {
 #define AX_G(G) \
     case G: axc_kernel<VT, G, NT><<<grid, 256, 0, s>>>(a.nrows, a.brp, vp, a.mapx, a.long_slots, x, y); break;

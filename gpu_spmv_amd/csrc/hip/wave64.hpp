@@ -68,6 +68,46 @@ __device__ __forceinline__ double strided_dot(const VT *__restrict__ val, const 
     return acc;
 }
 
+// Rows a group of G lanes takes at once in the row-per-group kernels (CSR
+// vector, AXC): two with 32 lanes, where most rows are one short round each
+// and the waves' own cost shows (the 80^3 stencil in natural order, CSR / AXC
+// 67.3 -> 52.6 / 71.7 -> 56.1 us; four rows take 48.5 / 50.9 there but lose 4 %
+// on random rows of 20 to 46 entries); with 64 lanes two lost 8 % on rows of
+// 60 to 90 entries, with fewer a group has four terms in flight already.
+__host__ __device__ constexpr uint32_t rows_per_group(uint32_t G) { return G == 32 ? 2 : 1; }
+
+// R rows at once: acc[i] = the sum of val[j] x[col[j]] over j = b[i] + g, b[i] +
+// g + stride, ... < e[i], term by term with the R rows' loads in flight
+// together.
+template <bool NT, bool PAD, uint32_t R, class VT>
+__device__ __forceinline__ void strided_dots(const VT *__restrict__ val, const uint32_t *__restrict__ col,
+                                             const uint32_t *b, const uint32_t *e, uint32_t g, uint32_t stride,
+                                             const double *__restrict__ x, double *acc) {
+    uint32_t most = 0;  // the longest row
+#pragma unroll
+    for (uint32_t i = 0; i < R; ++i) {
+        acc[i] = 0.0;
+        most = max(most, e[i] - b[i]);
+    }
+    for (uint32_t k = g; k < most; k += stride) {
+        VT v[R];
+        uint32_t c[R];
+        double xv[R];
+#pragma unroll
+        for (uint32_t i = 0; i < R; ++i)
+            if (k < e[i] - b[i]) {
+                v[i] = stream_load<NT>(val + b[i] + k);
+                c[i] = stream_load<NT>(col + b[i] + k);
+            }
+#pragma unroll
+        for (uint32_t i = 0; i < R; ++i)
+            if (k < e[i] - b[i]) xv[i] = PAD ? xpad(x, c[i]) : x[c[i]];
+#pragma unroll
+        for (uint32_t i = 0; i < R; ++i)
+            if (k < e[i] - b[i]) acc[i] = fma(double(v[i]), xv[i], acc[i]);
+    }
+}
+
 // DPP control words (GFX9 encoding).
 enum : int {
     DPP_ROW_SHR1 = 0x111,

@@ -501,3 +501,27 @@ def test_axt_slices_layout_and_dispatch(slices):
         p.vbar(dw, ax.DeviceBuffer.from_array(x), ax.DeviceBuffer(8 * m.nnz))
     with pytest.raises(ax.AxspmvError, match="column slices"):
         ax.Plan(m, ax.FMT_AXT, thw=64, th=4, slices=slices)
+
+
+@pytest.mark.parametrize("last", [0, 1, 32, 33, 2100])
+@pytest.mark.parametrize("nrows", [1, 2, 3, 9, 64, 65])
+@pytest.mark.parametrize("fmt,kw", [(ax.FMT_CSR, dict(kernel=ax.KER_STREAM, hbs=32)), (ax.FMT_AXC, dict(hbs=32)),
+                                    (ax.FMT_AXC, dict(hbs=32, vtype=ax.F32))], ids=["csr", "axc", "axc_f32"])
+def test_two_rows_per_group(fmt, kw, nrows, last):
+    """32 lanes per row take two rows at once: an odd last row, a long row
+    (done by a wave of its own) or an empty one beside a short one."""
+    rng = np.random.default_rng(nrows)
+    lens = rng.choice([0, 1, 31, 32, 33, 65, 300], nrows)
+    lens[-1] = last
+    row = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    n = 2200
+    col = np.concatenate([np.sort(rng.choice(n, k, replace=False)) for k in lens]).astype(np.uint32)
+    m = ax.CsrMatrix(row, col, rng.standard_normal(col.size), ncols=n)
+    x = ax.uniform(33, n)
+    ref = orc.ncsr_f32val(m, x) if kw.get("vtype") == ax.F32 else orc.ncsr(m, x)
+    p = ax.Plan(m, fmt, **kw)
+    dx, dy = ax.DeviceBuffer.from_array(x), ax.DeviceBuffer.from_array(np.full(nrows + 1, np.nan))
+    p.spmv(dx, dy)
+    y = dy.download(np.float64, nrows + 1)
+    assert np.isnan(y[-1])
+    assert rel_err(ref, y[:-1]) <= TOL
