@@ -38,7 +38,9 @@
 namespace {
 using axspmv::launch::RctArgs;
 
-// Entry e of a tile: value val[e]; its column and tile row stored one of
+// Entry e of a tile: value val[e] (VT double or float; uint8_t: the value's
+// index in a table of at most 256, for matrices of few different values); its
+// column and tile row stored one of
 // three ways (KEY):
 //  * KEY_SPLIT: col[e] and lrow[e];
 //  * KEY_PACKED: one word key[e] = offset << rbits | row, the column being
@@ -79,27 +81,22 @@ struct RctEntries {
         c = base + (k & ((1u << cbits) - 1));
         r = c + (k >> cbits) + rofs;
     }
-    __device__ __forceinline__ void load(uint32_t e, uint32_t &c, uint32_t &r, double &v) const {
-        v = double(val[e]);
-        at(e, c, r);
-    }
-    // entries 2q and 2q + 1 with one 16-byte (8 for FP32 values) and one
-    // 8-byte (KEY_DIAG: 4-byte) load; the plan pads the arrays to an even
-    // number of entries
-    __device__ __forceinline__ void load2(uint32_t q, uint32_t (&c)[2], uint32_t (&r)[2], double (&v)[2]) const {
-        typedef double f64x2 __attribute__((ext_vector_type(2)));
-        typedef float f32x2 __attribute__((ext_vector_type(2)));
+    // entries 2q and 2q + 1 with one 16-byte (8 for FP32 values, 2 for table
+    // indices) and one 8-byte (KEY_DIAG: 4-byte) load; the plan pads the
+    // arrays to an even number of entries
+    __device__ __forceinline__ void load2(uint32_t q, uint32_t (&c)[2], uint32_t (&r)[2], VT (&v)[2]) const {
         typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-        if constexpr (sizeof(VT) == 8) {
-            const f64x2 *p = reinterpret_cast<const f64x2 *>(val) + q;
-            const f64x2 vv = NT ? __builtin_nontemporal_load(p) : *p;
+        if constexpr (sizeof(VT) == 1) {
+            const uint16_t *p = reinterpret_cast<const uint16_t *>(val) + q;
+            const uint16_t vv = NT ? __builtin_nontemporal_load(p) : *p;
+            v[0] = VT(vv & 0xff);
+            v[1] = VT(vv >> 8);
+        } else {
+            typedef VT v2 __attribute__((ext_vector_type(2)));
+            const v2 *p = reinterpret_cast<const v2 *>(val) + q;
+            const v2 vv = NT ? __builtin_nontemporal_load(p) : *p;
             v[0] = vv.x;
             v[1] = vv.y;
-        } else {
-            const f32x2 *p = reinterpret_cast<const f32x2 *>(val) + q;
-            const f32x2 vv = NT ? __builtin_nontemporal_load(p) : *p;
-            v[0] = double(vv.x);
-            v[1] = double(vv.y);
         }
         if constexpr (KEY == KEY_DIAG) {
             const uint32_t *pk = reinterpret_cast<const uint32_t *>(key16) + q;
@@ -140,6 +137,12 @@ struct RctEntries {
         }
     }
 };
+
+template <class VT>
+__device__ __forceinline__ double entry_value(VT v, const double *table) {
+    if constexpr (sizeof(VT) == 1) return table[v];
+    else return double(v);
+}
 
 int key_mode(const RctArgs &a) { return a.key16 ? KEY_DIAG : a.key ? KEY_PACKED : KEY_SPLIT; }
 
@@ -209,6 +212,9 @@ __global__ void __launch_bounds__(1024) rct_kernel(RctArgs a, const double *__re
     const uint32_t tid = threadIdx.x, nt = blockDim.x;
     const uint32_t row0 = tile.row0, rows = tile.rows;
     double *xs = yl + a.R;  // VB: xr of the tile's rows
+    __shared__ double table[sizeof(VT) == 1 ? 256 : 1];
+    if constexpr (sizeof(VT) == 1)
+        for (uint32_t k = tid; k < 256; k += nt) table[k] = a.pal[k];
     for (uint32_t k = tid; k < rows; k += nt) {
         yl[k] = 0.0;
         if constexpr (VB) xs[k] = xr[row0 + k];
@@ -245,7 +251,7 @@ __global__ void __launch_bounds__(1024) rct_kernel(RctArgs a, const double *__re
     struct PSet {
         uint32_t c[UP][2], r[UP][2];
         uint32_t at[UP][2];  // VB: the entries the two stores write
-        double v[UP][2];
+        VT v[UP][2];
         bool ok[UP][2];      // adds its product
     };
     if (beg < end) {
@@ -271,7 +277,7 @@ __global__ void __launch_bounds__(1024) rct_kernel(RctArgs a, const double *__re
                 }
             }
         };
-        auto gather = [&](const PSet &S, double (&xv)[UP][2], double (&xl)[UP][2]) {
+        auto gather = [&](const PSet &S, double (&xv)[UP][2], double (&xl)[UP][2], double (&vv)[UP][2]) {
 #pragma unroll
             for (int j = 0; j < UP; ++j) {
                 xv[j][0] = x[S.c[j][0]];
@@ -284,12 +290,17 @@ __global__ void __launch_bounds__(1024) rct_kernel(RctArgs a, const double *__re
                     xl[j][1] = xs[S.r[j][1]];
                 }
             }
+#pragma unroll
+            for (int j = 0; j < UP; ++j) {
+                vv[j][0] = entry_value(S.v[j][0], table);
+                vv[j][1] = entry_value(S.v[j][1], table);
+            }
         };
-        auto add = [&](const PSet &S, const double (&xv)[UP][2], const double (&xl)[UP][2]) {
+        auto add = [&](const PSet &S, const double (&xv)[UP][2], const double (&xl)[UP][2], const double (&vv)[UP][2]) {
 #pragma unroll
             for (int j = 0; j < UP; ++j) {
 #pragma unroll
-                for (int h = 0; h < 2; ++h) atomicAdd(&yl[S.r[j][h]], S.ok[j][h] ? S.v[j][h] * xv[j][h] : 0.0);
+                for (int h = 0; h < 2; ++h) atomicAdd(&yl[S.r[j][h]], S.ok[j][h] ? vv[j][h] * xv[j][h] : 0.0);
                 if constexpr (VB) {
                     const double p0 = xl[j][0] * xv[j][0], p1 = xl[j][1] * xv[j][1];
                     if (__all(vb16 && S.at[j][1] == S.at[j][0] + 1)) {  // whole pairs (at[j][0] even)
@@ -303,15 +314,15 @@ __global__ void __launch_bounds__(1024) rct_kernel(RctArgs a, const double *__re
             }
         };
         auto round = [&](const PSet &S, PSet &N, uint32_t q0) {
-            double xv[UP][2], xl[UP][2];
-            gather(S, xv, xl);
+            double xv[UP][2], xl[UP][2], vv[UP][2];
+            gather(S, xv, xl, vv);
             fetch(N, q0 + span);
-            add(S, xv, xl);
+            add(S, xv, xl, vv);
         };
         auto final_round = [&](const PSet &S) {
-            double xv[UP][2], xl[UP][2];
-            gather(S, xv, xl);
-            add(S, xv, xl);
+            double xv[UP][2], xl[UP][2], vv[UP][2];
+            gather(S, xv, xl, vv);
+            add(S, xv, xl, vv);
         };
         PSet A, B;
         uint32_t q = pb + tid;
@@ -457,6 +468,14 @@ __global__ void __launch_bounds__(1024) rct_spmm_kernel(RctArgs a, uint32_t k, u
     const uint32_t kx = k0 + l * V < k ? k0 + l * V : k0;
     double *const al = acc + l;
     auto work = [&](const Batch &b, uint32_t left) {
+        // a table index becomes its value before it is handed round
+        using BV = std::conditional_t<sizeof(VT) == 1, double, VT>;
+        BV bv[Batch::E];
+#pragma unroll
+        for (int u = 0; u < Batch::E; ++u) {
+            if constexpr (sizeof(VT) == 1) bv[u] = a.pal[b.v[u]];
+            else bv[u] = b.v[u];
+        }
         static_for<B / STEP ? B / STEP : 1>([&](auto H) {
             constexpr int N = B < STEP ? B : STEP, j0 = H.value * N;
             XV xv[N];
@@ -471,7 +490,7 @@ __global__ void __launch_bounds__(1024) rct_spmm_kernel(RctArgs a, uint32_t k, u
             __builtin_amdgcn_sched_barrier(0);
             static_for<N>([&](auto J) {
                 constexpr int j = j0 + J.value;
-                const double v = double(group_bcast<ROW, j % ROW>(b.v[j / ROW]));
+                const double v = double(group_bcast<ROW, j % ROW>(bv[j / ROW]));
                 const uint32_t r = group_bcast_u32<ROW, j % ROW>(b.r[j / ROW]);
                 if (uint32_t(j) < left) {
                     if constexpr (V == 1) {
@@ -582,13 +601,13 @@ hipError_t rct_spmm(const RctArgs &a, uint32_t k, uint32_t kt, const double *X, 
         if (e != hipSuccess) return e;
     }
     const int km = key_mode(a);
-    if (a.vtype == 1)
-        return km == KEY_DIAG     ? rct_spmm_vt<float, KEY_DIAG>(a, k, kt, X, Y, s)
-               : km == KEY_PACKED ? rct_spmm_vt<float, KEY_PACKED>(a, k, kt, X, Y, s)
-                                  : rct_spmm_vt<float, KEY_SPLIT>(a, k, kt, X, Y, s);
-    return km == KEY_DIAG     ? rct_spmm_vt<double, KEY_DIAG>(a, k, kt, X, Y, s)
-           : km == KEY_PACKED ? rct_spmm_vt<double, KEY_PACKED>(a, k, kt, X, Y, s)
-                              : rct_spmm_vt<double, KEY_SPLIT>(a, k, kt, X, Y, s);
+    auto with = [&](auto vt) {
+        using VT = decltype(vt);
+        return km == KEY_DIAG     ? rct_spmm_vt<VT, KEY_DIAG>(a, k, kt, X, Y, s)
+               : km == KEY_PACKED ? rct_spmm_vt<VT, KEY_PACKED>(a, k, kt, X, Y, s)
+                                  : rct_spmm_vt<VT, KEY_SPLIT>(a, k, kt, X, Y, s);
+    };
+    return a.pal ? with(uint8_t()) : a.vtype == 1 ? with(float()) : with(double());
 }
 
 hipError_t rct_vbar(const RctArgs &a, const double *ybar, const double *x, double *vbar, hipStream_t s) {
@@ -641,21 +660,21 @@ hipError_t rct(const RctArgs &a, const double *x, double *y, hipStream_t s, hipE
         else                                                                                         \
             rct_kernel<VT, P, false, false><<<grid, a.block, lds, s>>>(a, x, y, xr, vbar, rb, res); \
     } while (0)
-    if (a.vtype == 1) {
+    auto with = [&](auto vt) {
+        using VT = decltype(vt);
         if (km == KEY_DIAG)
-            AX_RCT_LAUNCH(float, KEY_DIAG);
+            AX_RCT_LAUNCH(VT, KEY_DIAG);
         else if (km == KEY_PACKED)
-            AX_RCT_LAUNCH(float, KEY_PACKED);
+            AX_RCT_LAUNCH(VT, KEY_PACKED);
         else
-            AX_RCT_LAUNCH(float, KEY_SPLIT);
-    } else {
-        if (km == KEY_DIAG)
-            AX_RCT_LAUNCH(double, KEY_DIAG);
-        else if (km == KEY_PACKED)
-            AX_RCT_LAUNCH(double, KEY_PACKED);
-        else
-            AX_RCT_LAUNCH(double, KEY_SPLIT);
-    }
+            AX_RCT_LAUNCH(VT, KEY_SPLIT);
+    };
+    if (a.pal)
+        with(uint8_t());
+    else if (a.vtype == 1)
+        with(float());
+    else
+        with(double());
 #undef AX_RCT_LAUNCH
     hipError_t e = hipGetLastError();
     if (partials) {

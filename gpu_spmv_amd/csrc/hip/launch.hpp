@@ -106,6 +106,9 @@ struct RctArgs {
     // 2^32)
     const uint16_t *key16 = nullptr;
     uint32_t cbits16 = 0, dmin = 0;
+    // a matrix of at most 256 different values: val holds a byte per entry,
+    // the index of its value in pal (256 doubles)
+    const double *pal = nullptr;
     // rows of many entries kept apart (nhb > 0; not with key16 or partials):
     // nheavy rows listed in hrows (and marked in hmask, a bit per row; their
     // rows of the row blocks hold no entries), cut into nhb blocks (hb_start,

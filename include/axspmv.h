@@ -233,7 +233,9 @@ enum axspmv_format {
     AXSPMV_FMT_AXT = 3, /* tiled: UNC/COM x th==1 / th>1                 */
     AXSPMV_FMT_RCT = 4  /* row-block x column-slice tiles, entries sorted
                            by column, one workgroup per tile (no reference
-                           counterpart: built for gather-bound matrices)  */
+                           counterpart: built for gather-bound matrices);
+                           a matrix of at most 256 different values keeps a
+                           byte per entry and a table of the values  */
 };
 enum axspmv_kernel {
     AXSPMV_KER_DEFAULT = 0, /* the format's own kernel                  */

@@ -525,3 +525,69 @@ def test_two_rows_per_group(fmt, kw, nrows, last):
     y = dy.download(np.float64, nrows + 1)
     assert np.isnan(y[-1])
     assert rel_err(ref, y[:-1]) <= TOL
+
+
+def _few_values(count, band):
+    """A matrix whose values are drawn from `count` different ones, among them
+    both zeros, a denormal and large ones."""
+    rng = np.random.default_rng(count)
+    m = ax.banded(4001, 5, 0.6, seed=3) if band else ax.random_sparse(4001, 0, 23, seed=4)
+    values = rng.standard_normal(count)
+    values[:4] = [-0.0, 5e-324, 1e300, 0.0][:count]
+    val = rng.choice(values, m.nnz)
+    val[:count] = values  # each one occurs
+    return ax.CsrMatrix(m.row, m.col, val, ncols=m.ncols)
+
+
+@pytest.mark.parametrize("count", [1, 2, 256, 257])
+@pytest.mark.parametrize("band,kw", [(True, {}), (True, dict(flags=ax.PLAN_RCT_WIDE_KEY)), (False, dict(tile_rows=500, slices=2)),
+                                     (False, dict(tile_rows=500, flags=ax.PLAN_RCT_SPLIT))],
+                         ids=["k16", "packed", "s2", "split"])
+def test_rct_value_table(count, band, kw):
+    """Up to 256 different values: a byte per entry; 257: the values."""
+    m = _few_values(count, band)
+    p = ax.Plan(m, ax.FMT_RCT, **dict(kw, flags=kw.get("flags", 0) | ax.PLAN_TRANSPOSE))
+    q = ax.Plan(_few_values(257, band), ax.FMT_RCT, **dict(kw, flags=kw.get("flags", 0) | ax.PLAN_TRANSPOSE))
+    per = (q.info()["stream_bytes"] - p.info()["stream_bytes"]) / m.nnz
+    assert per == (7 if count <= 256 else 0)
+    x, w = ax.uniform(17, m.ncols) * 1e-3, ax.uniform(18, m.nrows)
+    assert rel_err(orc.ncsr(m, x), ax.spmv_host(p, x)) <= TOL
+    dw, dxb = ax.DeviceBuffer.from_array(w), ax.DeviceBuffer(8 * m.ncols)
+    p.adjoint(dw, dxb)
+    assert rel_err(orc.ncsr_t(m, w, m.ncols), dxb.download(np.float64, m.ncols)) <= TOL
+
+
+def test_rct_value_table_f32():
+    """300 doubles that round to 150 floats: the table holds the floats."""
+    m = _few_values(300, False)
+    base = np.repeat(np.random.default_rng(1).standard_normal(150).astype(np.float32).astype(np.float64), 2)
+    base[1::2] = np.nextafter(base[1::2], 10)
+    val = np.random.default_rng(2).choice(base, m.nnz)
+    val[:300] = base
+    m = ax.CsrMatrix(m.row, m.col, val, ncols=m.ncols)
+    p32, p64 = (ax.Plan(m, ax.FMT_RCT, vtype=v, tile_rows=256) for v in (ax.F32, ax.F64))
+    assert (p64.info()["stream_bytes"] - p32.info()["stream_bytes"]) / m.nnz == 7
+    x = ax.uniform(19, m.ncols)
+    assert rel_err(orc.ncsr_f32val(m, x), ax.spmv_host(p32, x)) <= TOL
+    k = 6
+    X = ax.uniform(20, m.ncols * k).reshape(m.ncols, k)
+    dX, dY = ax.DeviceBuffer.from_array(X), ax.DeviceBuffer(8 * m.nrows * k)
+    p32.spmm(k, dX, dY)
+    m32 = ax.CsrMatrix(m.row, m.col, m.val.astype(np.float32).astype(np.float64), ncols=m.ncols)
+    assert rel_err(orc.spmm(m32, X), dY.download(np.float64, m.nrows * k).reshape(m.nrows, k)) <= TOL
+
+
+def test_rct_value_table_without_room():
+    """Tiles that fill the LDS leave no room for the table: plain values, and
+    SpMM at the LDS limit runs with one."""
+    m = _few_values(2, False)
+    full = ax.Plan(m, ax.FMT_RCT, tile_rows=2560)  # 2560 x 8 right-hand sides fill 160 KB
+    k = 8
+    X = ax.uniform(21, m.ncols * k).reshape(m.ncols, k)
+    dX, dY = ax.DeviceBuffer.from_array(X), ax.DeviceBuffer(8 * m.nrows * k)
+    full.spmm(k, dX, dY)
+    assert rel_err(orc.spmm(m, X), dY.download(np.float64, m.nrows * k).reshape(m.nrows, k)) <= TOL
+    n = 20480
+    d = ax.CsrMatrix(np.arange(n + 1), np.arange(n), np.ones(n))
+    x = ax.uniform(22, n)
+    assert np.array_equal(ax.spmv_host(ax.Plan(d, ax.FMT_RCT, tile_rows=n), x), x)
