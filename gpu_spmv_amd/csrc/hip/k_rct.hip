@@ -360,7 +360,7 @@ __global__ void __launch_bounds__(1024) rct_kernel(RctArgs a, const double *__re
         }
     } else if (a.part && !VB) {
         // the slice's partial vector, read once by the merge: non-temporal
-        double *ps = a.part + size_t(tile.s) * a.nrows + row0;
+        double *ps = a.part + tile.s * a.pstride + row0;
         for (uint32_t k = tid; k < rows; k += nt) __builtin_nontemporal_store(yl[k], ps + k);
     } else {
         for (uint32_t k = tid; k < rows; k += nt) unsafeAtomicAdd(out + k, yl[k]);
@@ -623,16 +623,18 @@ hipError_t rct_vbar(const RctArgs &a, const double *ybar, const double *x, doubl
 }
 
 hipError_t rct(const RctArgs &a, const double *x, double *y, hipStream_t s, hipEvent_t mid, const double *xr,
-               double *vbar, const double *rb, double *res) {
-    if (!a.nrows) return hipSuccess;
+               double *vbar, const double *rb, double *res, double *clear, size_t nclear, bool cleared) {
+    if (!a.nrows) return clear ? clear_f64(clear, nclear, s) : hipSuccess;
     if (vbar) rb = res = nullptr;  // the residual belongs to a forward pass
     const unsigned grid = rct_grid(a);
     const bool vb = vbar != nullptr;
     const size_t lds = size_t(a.R) * sizeof(double) * (vb ? 2 : 1);
     const bool partials = a.S > 1 && a.part && !vb;
     if (a.S > 1 && !partials) {
-        const hipError_t e = clear_f64(y, a.nrows, s);
-        if (e != hipSuccess) return e;
+        if (!cleared) {
+            const hipError_t e = clear_f64(y, a.nrows, s);
+            if (e != hipSuccess) return e;
+        }
         if (mid) {
             const hipError_t e = hipEventRecord(mid, s);
             if (e != hipSuccess) return e;
@@ -679,8 +681,11 @@ hipError_t rct(const RctArgs &a, const double *x, double *y, hipStream_t s, hipE
     hipError_t e = hipGetLastError();
     if (partials) {
         if (e == hipSuccess && mid) e = hipEventRecord(mid, s);
-        if (e == hipSuccess) e = part_merge(a.part, a.S, a.nrows, y, s, rb, res);
-    } else if (res && (a.S > 1 || a.nhb) && e == hipSuccess) {
+        if (e == hipSuccess) e = part_merge(a.part, a.S, a.nrows, a.pstride, y, s, rb, res, clear, nclear);
+        return e;
+    }
+    if (clear && e == hipSuccess) e = clear_f64(clear, nclear, s);
+    if (res && (a.S > 1 || a.nhb) && e == hipSuccess) {
         e = residual(a.nrows, y, rb, res, s);  // after the slices' adds
     }
     return e;

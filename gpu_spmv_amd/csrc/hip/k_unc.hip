@@ -215,7 +215,7 @@ hipError_t run(const Src &src, const axspmv::launch::SegArgs &a, const double *x
                                                             a.nrows_add, x, a.part);
         hipError_t e = hipGetLastError();
         if (e == hipSuccess && a.mid) e = hipEventRecord(a.mid, s);
-        if (e == hipSuccess) e = axspmv::launch::part_merge(a.part, a.S, a.nrows_add, y, s);
+        if (e == hipSuccess) e = axspmv::launch::part_merge(a.part, a.S, a.nrows_add, a.nrows_add, y, s);
         return e;
     }
     if (a.nrows_add) {  // column slices: clear y, then add every slice's row sums

@@ -43,31 +43,40 @@ __global__ void __launch_bounds__(256) clear_kernel(double *__restrict__ y, size
 }
 
 // y[r] = sum of the S slice partials of row r, in slice order; two rows per
-// lane (VEC: part and y 16-byte aligned, nrows even).  Non-temporal loads
-// and stores: the partials are read once, and y kept in the L2s would take
-// the room the next SpMV's x slices need (RCT on the 2^20-row power-law
-// matrix, y stored normally: 61.7 or 78.5 us per SpMV depending on where y
-// lies, as with a y cleared by ordinary stores).
+// lane (VEC: part, y, rb, res and clear 16-byte aligned, the stride between
+// partials even).  Non-temporal loads and stores: the partials are read once,
+// and y kept in the L2s would take the room the next SpMV's x slices need (RCT
+// on the 2^20-row power-law matrix, y stored normally: 61.7 or 78.5 us per
+// SpMV depending on where y lies, as with a y cleared by ordinary stores).
 // With res (a forward + adjoint pass), res = y - rb as well, stored
-// normally: the adjoint reads it next.
+// normally: the adjoint reads it next; with clear, the vector that the adjoint
+// adds into is cleared by the same lanes.
 template <bool VEC>
 __global__ void __launch_bounds__(256) merge_kernel(const double *__restrict__ part, uint32_t S, uint32_t nrows,
-                                                    double *__restrict__ y, const double *__restrict__ rb,
-                                                    double *__restrict__ res) {
+                                                    size_t stride, double *__restrict__ y,
+                                                    const double *__restrict__ rb, double *__restrict__ res,
+                                                    double *__restrict__ clear, size_t nclear) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if constexpr (VEC) {
-        if (2 * i >= nrows) return;
-        const f64x2 *p2 = reinterpret_cast<const f64x2 *>(part) + i;
+    constexpr uint32_t W = VEC ? 2 : 1;
+    for (size_t k = size_t(i) * W; k < nclear; k += size_t(gridDim.x) * blockDim.x * W) {
+        if (VEC && k + 1 < nclear)
+            __builtin_nontemporal_store(f64x2{0.0, 0.0}, reinterpret_cast<f64x2 *>(clear + k));
+        else
+            __builtin_nontemporal_store(0.0, clear + k);
+    }
+    const size_t r = size_t(i) * W;
+    if (r >= nrows) return;
+    if (VEC && r + 1 < nrows) {
+        const f64x2 *p2 = reinterpret_cast<const f64x2 *>(part + r);
         f64x2 v = __builtin_nontemporal_load(p2);
-        for (uint32_t k = 1; k < S; ++k) v += __builtin_nontemporal_load(p2 + size_t(k) * (nrows / 2));
-        __builtin_nontemporal_store(v, reinterpret_cast<f64x2 *>(y) + i);
-        if (res) reinterpret_cast<f64x2 *>(res)[i] = v - reinterpret_cast<const f64x2 *>(rb)[i];
+        for (uint32_t k = 1; k < S; ++k) v += __builtin_nontemporal_load(p2 + k * (stride / 2));
+        __builtin_nontemporal_store(v, reinterpret_cast<f64x2 *>(y + r));
+        if (res) *reinterpret_cast<f64x2 *>(res + r) = v - *reinterpret_cast<const f64x2 *>(rb + r);
     } else {
-        if (i >= nrows) return;
-        double v = __builtin_nontemporal_load(part + i);
-        for (uint32_t k = 1; k < S; ++k) v += __builtin_nontemporal_load(part + size_t(k) * nrows + i);
-        __builtin_nontemporal_store(v, y + i);
-        if (res) res[i] = v - rb[i];
+        double v = __builtin_nontemporal_load(part + r);
+        for (uint32_t k = 1; k < S; ++k) v += __builtin_nontemporal_load(part + k * stride + r);
+        __builtin_nontemporal_store(v, y + r);
+        if (res) res[r] = v - rb[r];
     }
 }
 
@@ -354,14 +363,15 @@ hipError_t clear_f64(double *y, size_t n, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t part_merge(const double *part, uint32_t S, uint32_t nrows, double *y, hipStream_t s, const double *rb,
-                      double *res) {
-    if (!nrows) return hipSuccess;
+hipError_t part_merge(const double *part, uint32_t S, uint32_t nrows, size_t stride, double *y, hipStream_t s,
+                      const double *rb, double *res, double *clear, size_t nclear) {
+    if (!nrows) return nclear ? clear_f64(clear, nclear, s) : hipSuccess;
     auto a16 = [](const void *q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
-    if (nrows % 2 == 0 && a16(part) && a16(y) && (!res || (a16(res) && a16(rb))))
-        merge_kernel<true><<<(nrows / 2 + 255) / 256, 256, 0, s>>>(part, S, nrows, y, rb, res);
+    if (!clear) nclear = 0;
+    if (stride % 2 == 0 && a16(part) && a16(y) && a16(clear) && (!res || (a16(res) && a16(rb))))
+        merge_kernel<true><<<(nrows / 2 + 256) / 256, 256, 0, s>>>(part, S, nrows, stride, y, rb, res, clear, nclear);
     else
-        merge_kernel<false><<<(nrows + 255) / 256, 256, 0, s>>>(part, S, nrows, y, rb, res);
+        merge_kernel<false><<<(nrows + 255) / 256, 256, 0, s>>>(part, S, nrows, stride, y, rb, res, clear, nclear);
     return hipGetLastError();
 }
 

@@ -98,7 +98,8 @@ struct RctArgs {
     const uint32_t *tile_ptr;
     const uint32_t *rb_start;  // nrb + 1 row-block starts
     uint32_t nrows, R, S, nrb, vtype, block, rbits, ncols;
-    double *part;  // S > 1: S x nrows slice partials (nullptr: atomic adds into y)
+    double *part;  // S > 1: S slice partials, pstride doubles apart (nullptr: atomic adds into y)
+    size_t pstride;
     uint32_t nt_stream = 0;  // 1: the tile kernel (SpMV, value-gradient sweep) streams with non-temporal loads
     // narrow bands: a 16-bit key per entry (key16 != nullptr; key, col and
     // lrow unused) with the column as an offset of cbits16 bits from sbase
@@ -125,10 +126,12 @@ struct RctArgs {
 // no partials): also vbar[e] = xr[row(e)] * x[col(e)] for every entry, in
 // entry order.  res != nullptr (vbar == nullptr): also res = y - rb, written
 // where y's rows are (the merge, or one slice's tile kernel; after the adds,
-// a pass of its own).
+// a pass of its own).  clear (vbar == nullptr): also clear[0 .. nclear) = 0, by
+// the merge where there is one; it must not overlap y, rb or res.  cleared:
+// the caller has cleared y for the adds.
 hipError_t rct(const RctArgs &a, const double *x, double *y, hipStream_t s, hipEvent_t mid = nullptr,
                const double *xr = nullptr, double *vbar = nullptr, const double *rb = nullptr,
-               double *res = nullptr);
+               double *res = nullptr, double *clear = nullptr, size_t nclear = 0, bool cleared = false);
 // Y = A X (k interleaved right-hand sides) on a one-slice plan, kt (8, 16,
 // 32 or 64) right-hand sides per launch; needs R * kt * 8 bytes of LDS
 hipError_t rct_spmm(const RctArgs &a, uint32_t k, uint32_t kt, const double *X, double *Y, hipStream_t s);
@@ -251,10 +254,11 @@ hipError_t fill_f64(double *dst, size_t n, double v, hipStream_t s);
 hipError_t fill_u32(uint32_t *dst, size_t n, uint32_t v, hipStream_t s);
 // y[0 .. n) = 0 in one pass (16-byte stores where y is 16-byte aligned)
 hipError_t clear_f64(double *y, size_t n, hipStream_t s);
-// y[r] = part[r] + part[nrows + r] + ... + part[(S - 1) nrows + r], in that
-// order; with res, also res[r] = y[r] - rb[r]
-hipError_t part_merge(const double *part, uint32_t S, uint32_t nrows, double *y, hipStream_t s,
-                      const double *rb = nullptr, double *res = nullptr);
+// y[r] = part[r] + part[stride + r] + ... + part[(S - 1) stride + r], in that
+// order; with res, also res[r] = y[r] - rb[r]; with clear, also clear[0 ..
+// nclear) = 0
+hipError_t part_merge(const double *part, uint32_t S, uint32_t nrows, size_t stride, double *y, hipStream_t s,
+                      const double *rb = nullptr, double *res = nullptr, double *clear = nullptr, size_t nclear = 0);
 // reads p[0 .. n) (n even, p 16-byte aligned): evicts caches without dirtying them
 hipError_t touch(const double *p, size_t n, double *sink, hipStream_t s);
 // the wave64 primitive op (enum axspmv_wave_op) lane by lane; n a multiple of 64

@@ -1139,11 +1139,12 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
     // atomics).  The plan of A^T, which adds into x_bar from its fused
     // value-gradient sweep, keeps the atomic adds.
     double *dpart = nullptr;
+    const size_t pstride = (size_t(n) + 1) & ~size_t(1);  // every partial 16-byte aligned: two rows per lane in the merge
     if (S > 1 && !nhb && p.lds_per_row == 8 && !(p.o.flags & AXSPMV_PLAN_RCT_ATOMIC) && 6ull * S * n >= nnz) {
-        dpart = static_cast<double *>(p.dalloc(8ull * S * n));
+        dpart = static_cast<double *>(p.dalloc(8ull * S * pstride));
         if (!dpart) return AXSPMV_E_NOMEM;
     }
-    p.rct = launch::RctArgs{dv, dc, dl, dk, dcb, dt, drb, n, R, S, nrb, p.o.vtype, block, rbits, a->ncols, dpart};
+    p.rct = launch::RctArgs{dv, dc, dl, dk, dcb, dt, drb, n, R, S, nrb, p.o.vtype, block, rbits, a->ncols, dpart, pstride};
     // A matrix stream larger than the 256 MB Infinity Cache comes from HBM
     // on every SpMV whatever the loads do: it is streamed with non-temporal
     // loads, whatever the tile height (permuted 100^3 stencil, renumbered, one
@@ -1547,6 +1548,9 @@ launch::SegArgs fused_args(const Plan &p) {
     return g;
 }
 
+// u[0 .. nu) and v[0 .. nv) do not overlap
+bool apart(const double *u, uint64_t nu, const double *v, uint64_t nv) { return u + nu <= v || v + nv <= u; }
+
 hipError_t launch_vbar(Plan *p, const double *ybar, const double *x, double *vbar, hipStream_t s) {
     // RCT: over the plan of A^T (rows = columns of A), whose entry order is
     // the one the fused forward + adjoint writes: x rows in LDS, ybar gathered
@@ -1573,6 +1577,15 @@ hipError_t launch_fwd_adj(Plan *p, const double *x, const double *b, double *y, 
         // kernel of one slice).  With the non-temporal v_bar stores of the
         // sweep over A^T, forward + adjoint on the 2^20-row power-law matrix,
         // one box: 232.6 -> 223.4 us.
+        // The merge also clears x_bar where the sweep will add slices into it.
+        const uint32_t nx = p->ncols;
+        if (fused && p->T->rct.S > 1 && apart(xbar, nx, y, p->nrows) && apart(xbar, nx, b, p->nrows) &&
+            apart(xbar, nx, r, p->nrows)) {
+            e = launch::rct(p->rct, x, y, s, nullptr, nullptr, nullptr, b, r, xbar, nx);
+            if (e == hipSuccess)
+                e = launch::rct(p->T->rct, r, xbar, s, nullptr, x, vbar, nullptr, nullptr, nullptr, 0, true);
+            return e;
+        }
         e = launch::rct(p->rct, x, y, s, nullptr, nullptr, nullptr, b, r);
     } else {
         e = plan_launch(p, x, y, s);
@@ -1669,7 +1682,7 @@ static hipError_t reordered_op(Plan *p, uint32_t op, const axspmv_operands &o, h
         double *const t[2] = {w[2], w[p->nscratch - 1]};
         return permute(p, p->to_b, launch::PermVecs{{u, v}, {w[0], w[1]}, 2, nullptr, nullptr}, t, s);
     };
-    auto apart = [&](const double *u, const double *v) { return u + p->nrows <= v || v + p->nrows <= u; };
+    auto free_of_b = [&](const double *v) { return apart(o.b, p->nrows, v, p->nrows); };
     axspmv_operands io{};
     hipError_t e = hipSuccess;
     switch (op) {
@@ -1703,7 +1716,7 @@ static hipError_t reordered_op(Plan *p, uint32_t op, const axspmv_operands &o, h
                 e = in2(o.x, o.b);
                 if (e == hipSuccess) e = plan_op(p->inner, op, io, s);
                 if (e != hipSuccess) return e;
-                if (apart(o.b, o.y) && apart(o.b, o.xbar) && apart(o.b, o.r))
+                if (free_of_b(o.y) && free_of_b(o.xbar) && free_of_b(o.r))
                     return permute(p, p->from_b, launch::PermVecs{{w[2], w[4]}, {o.y, o.xbar}, 2, o.b, o.r}, w, s);
                 double *const t[3] = {w[0], w[1], w[p->nscratch - 1]};
                 return permute(p, p->from_b, launch::PermVecs{{w[2], w[3], w[4]}, {o.y, o.r, o.xbar}, 3, nullptr, nullptr}, t, s);
@@ -1719,7 +1732,7 @@ static hipError_t reordered_op(Plan *p, uint32_t op, const axspmv_operands &o, h
             // stencil, RCT, 483.4 -> 470.0 us).
             e = in(o.x, w[0]);
             if (e == hipSuccess) e = plan_launch(p->inner, w[0], w[1], s);
-            if (!p->to_b.L && !(apart(o.b, o.y) && apart(o.b, o.r))) {  // y or r over b: r from y, then r in
+            if (!p->to_b.L && !(free_of_b(o.y) && free_of_b(o.r))) {  // y or r over b: r from y, then r in
                 if (e == hipSuccess)
                     e = permute(p, p->from_b, launch::PermVecs{{w[1]}, {o.y}, 1, o.b, o.r}, w, s);
                 if (e == hipSuccess) e = in(o.r, w[2]);
