@@ -41,7 +41,7 @@ using axspmv::launch::RctArgs;
 // Entry e of a tile: value val[e] (VT double or float; uint8_t: the value's
 // index in a table of at most 256, for matrices of few different values); its
 // column and tile row stored one of
-// three ways (KEY):
+// four ways (KEY):
 //  * KEY_SPLIT: col[e] and lrow[e];
 //  * KEY_PACKED: one word key[e] = offset << rbits | row, the column being
 //    (sbase[e >> 10] + offset) mod ncols: every run of 1024 entries has a
@@ -49,6 +49,8 @@ using axspmv::launch::RctArgs;
 //    sorted by column tile by tile, lie a short way past it -- going round
 //    from the last column to column 0 where a run passes from one row block
 //    to the next;
+//  * KEY_PACKED24: the same word in 24 bits, its low 16 in key24[e] and its
+//    high 8 in key8[e], with a base per run of 128 entries;
 //  * KEY_DIAG (narrow bands): a 16-bit key16[e] = d << cbits | offset, the
 //    column being sbase[e >> 7] + offset (the smallest column of its run of
 //    128 entries) and the row (global) column + d + dmin, where d + dmin is
@@ -58,7 +60,7 @@ using axspmv::launch::RctArgs;
 // when the matrix stream is too large to stay in the Infinity Cache from one
 // SpMV to the next; there the L2 lines it would leave behind only crowd out
 // x).
-enum : int { KEY_SPLIT = 0, KEY_PACKED = 1, KEY_DIAG = 2 };
+enum : int { KEY_SPLIT = 0, KEY_PACKED = 1, KEY_DIAG = 2, KEY_PACKED24 = 3 };
 
 template <class VT, int KEY, bool NT = false>
 struct RctEntries {
@@ -66,12 +68,14 @@ struct RctEntries {
     const uint32_t *__restrict__ key;
     const uint32_t *__restrict__ col;
     const uint16_t *__restrict__ lrow;
-    const uint16_t *__restrict__ key16;
+    const uint16_t *__restrict__ key16;  // KEY_PACKED24: key24
+    const uint8_t *__restrict__ key8;
     const uint32_t *__restrict__ sbase;
     uint32_t rbits, ncols, cbits, rofs;
     // the tile whose rows start at row0
     __device__ __forceinline__ RctEntries(const RctArgs &a, uint32_t row0)
-        : val(static_cast<const VT *>(a.val)), key(a.key), col(a.col), lrow(a.lrow), key16(a.key16),
+        : val(static_cast<const VT *>(a.val)), key(a.key), col(a.col), lrow(a.lrow),
+          key16(KEY == KEY_PACKED24 ? a.key24 : a.key16), key8(a.key8),
           sbase(a.sbase), rbits(a.rbits), ncols(a.ncols), cbits(a.cbits16), rofs(a.dmin - row0) {}
     __device__ __forceinline__ uint32_t column(uint32_t base, uint32_t off) const {
         const uint32_t room = ncols - base;  // columns from base to the end
@@ -82,8 +86,8 @@ struct RctEntries {
         r = c + (k >> cbits) + rofs;
     }
     // entries 2q and 2q + 1 with one 16-byte (8 for FP32 values, 2 for table
-    // indices) and one 8-byte (KEY_DIAG: 4-byte) load; the plan pads the
-    // arrays to an even number of entries
+    // indices) and one 8-byte load (KEY_DIAG: 4 bytes; KEY_PACKED24: 4 and 2);
+    // the plan pads the arrays to an even number of entries
     __device__ __forceinline__ void load2(uint32_t q, uint32_t (&c)[2], uint32_t (&r)[2], VT (&v)[2]) const {
         typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
         if constexpr (sizeof(VT) == 1) {
@@ -104,6 +108,17 @@ struct RctEntries {
             const uint32_t b = sbase[q >> 6];  // entries 2q, 2q + 1: one run of 128
             diag(b, k & 0xffffu, c[0], r[0]);
             diag(b, k >> 16, c[1], r[1]);
+        } else if constexpr (KEY == KEY_PACKED24) {
+            const uint32_t *pl = reinterpret_cast<const uint32_t *>(key16) + q;
+            const uint16_t *ph = reinterpret_cast<const uint16_t *>(key8) + q;
+            const uint32_t lo = NT ? __builtin_nontemporal_load(pl) : *pl;
+            const uint32_t hi = NT ? __builtin_nontemporal_load(ph) : *ph;
+            const uint32_t m = (1u << rbits) - 1, b = sbase[q >> 6];  // entries 2q, 2q + 1: one run of 128
+            const uint32_t k0 = (lo & 0xffffu) | (hi & 0xffu) << 16, k1 = lo >> 16 | hi >> 8 << 16;
+            c[0] = column(b, k0 >> rbits);
+            r[0] = k0 & m;
+            c[1] = column(b, k1 >> rbits);
+            r[1] = k1 & m;
         } else if constexpr (KEY == KEY_PACKED) {
             const u32x2 *pk = reinterpret_cast<const u32x2 *>(key) + q;
             const u32x2 k = NT ? __builtin_nontemporal_load(pk) : *pk;
@@ -127,6 +142,10 @@ struct RctEntries {
     __device__ __forceinline__ void at(uint32_t e, uint32_t &c, uint32_t &r) const {
         if constexpr (KEY == KEY_DIAG) {
             diag(sbase[e >> 7], key16[e], c, r);
+        } else if constexpr (KEY == KEY_PACKED24) {
+            const uint32_t k = key16[e] | uint32_t(key8[e]) << 16;
+            c = column(sbase[e >> 7], k >> rbits);
+            r = k & ((1u << rbits) - 1);
         } else if constexpr (KEY == KEY_PACKED) {
             const uint32_t k = key[e];
             c = column(sbase[e >> 10], k >> rbits);
@@ -144,7 +163,9 @@ __device__ __forceinline__ double entry_value(VT v, const double *table) {
     else return double(v);
 }
 
-int key_mode(const RctArgs &a) { return a.key16 ? KEY_DIAG : a.key ? KEY_PACKED : KEY_SPLIT; }
+int key_mode(const RctArgs &a) {
+    return a.key16 ? KEY_DIAG : a.key24 ? KEY_PACKED24 : a.key ? KEY_PACKED : KEY_SPLIT;
+}
 
 // Tile w of nb row blocks x S slices: XCD w % 8 takes slice (w % 8) % S; false
 // for the workgroups past the last row block.
@@ -603,9 +624,10 @@ hipError_t rct_spmm(const RctArgs &a, uint32_t k, uint32_t kt, const double *X, 
     const int km = key_mode(a);
     auto with = [&](auto vt) {
         using VT = decltype(vt);
-        return km == KEY_DIAG     ? rct_spmm_vt<VT, KEY_DIAG>(a, k, kt, X, Y, s)
-               : km == KEY_PACKED ? rct_spmm_vt<VT, KEY_PACKED>(a, k, kt, X, Y, s)
-                                  : rct_spmm_vt<VT, KEY_SPLIT>(a, k, kt, X, Y, s);
+        return km == KEY_DIAG       ? rct_spmm_vt<VT, KEY_DIAG>(a, k, kt, X, Y, s)
+               : km == KEY_PACKED24 ? rct_spmm_vt<VT, KEY_PACKED24>(a, k, kt, X, Y, s)
+               : km == KEY_PACKED   ? rct_spmm_vt<VT, KEY_PACKED>(a, k, kt, X, Y, s)
+                                    : rct_spmm_vt<VT, KEY_SPLIT>(a, k, kt, X, Y, s);
     };
     return a.pal ? with(uint8_t()) : a.vtype == 1 ? with(float()) : with(double());
 }
@@ -616,6 +638,7 @@ hipError_t rct_vbar(const RctArgs &a, const double *ybar, const double *x, doubl
     const size_t lds = size_t(a.R) * sizeof(double);
     switch (key_mode(a)) {
         case KEY_DIAG: rct_vbar_kernel<KEY_DIAG><<<grid, a.block, lds, s>>>(a, ybar, x, vbar); break;
+        case KEY_PACKED24: rct_vbar_kernel<KEY_PACKED24><<<grid, a.block, lds, s>>>(a, ybar, x, vbar); break;
         case KEY_PACKED: rct_vbar_kernel<KEY_PACKED><<<grid, a.block, lds, s>>>(a, ybar, x, vbar); break;
         default: rct_vbar_kernel<KEY_SPLIT><<<grid, a.block, lds, s>>>(a, ybar, x, vbar);
     }
@@ -648,24 +671,28 @@ hipError_t rct(const RctArgs &a, const double *x, double *y, hipStream_t s, hipE
     // plan asks for them (its v_bar stores are non-temporal anyway): the
     // permuted 128^3 stencil's forward + adjoint, renumbered, 472.8 -> 467.7
     // us, one box
-#define AX_RCT_LAUNCH(VT, P)                                                                         \
-    do {                                                                                             \
-        if (P != KEY_DIAG && a.nhb)                                                                  \
+    // (24-bit keys are for streams that are loaded the ordinary way)
+#define AX_RCT_LAUNCH(VT, P)                                                                              \
+    do {                                                                                                  \
+        constexpr bool nt = P != KEY_PACKED24;                                                            \
+        if (P != KEY_DIAG && a.nhb)                                                                       \
             rct_kernel<VT, P == KEY_DIAG ? KEY_SPLIT : P, false, false, true><<<grid, a.block, lds, s>>>( \
-                a, x, y, xr, vbar, rb, res);                                                         \
-        else if (vb && a.nt_stream)                                                                       \
-            rct_kernel<VT, P, true, true><<<grid, a.block, lds, s>>>(a, x, y, xr, vbar, rb, res);   \
-        else if (vb)                                                                                 \
-            rct_kernel<VT, P, true, false><<<grid, a.block, lds, s>>>(a, x, y, xr, vbar, rb, res);  \
-        else if (a.nt_stream)                                                                        \
-            rct_kernel<VT, P, false, true><<<grid, a.block, lds, s>>>(a, x, y, xr, vbar, rb, res);  \
-        else                                                                                         \
-            rct_kernel<VT, P, false, false><<<grid, a.block, lds, s>>>(a, x, y, xr, vbar, rb, res); \
+                a, x, y, xr, vbar, rb, res);                                                              \
+        else if (vb && nt && a.nt_stream)                                                                 \
+            rct_kernel<VT, P, true, nt><<<grid, a.block, lds, s>>>(a, x, y, xr, vbar, rb, res);           \
+        else if (vb)                                                                                      \
+            rct_kernel<VT, P, true, false><<<grid, a.block, lds, s>>>(a, x, y, xr, vbar, rb, res);        \
+        else if (nt && a.nt_stream)                                                                       \
+            rct_kernel<VT, P, false, nt><<<grid, a.block, lds, s>>>(a, x, y, xr, vbar, rb, res);          \
+        else                                                                                              \
+            rct_kernel<VT, P, false, false><<<grid, a.block, lds, s>>>(a, x, y, xr, vbar, rb, res);       \
     } while (0)
     auto with = [&](auto vt) {
         using VT = decltype(vt);
         if (km == KEY_DIAG)
             AX_RCT_LAUNCH(VT, KEY_DIAG);
+        else if (km == KEY_PACKED24)
+            AX_RCT_LAUNCH(VT, KEY_PACKED24);
         else if (km == KEY_PACKED)
             AX_RCT_LAUNCH(VT, KEY_PACKED);
         else

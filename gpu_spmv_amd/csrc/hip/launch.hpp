@@ -107,6 +107,10 @@ struct RctArgs {
     // 2^32)
     const uint16_t *key16 = nullptr;
     uint32_t cbits16 = 0, dmin = 0;
+    // a packed key of 24 bits, its low 16 in key24 and its high 8 in key8, with
+    // sbase per run of 128 entries (key24 != nullptr; key, col, lrow unused)
+    const uint16_t *key24 = nullptr;
+    const uint8_t *key8 = nullptr;
     // a matrix of at most 256 different values: val holds a byte per entry,
     // the index of its value in pal (256 doubles)
     const double *pal = nullptr;

@@ -1004,17 +1004,22 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
     std::vector<uint32_t> sbase(nseg, 0);
     const uint64_t nc = std::max<uint64_t>(1, a->ncols);
     uint64_t span = 1;
-#pragma omp parallel for schedule(static) reduction(max : span)
-    for (uint64_t g = 0; g < nseg; ++g) {
-        const uint64_t q0 = g << SEG_LOG, q1 = std::min<uint64_t>(nnz, q0 + (uint64_t(1) << SEG_LOG));
-        if (q0 >= nnz) continue;
+    // base of run g of 1 << log entries; returns the columns the run spans from it
+    auto run_base = [&](uint64_t g, uint32_t log, uint32_t &base) -> uint64_t {
+        const uint64_t q0 = g << log, q1 = std::min<uint64_t>(nnz, q0 + (uint64_t(1) << log));
+        if (q0 >= nnz) return 1;
         const auto mm = std::minmax_element(col.begin() + q0, col.begin() + q1);
         const uint64_t lin = uint64_t(*mm.second) - *mm.first + 1;  // from the smallest column
         uint64_t cyc = 1;                                            // round from the first column
-        for (uint64_t q = q0; q < q1; ++q) cyc = std::max<uint64_t>(cyc, (col[q] + nc - col[q0]) % nc + 1);
-        sbase[g] = lin <= cyc ? *mm.first : col[q0];
-        span = std::max(span, std::min(lin, cyc));
-    }
+        for (uint64_t q = q0; q < q1; ++q) {
+            const uint64_t off = col[q] >= col[q0] ? col[q] - col[q0] : col[q] + nc - col[q0];
+            cyc = std::max(cyc, off + 1);
+        }
+        base = lin <= cyc ? *mm.first : col[q0];
+        return std::min(lin, cyc);
+    };
+#pragma omp parallel for schedule(static) reduction(max : span)
+    for (uint64_t g = 0; g < nseg; ++g) span = std::max(span, run_base(g, SEG_LOG, sbase[g]));
     const uint32_t rbits = bits(R), cbits = bits(span);
     const bool packed = rbits + cbits <= 32 && !(p.o.flags & AXSPMV_PLAN_RCT_SPLIT);
     // Narrow bands: one 16-bit key per entry, the column as an offset from
@@ -1053,12 +1058,32 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
         cbits16 = bits(span16);
         diag = cbits16 + bits(uint64_t(hi - lo) + 1) <= 16;
     }
-    const uint64_t kbytes = diag ? 2 : packed ? 4 : 6;  // column and row per entry
     std::vector<double> table;
     std::vector<uint8_t> vidx;
     const bool few = uint64_t(R) * p.lds_per_row + 2048 <= lds_max && nnz &&
                      value_table(val.data(), nnz, p.o.vtype == AXSPMV_F32, table, vidx);
     const size_t vbytes = few ? 1 : vs;
+    // The packed key in 24 bits, with a base per run of 128 entries, where both
+    // fields fit and the stream of 32-bit keys takes 64 to 256 MB.  Below, it
+    // comes from the caches and the third load costs more than the bytes (FP64
+    // power-law matrix, 32 / 24 bits: 50,000 rows 9.3 / 9.5 us; random rows,
+    // 150,001, FP32 15.0 / 15.8); between, the bytes count, most of all where
+    // they let the stream stay in the Infinity Cache (power-law, 400,000 rows
+    // 40.1 / 37.9 us; 2^20 rows 86.8 / 85.8, run again and again 59.8 / 54.7,
+    // FP32 78.3 / 74.9; random, 450,007 rows, FP32 38.5 / 33.3); above, with
+    // non-temporal loads, it is level or slightly behind (1.4M rows 160.0 / 161.0).
+    const uint64_t stream32 = nnz * (4 + vbytes);
+    std::vector<uint32_t> sbase24;
+    bool key24 = packed && !diag && rbits < 24 && !(p.o.flags & AXSPMV_PLAN_RCT_WIDE_KEY) &&
+                 stream32 >= (64ull << 20) && stream32 <= (256ull << 20);
+    if (key24) {
+        sbase24.assign(nseg16, 0);
+        uint64_t span24 = 1;
+#pragma omp parallel for schedule(static) reduction(max : span24)
+        for (uint64_t g = 0; g < nseg16; ++g) span24 = std::max(span24, run_base(g, DSEG_LOG, sbase24[g]));
+        key24 = rbits + bits(span24) <= 24;
+    }
+    const uint64_t kbytes = diag ? 2 : key24 ? 3 : packed ? 4 : 6;  // column and row per entry
     // one spare entry when nnz is odd: a kernel may load entries in aligned pairs
     const uint64_t nnz_pad = nnz + (nnz & 1);
     void *dv = p.dalloc(vbytes * nnz_pad);
@@ -1084,7 +1109,8 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
     }
     AX_TRY(p.upload(dt, tptr.data(), 4 * tptr.size(), s));
     uint32_t *dc = nullptr, *dk = nullptr, *dcb = nullptr;
-    uint16_t *dl = nullptr, *dk16 = nullptr;
+    uint16_t *dl = nullptr, *dk16 = nullptr, *dk24 = nullptr;
+    uint8_t *dk8 = nullptr;
     if (diag) {
         std::vector<uint16_t> key(nnz);
 #pragma omp parallel for schedule(dynamic, 1)
@@ -1098,6 +1124,23 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
         if (!dk16 || !dcb) return AXSPMV_E_NOMEM;
         AX_TRY(p.upload(dk16, key.data(), 2 * nnz, s));
         AX_TRY(p.upload(dcb, sbase16.data(), 4 * nseg16, s));
+    } else if (key24) {
+        std::vector<uint16_t> lo(nnz);
+        std::vector<uint8_t> hi(nnz);
+#pragma omp parallel for schedule(static)
+        for (uint64_t q = 0; q < nnz; ++q) {
+            const uint64_t b = sbase24[q >> DSEG_LOG], off = col[q] >= b ? col[q] - b : col[q] + nc - b;
+            const uint32_t k = uint32_t(off << rbits) | lrow[q];
+            lo[q] = uint16_t(k);
+            hi[q] = uint8_t(k >> 16);
+        }
+        dk24 = static_cast<uint16_t *>(p.dalloc(2 * nnz_pad));
+        dk8 = static_cast<uint8_t *>(p.dalloc(nnz_pad));
+        dcb = static_cast<uint32_t *>(p.dalloc(4 * nseg16));
+        if (!dk24 || !dk8 || !dcb) return AXSPMV_E_NOMEM;
+        AX_TRY(p.upload(dk24, lo.data(), 2 * nnz, s));
+        AX_TRY(p.upload(dk8, hi.data(), nnz, s));
+        AX_TRY(p.upload(dcb, sbase24.data(), 4 * nseg16, s));
     } else if (packed) {
         std::vector<uint32_t> key(nnz ? nnz : 1);
 #pragma omp parallel for schedule(static)
@@ -1157,6 +1200,8 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
     p.rct.pal = dpal;
     p.rct.nt_stream = (vbytes + kbytes) * nnz > (256ull << 20) ? 1 : 0;
     p.rct.key16 = dk16;
+    p.rct.key24 = dk24;
+    p.rct.key8 = dk8;
     p.rct.cbits16 = cbits16;
     p.rct.dmin = uint32_t(uint64_t(dlo));
     if (nhb) {

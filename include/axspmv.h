@@ -359,7 +359,9 @@ typedef struct axspmv_opts {
                                     Q costs a few breadth-first passes over
                                     A on the host. */
 #define AXSPMV_PLAN_RCT_WIDE_KEY 128u /* RCT: keep the 32-bit key where a
-                                    16-bit one would fit.  By default a
+                                    16- or 24-bit one would fit.  By default
+                                    a stream of 64 to 256 MB takes 24 bits
+                                    where they are enough, and a
                                     matrix whose entries lie close to the
                                     diagonal (a band of up to about 127 on
                                     each side) stores each entry's column and

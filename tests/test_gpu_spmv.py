@@ -591,3 +591,86 @@ def test_rct_value_table_without_room():
     d = ax.CsrMatrix(np.arange(n + 1), np.arange(n), np.ones(n))
     x = ax.uniform(22, n)
     assert np.array_equal(ax.spmv_host(ax.Plan(d, ax.FMT_RCT, tile_rows=n), x), x)
+
+
+def _uneven(n, per, ncols, seed):
+    """Rows of 0 .. 2 * per entries in random order of length, an odd number
+    of entries in all, columns anywhere."""
+    rng = np.random.default_rng(seed)
+    length = rng.integers(0, 2 * per + 1, n)
+    length[-1] += 1 - int(length.sum()) % 2
+    row = np.concatenate([[0], np.cumsum(length)]).astype(np.uint32)
+    col = rng.integers(0, ncols, row[-1]).astype(np.uint32)
+    return ax.CsrMatrix(row, col, rng.standard_normal(row[-1]), ncols=ncols)
+
+
+@pytest.mark.parametrize("n,per,ncols,kw,few,bits", [
+    # a run of 128 entries covers ncols / 8000 x 128 / R columns: 9 + 15 bits
+    # at most at 400 rows, 14 + 10 at 16,000
+    (300001, 20, 300001, dict(tile_rows=400), False, 8),
+    (300001, 20, 300001, dict(tile_rows=16000), False, 8),
+    (300001, 20, 300001, dict(tile_rows=16000, slices=4), False, 8),
+    (300001, 20, 300001, dict(tile_rows=1), False, 8),       # 1 + 19 bits: runs over many tiles
+    (450007, 20, 450007, dict(vtype=ax.F32), False, 8),
+    (700001, 20, 700001, {}, True, 8),                        # values from a table, 5 bytes an entry
+    (1200001, 5, 1200001, dict(tile_rows=16000), False, 0),   # runs over 30,000 columns: 14 + 15 bits
+    (270001, 20, 270001, dict(tile_rows=400), False, 0),      # less than 64 MB
+], ids=["r400", "r16000", "s4", "r1", "f32", "table", "wide", "small"])
+def test_rct_key24(n, per, ncols, kw, few, bits):
+    """A stream of 64 to 256 MB takes 24-bit keys where they are enough, with
+    the products, the adjoint and the value gradient of 32-bit ones."""
+    m = _uneven(n, per, ncols, seed=n)
+    if few:
+        m = ax.CsrMatrix(m.row, m.col, np.sign(m.val), ncols=ncols)
+    p = ax.Plan(m, ax.FMT_RCT, **kw)
+    q = ax.Plan(m, ax.FMT_RCT, flags=ax.PLAN_RCT_WIDE_KEY, **kw)
+    saved = 8 * (q.info()["stream_bytes"] - p.info()["stream_bytes"]) / m.nnz
+    assert abs(saved - bits) < 0.3, saved  # less a base per 128 entries
+    x = ax.uniform(23, ncols)
+    ref = (orc.ncsr_f32val if kw.get("vtype") == ax.F32 else orc.ncsr)(m, x)
+    assert rel_err(ref, ax.spmv_host(p, x)) <= TOL
+    if kw.get("tile_rows", n) > 2560:
+        return  # no room for the sums of a k-tile of 8
+    dX, dY = ax.DeviceBuffer.from_array(ax.uniform(24, ncols * 2)), ax.DeviceBuffer(16 * n)
+    out = []
+    for plan in (p, q):
+        plan.spmm(2, dX, dY)
+        out.append(dY.download(np.float64, 2 * n))
+    assert rel_err(out[1], out[0]) <= TOL
+
+
+def test_rct_key24_gradients():
+    m = _uneven(300001, 20, 290003, seed=25)
+    p = ax.Plan(m, ax.FMT_RCT, flags=ax.PLAN_TRANSPOSE)
+    x, b = ax.uniform(25, m.ncols), ax.uniform(26, m.nrows)
+    dx, db = ax.DeviceBuffer.from_array(x), ax.DeviceBuffer.from_array(b)
+    for fused in (True, False):
+        dy, dr, dxb, dvb = (ax.DeviceBuffer.from_array(np.full(s, np.nan)) for s in (m.nrows, m.nrows, m.ncols, m.nnz))
+        p.fwd_adj(dx, db, dy, dr, dxb, dvb, fused=fused)
+        r = dr.download(np.float64, m.nrows)
+        assert rel_err(orc.ncsr(m, x) - b, r) <= TOL
+        assert rel_err(orc.ncsr_t(m, r, m.ncols), dxb.download(np.float64, m.ncols)) <= TOL
+        assert np.array_equal(p.vbar_csr(dvb.download(np.float64, m.nnz)), orc.vbar(m, r, x))
+
+
+def test_rct_fused_clear_of_x_bar():
+    """The adjoint of a sliced plan adds into x_bar: cleared by the forward's
+    merge, rows an odd number, x_bar longer or shorter than y -- or, where
+    x_bar shares memory with b, not before b is read."""
+    for n, nc in ((20001, 20001), (4097, 40000), (30000, 4097)):
+        m = _uneven(n, 12, nc, seed=nc)
+        p = ax.Plan(m, ax.FMT_RCT, flags=ax.PLAN_TRANSPOSE, slices=4, tile_rows=512)
+        x, b = ax.uniform(27, nc), ax.uniform(28, n)
+        r_ref = orc.ncsr(m, x) - b
+        xb_ref = orc.ncsr_t(m, r_ref, nc)
+        for shared in (False, True):
+            dx, dm = ax.DeviceBuffer.from_array(x), ax.DeviceBuffer.from_array(np.concatenate([b, np.full(nc + n, np.nan)]))
+            dy, dr, dvb = (ax.DeviceBuffer(8 * s) for s in (n, n, m.nnz))
+            xb = dm.ptr if shared else dm.ptr + 8 * n
+            p.fwd_adj(dx, dm.ptr, dy, dr, xb, dvb, fused=True)
+            ax._lib.call("axspmv_device_sync")
+            assert rel_err(r_ref, dr.download(np.float64, n)) <= TOL
+            got = dm.download(np.float64, nc + 2 * n)
+            assert rel_err(xb_ref, got[:nc] if shared else got[n:n + nc]) <= 1e-11
+            if not shared:
+                assert np.array_equal(got[:n], b) and np.all(np.isnan(got[n + nc:]))
