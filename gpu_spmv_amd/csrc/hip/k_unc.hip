@@ -61,7 +61,21 @@ __global__ void __launch_bounds__(256) rowblock_slices_kernel(Src src, const Blo
                                                               double *__restrict__ y) {
     const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     if (wave >= nblocks) return;
-    rowblock_process<Src, XGlobal, true>(src, blocks[wave], XGlobal{x}, y);
+    rowblock_process<Src, XGlobal, Put::ATOMIC>(src, blocks[wave], XGlobal{x}, y);
+}
+
+// One slice after another, all XCDs on the same one, the first stored as
+// rows are, the next added to y: bit-identical results from call to call, and
+// nothing held between launches.  Gathers from L2 (about 213 G/s at 4 MB of
+// x) and the stream share a CU's outstanding loads, so a slice's two times
+// add up: 2^20-row power-law matrix, two slices, 98 + 45 of 162 us (in row
+// order 209).
+template <class Src>
+__global__ void __launch_bounds__(256) rowblock_next_kernel(Src src, const Block *__restrict__ blocks, uint32_t nblocks,
+                                                            const double *__restrict__ x, double *__restrict__ y) {
+    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    if (wave >= nblocks) return;
+    rowblock_process<Src, XGlobal, Put::ADD>(src, blocks[wave], XGlobal{x}, y);
 }
 
 // The deterministic form: slice s's row sums are stored (not added) into
@@ -81,7 +95,7 @@ __global__ void __launch_bounds__(256) rowblock_partial_kernel(Src src, const Bl
     for (uint32_t i = wave * 64 + lane; i < nempty; i += nwaves * 64) part[empty[i]] = 0.0;
     if (wave >= nblocks) return;
     double *ys = part + size_t((blockIdx.x % 8) % S) * nrows;
-    rowblock_process<Src, XGlobal, false>(src, blocks[wave], XGlobal{x}, ys);
+    rowblock_process(src, blocks[wave], XGlobal{x}, ys);
 }
 
 // ------------------------------------------------------------------ adjoint
@@ -210,6 +224,19 @@ hipError_t run(const Src &src, const axspmv::launch::SegArgs &a, const double *x
     const uint32_t block = 256;  // 4 waves: the LDS windows are indexed by wave
     uint32_t waves = a.nblocks ? a.nblocks : 1;
     const unsigned grid = (waves + block / 64 - 1) / (block / 64);
+    if (a.seq) {  // column slices, one after another
+        for (uint32_t k = 0; k < a.S; ++k) {
+            const uint32_t n = a.seq[k + 1] - a.seq[k];
+            const unsigned groups = n ? (n + 3) / 4 : 1;  // the first slice also zeroes the rows without entries in it
+            if (!k)
+                rowblock_kernel<Src, false><<<groups, block, 0, s>>>(src, a.blocks, n, a.empty, a.nempty, nullptr, x, y);
+            else
+                rowblock_next_kernel<Src><<<groups, block, 0, s>>>(src, a.blocks + a.seq[k], n, x, y);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
     if (a.part) {  // column slices, deterministic: partials, then their sum in slice order
         rowblock_partial_kernel<Src><<<grid, block, 0, s>>>(src, a.blocks, a.nblocks, a.empty, a.nempty, a.S,
                                                             a.nrows_add, x, a.part);

@@ -43,6 +43,8 @@ struct SegArgs {
                               // rows without entries in slice s), summed in
                               // slice order by a merge kernel
     uint32_t S;               // column slices (with part)
+    const uint32_t *seq = nullptr;  // column slices one after another: slice k is
+                              // blocks seq[k] .. seq[k + 1] (host memory, S + 1)
     uint32_t nt = 0;          // AXT UNC: 1 streams the planes with
                               // non-temporal loads
 };

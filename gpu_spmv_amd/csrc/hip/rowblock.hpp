@@ -213,17 +213,21 @@ struct UncHSrc {
     __device__ __forceinline__ uint32_t row(uint32_t g) const { return sec[g]; }
 };
 
-// ADD: the block holds the row sums of one column slice; they are added to
-// y (cleared beforehand) with FP64 atomics instead of stored.
-template <bool ADD>
+// How a block's row sums go to y: stored; or, where they are the sums of one
+// column slice, added with FP64 atomics (all slices at once, y cleared
+// beforehand) or plainly (one slice after another).
+enum class Put { STORE, ATOMIC, ADD };
+template <Put P>
 __device__ __forceinline__ void put_row(double *__restrict__ y, uint32_t r, double v) {
-    if constexpr (ADD)
+    if constexpr (P == Put::ATOMIC)
         unsafeAtomicAdd(y + r, v);
+    else if constexpr (P == Put::ADD)
+        y[r] += v;
     else
         y[r] = v;
 }
 
-template <class Src, class XA, bool ADD = false>
+template <class Src, class XA, Put P = Put::STORE>
 __device__ __forceinline__ void rowblock_process(const Src &src, const Block b, const XA &x, double *__restrict__ y) {
     const uint32_t lane = threadIdx.x & 63;
     uint32_t crow = NOROW;  // row of the segment still open at the end of the previous 64 units
@@ -240,7 +244,7 @@ __device__ __forceinline__ void rowblock_process(const Src &src, const Block b, 
         // The carried segment ends here if these units start with another row.
         const uint32_t r0 = readfirst_u32(r);
         if (crow != NOROW && r0 != crow) {
-            if (lane == 0) put_row<ADD>(y, crow, carry);
+            if (lane == 0) put_row<P>(y, crow, carry);
             crow = NOROW;
             carry = 0.0;
         }
@@ -250,7 +254,7 @@ __device__ __forceinline__ void rowblock_process(const Src &src, const Block b, 
         const bool last = u0 + 64 >= b.end;
         bool end = act && shift_down_u32(r, NOROW) != r;
         if (!last && lane == 63) end = false;
-        if (end) put_row<ADD>(y, r, v);
+        if (end) put_row<P>(y, r, v);
         if (!last) {
             crow = readlane_u32(r, 63);
             carry = readlane_f64(v, 63);

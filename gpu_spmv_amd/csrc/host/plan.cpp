@@ -45,6 +45,7 @@ int axspmv_plan::upload(void *dst, const void *src, size_t bytes, hipStream_t s)
 axspmv_plan::~axspmv_plan() {
     delete T;
     delete Tdet;
+    delete by_slice;
     delete inner;
     for (void *p : bufs) (void)hipFree(p);
 }
@@ -364,8 +365,7 @@ int upload_ax_layout(Plan &p, const axspmv_csr *a, const axspmv_axt *m, hipStrea
 
 // AXT UNC th == 1 in S column slices: slice k holds the entries of columns
 // [k C, (k + 1) C) (C = ceil(ncols / S)) and is the AXT layout of that part
-// of the matrix, built by the same builder (global column indices, so x is
-// indexed directly).  The slices' planes and sec arrays are concatenated;
+// of the matrix (global column indices, so x is indexed directly).  The slices' planes and sec arrays are concatenated;
 // every slice gets its own row-aligned wave blocks (unit offsets moved to the
 // concatenated planes).  The dispatch list gives workgroup g (four waves,
 // four blocks) slice (g % 8) % S, and workgroups run on XCD g % 8, so an XCD
@@ -394,7 +394,9 @@ uint32_t axt_stream_nt(const axspmv_csr *a, uint64_t stream_bytes) {
     return stream_bytes > (256ull << 20) && wide_gathers(a) ? 1 : 0;
 }
 
-int plan_axt_sliced(Plan &p, const axspmv_csr *a, hipStream_t s) {
+// one_by_one: the slices run one after another, each on all XCDs, and add
+// their row sums plainly (no atomics, the order of the additions is fixed).
+int plan_axt_sliced(Plan &p, const axspmv_csr *a, bool one_by_one, hipStream_t s) {
     const uint32_t thw = p.o.thw, S = p.o.slices, n = a->nrows;
     if (S != 2 && S != 4 && S != 8) return fail(AXSPMV_E_UNSUPPORTED, "AXT column slices must be 2, 4 or 8, got %u", S);
     const uint64_t C = ceil_div(std::max<uint32_t>(a->ncols, 1), S);
@@ -402,51 +404,50 @@ int plan_axt_sliced(Plan &p, const axspmv_csr *a, hipStream_t s) {
     const size_t vs = p.o.vtype == AXSPMV_F32 ? 4 : 8;
     // entries of each row by slice
     std::vector<uint32_t> cnt(size_t(S) * n, 0);
+#pragma omp parallel for schedule(dynamic, 4096)
     for (uint32_t r = 0; r < n; ++r)
         for (uint32_t j = a->row[r]; j < a->row[r + 1]; ++j) cnt[size_t(a->col[j] / C) * n + r]++;
-    std::vector<double> vcat;
-    std::vector<uint32_t> ccat, scat;
+    // planes: first slot of every row's part of every slice, then the parts
     std::vector<std::vector<launch::Block>> sblocks(S);
-    uint64_t units_before = 0;
+    std::vector<uint32_t> at(size_t(S) * n);
+    std::vector<uint32_t> units(n);
+    uint64_t slots = 0;
     for (uint32_t k = 0; k < S; ++k) {
-        axspmv_csr sub{};
-        sub.nrows = n;
-        sub.ncols = a->ncols;
-        std::vector<uint32_t> row(size_t(n) + 1, 0), col;
-        std::vector<double> val;
-        for (uint32_t r = 0; r < n; ++r) row[r + 1] = row[r] + cnt[size_t(k) * n + r];
-        col.resize(row[n]);
-        val.resize(row[n]);
+        const uint64_t s0 = slots;
         for (uint32_t r = 0; r < n; ++r) {
-            uint32_t q = row[r];
-            for (uint32_t j = a->row[r]; j < a->row[r + 1]; ++j)
-                if (a->col[j] / C == k) {
-                    col[q] = a->col[j];
-                    val[q++] = a->val[j];
-                }
+            const uint64_t tiles = ceil_div(cnt[size_t(k) * n + r], thw);
+            at[size_t(k) * n + r] = uint32_t(slots);
+            units[r] = uint32_t(tiles * (thw / K));
+            slots += tiles * thw;
         }
-        sub.nnz = row[n];
-        sub.row = row.data();
-        sub.col = col.data();
-        sub.val = val.data();
-        axspmv_axt *m = nullptr;
-        AX_TRY(axspmv_build_axt(&sub, nullptr, p.o.bs, thw, 1, AXSPMV_AXT_UNC,
-                               AXSPMV_BUILD_PLANES | AXSPMV_BUILD_PAD_COL, &m, nullptr));
-        std::unique_ptr<axspmv_axt, void (*)(axspmv_axt *)> guard(m, axspmv_axt_free);
-        if (vcat.size() + m->lenAX / 2 >= (1ull << 32))
-            return fail(AXSPMV_E_OVERFLOW, "AXT slices: %llu slots exceed 32 bits",
-                        (unsigned long long)(vcat.size() + m->lenAX / 2));
-        vcat.insert(vcat.end(), m->vplane, m->vplane + m->lenAX / 2);
-        ccat.insert(ccat.end(), m->cplane, m->cplane + m->lenAX / 2);
-        scat.insert(scat.end(), m->sec, m->sec + m->lenSEC);
-        std::vector<uint32_t> units(n);
-        for (uint32_t r = 0; r < n; ++r) units[r] = uint32_t(ceil_div(cnt[size_t(k) * n + r], thw) * (thw / K));
+        if (2 * (slots - s0) >= (1ull << 32) || slots >= (1ull << 32))
+            return fail(AXSPMV_E_OVERFLOW, "AXT slices: %llu slots exceed 32 bits", (unsigned long long)slots);
         sblocks[k] = row_blocks(units, p.o.budget ? p.o.budget : 64);
         for (launch::Block &b : sblocks[k]) {
-            b.beg += uint32_t(units_before);
-            b.end += uint32_t(units_before);
+            b.beg += uint32_t(s0 / K);
+            b.end += uint32_t(s0 / K);
         }
-        units_before += uint64_t(m->lenAX / 2) / K;
+    }
+    const std::unique_ptr<double[]> vcat(new double[slots ? slots : 1]);
+    const std::unique_ptr<uint32_t[]> ccat(new uint32_t[slots ? slots : 1]), scat(new uint32_t[slots / thw + 1]);
+    const uint64_t nsec = slots / thw;
+#pragma omp parallel for schedule(dynamic, 4096)
+    for (uint32_t r = 0; r < n; ++r) {
+        uint32_t q[8];
+        for (uint32_t k = 0; k < S; ++k) {
+            q[k] = at[size_t(k) * n + r];
+            const uint32_t c = cnt[size_t(k) * n + r], tiles = uint32_t(ceil_div(c, thw));
+            for (uint32_t t = 0; t < tiles; ++t) scat[q[k] / thw + t] = r;
+            for (uint32_t i = c; i < tiles * thw; ++i) {
+                vcat[q[k] + i] = 0.0;
+                ccat[q[k] + i] = AXSPMV_PAD_COL;
+            }
+        }
+        for (uint32_t j = a->row[r]; j < a->row[r + 1]; ++j) {
+            const uint32_t w = q[a->col[j] / C]++;
+            vcat[w] = a->val[j];
+            ccat[w] = a->col[j];
+        }
     }
     // dispatch list: workgroup g takes blocks 4i .. 4i + 3 of slice (g % 8) % S,
     // i = (g / 8) * (8 / S) + (g % 8) / S; missing blocks are empty
@@ -461,15 +462,26 @@ int plan_axt_sliced(Plan &p, const axspmv_csr *a, hipStream_t s) {
         for (uint32_t w = 0; w < 4; ++w)
             if (4 * i + w < sblocks[k].size()) list[4 * g + w] = sblocks[k][4 * i + w];
     }
+    if (one_by_one) {  // slice after slice
+        list.clear();
+        p.seq.assign(1, 0);
+        for (const auto &b : sblocks) {
+            list.insert(list.end(), b.begin(), b.end());
+            p.seq.push_back(uint32_t(list.size()));
+        }
+    }
     if (list.size() >= (1ull << 32) / 64) return fail(AXSPMV_E_OVERFLOW, "AXT slices: too many wave blocks");
-    AX_TRY(upload_planes(p, vcat.data(), ccat.data(), vcat.size(), s));
-    p.d_sec = static_cast<uint32_t *>(p.dalloc(4ull * scat.size()));
+    AX_TRY(upload_planes(p, vcat.get(), ccat.get(), slots, s));
+    p.d_sec = static_cast<uint32_t *>(p.dalloc(4 * nsec));
     if (!p.d_sec) return AXSPMV_E_NOMEM;
-    AX_TRY(p.upload(p.d_sec, scat.data(), 4ull * scat.size(), s));
+    AX_TRY(p.upload(p.d_sec, scat.get(), 4 * nsec, s));
     // Deterministic: slice partials stored in part[k * n + r] (0 for the rows
     // without entries in slice k), summed in slice order by a merge kernel.
     const bool det = p.o.flags & AXSPMV_PLAN_DETERMINISTIC;
     std::vector<uint32_t> empty;
+    if (!p.seq.empty())
+        for (uint32_t r = 0; r < n; ++r)
+            if (!cnt[r]) empty.push_back(r);
     if (det) {
         if (uint64_t(S) * n >= (1ull << 32)) return fail(AXSPMV_E_OVERFLOW, "AXT slices: S x nrows exceeds 32 bits");
         for (uint32_t k = 0; k < S; ++k)
@@ -482,13 +494,97 @@ int plan_axt_sliced(Plan &p, const axspmv_csr *a, hipStream_t s) {
     p.thw = thw;
     p.th = 1;
     p.slices = S;
-    p.slots = vcat.size();
-    p.stream_bytes = (vs + 4) * p.slots + 4ull * scat.size() + 8ull * list.size();
+    p.stream_bytes = (vs + 4) * p.slots + 4 * nsec + 8ull * list.size();
     p.seg_nt = axt_stream_nt(a, p.stream_bytes);
-    p.launches = 2;
+    p.launches = one_by_one ? S : 2;
     p.kind = Plan::AXT_UNC_H1_SLICED;
     std::snprintf(p.name, sizeof p.name, "axt_unc_h1_thw%u_s%u%s", thw, S, det ? "_det" : "");
     return AXSPMV_OK;
+}
+
+// At least half of the entries lie outside the 2 MB of x (in pieces of 64 KB)
+// that their block of 16,384 rows reads most of: gathers without locality,
+// wherever a local matrix has its bands or blocks.
+bool scattered(const axspmv_csr *a) {
+    constexpr uint32_t PIECE_LOG = 13, PIECES = 32, ROWS = 16384;
+    const uint32_t np = (a->ncols >> PIECE_LOG) + 1, nb = uint32_t(ceil_div(a->nrows, ROWS));
+    uint64_t far = 0;
+#pragma omp parallel reduction(+ : far)
+    {
+        std::vector<uint32_t> cnt(np);
+#pragma omp for schedule(dynamic, 1)
+        for (uint32_t b = 0; b < nb; ++b) {
+            std::fill(cnt.begin(), cnt.end(), 0);
+            const uint32_t r1 = uint32_t(std::min<uint64_t>(a->nrows, uint64_t(b + 1) * ROWS));
+            for (uint32_t j = a->row[b * ROWS]; j < a->row[r1]; ++j) cnt[a->col[j] >> PIECE_LOG]++;
+            if (np <= PIECES) continue;
+            std::nth_element(cnt.begin(), cnt.begin() + PIECES, cnt.end(), std::greater<uint32_t>());
+            for (uint32_t k = PIECES; k < np; ++k) far += cnt[k];
+        }
+    }
+    return 2 * far >= a->nnz;
+}
+
+// Column slices that the SpMV of an AXT UNC th == 1 plan runs one after
+// another, or 1.  Where x outgrows an L2 (4 MB), row-order gathers go to the
+// Infinity Cache at 54 G lines/s, whatever the kernel; a slice of at most 4
+// MB is gathered from L2.  A slice costs tile padding and a pass over y: at
+// least two entries per row and slice.  All slices at once, by XCD, is no
+// alternative: those add with atomics (random rounding) or need partial sums
+// in the plan (calls that overlap would race).  One box, FP64, without / with:
+// power-law, 660,000 rows 106.5 / 105.6 us (run again and again 96.2 / 80.0),
+// 750,000 129.6 / 120.7 (121.0 / 92.6), 2^20 209.5 / 163.0, 3M 920 / 550;
+// permuted 100^3 stencil 270 / 194; random, 10^6 rows of 6 74.4 / 61.6.  Below
+// two entries: 2M rows of 2 72.7 / 81.8; 4M of 5, 4 slices 350 / 328, 8 slices
+// 350 (so 2).
+uint32_t axt_slices(const axspmv_csr *a) {
+    constexpr uint64_t SLICE = (4ull << 20) / 8;
+    if (a->ncols < 5 * SLICE / 4 || !a->nnz) return 1;
+    uint32_t S = 2;
+    while (S < 8 && ceil_div(a->ncols, S) > SLICE) S *= 2;
+    while (S > 1 && a->nnz < 2ull * S * a->nrows) S /= 2;
+    return S > 1 && scattered(a) ? S : 1;
+}
+
+// The plan's SpMV in column slices (a copy of the matrix), where axt_slices
+// finds it worth while and a quarter of the free memory holds it.  The planes
+// in row order stay for the value gradient and SpMM.  Streams of more than 200
+// MB are loaded non-temporally (power-law, without / with, one matrix after
+// another and, in brackets, one again and again: 2^20 rows 177.9 / 163.1 us,
+// 900,000 151.2 / 136.8 (134.7 / 136.6), 750,000 124.8 / 112.0 (93.3 / 112.0)).
+// Two slots per tile pad least: right for short rows and for the larger FP64
+// streams (2^20 rows, 2 / 4 slots 163.0 / 168.6 us); else four, with half the
+// load instructions (FP64, 750,000 rows 124.8 / 120.7; FP32, 2^20 rows 167.7 /
+// 158.1; random rows of 6 61.7 / 65.2).
+void axt_add_slices(Plan &p, const axspmv_csr *a, hipStream_t s) {
+    const uint32_t S = axt_slices(a);
+    size_t avail = 0, total = 0;
+    if (S == 1 || hipMemGetInfo(&avail, &total) != hipSuccess || 4ull * 16 * (a->nnz + uint64_t(S) * a->nrows) > avail) return;
+    auto q = std::make_unique<Plan>();
+    q->o = p.o;
+    const uint64_t vs = p.o.vtype == AXSPMV_F32 ? 4 : 8, cut = uint64_t(S) * a->nrows;  // rows of all slices
+    const bool nt = (vs + 4) * (a->nnz + cut / 2) > (200ull << 20);
+    q->o.thw = a->nnz < 6 * cut || (nt && vs == 8) ? 2 : 4;
+    q->o.slices = S;
+    q->o.flags &= ~AXSPMV_PLAN_DETERMINISTIC;
+    q->device = p.device;
+    q->nrows = p.nrows;
+    q->ncols = p.ncols;
+    q->nnz = p.nnz;
+    int rc = AXSPMV_E_NOMEM;
+    try {
+        rc = plan_axt_sliced(*q, a, true, s);
+    } catch (const std::bad_alloc &) {
+    }
+    if (rc) {  // no memory after all: row order
+        (void)hipGetLastError();
+        return;
+    }
+    q->seg_nt = nt;
+    p.device_bytes += q->device_bytes;
+    p.stream_bytes = q->stream_bytes;
+    p.launches = S;
+    p.by_slice = q.release();
 }
 
 int plan_axt(Plan &p, const axspmv_csr *a, hipStream_t s) {
@@ -500,7 +596,7 @@ int plan_axt(Plan &p, const axspmv_csr *a, hipStream_t s) {
     if (p.o.slices > 1) {
         if (th != 1 || p.o.mode != AXSPMV_AXT_UNC || axl || (p.o.flags & AXSPMV_PLAN_STAGE_X))
             return fail(AXSPMV_E_UNSUPPORTED, "AXT column slices: UNC th = 1 only, without the AX layout or x staging");
-        return plan_axt_sliced(p, a, s);
+        return plan_axt_sliced(p, a, false, s);
     }
     if (p.o.mode == AXSPMV_AXT_COM) return plan_axt_com(p, a, s);
     axspmv_axt *m = nullptr;
@@ -577,7 +673,9 @@ int plan_axt(Plan &p, const axspmv_csr *a, hipStream_t s) {
     p.d_fblocks = static_cast<launch::Block *>(p.dalloc(sizeof(launch::Block) * fb.size()));
     if (!p.d_fblocks) return AXSPMV_E_NOMEM;
     AX_TRY(p.upload(p.d_fblocks, fb.data(), sizeof(launch::Block) * fb.size(), s));
-    return setup_rowwise(p, a, d_first, p.d_vplane, p.d_cplane, s);
+    AX_TRY(setup_rowwise(p, a, d_first, p.d_vplane, p.d_cplane, s));
+    if (!p.d_win) axt_add_slices(p, a, s);
+    return AXSPMV_OK;
 }
 
 // Steps of one 64-lane K1 work item at most; longer chunks are split.
@@ -1542,9 +1640,12 @@ hipError_t plan_launch(axspmv_plan *p, const double *x, double *y, hipStream_t s
         case Plan::CSR_VECTOR:
             return launch::csr_vector(p->nrows, p->d_val, p->o.vtype, p->d_col, p->d_row, p->lanes, p->spmm.long_slots,
                                       p->spmm.longrows, p->spmm.nlong, x, y, s, p->seg_nt);
-        case Plan::AXT_UNC_H1: return launch::axt_unc_h1(seg_args(*p, p->d_sec), x, y, s);
+        case Plan::AXT_UNC_H1:
+            if (p->by_slice) return plan_launch(p->by_slice, x, y, s);
+            return launch::axt_unc_h1(seg_args(*p, p->d_sec), x, y, s);
         case Plan::AXT_UNC_H1_SLICED: {
             launch::SegArgs g = seg_args(*p, p->d_sec);
+            g.seq = p->seq.empty() ? nullptr : p->seq.data();
             g.nrows_add = p->nrows;
             g.mid = p->mid;
             g.part = p->d_part;

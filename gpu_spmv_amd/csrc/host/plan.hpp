@@ -71,6 +71,11 @@ struct axspmv_plan {
     // nrows slice partials
     uint32_t slices = 1;
     double *d_part = nullptr;
+    // ... run one after another: slice k is blocks seq[k] .. seq[k + 1]
+    std::vector<uint32_t> seq;
+    // AXT UNC th == 1 whose gathers outgrow the L2: the same matrix in such
+    // slices, for SpMV
+    axspmv_plan *by_slice = nullptr;
     // AXSPMV_PLAN_REORDER (kind REORDERED): the plan of B = Q A Q^T in
     // `inner`; the permutation into B's order (v~[k] = v[perm[k]]) and back
     // (v[i] = v~[iperm[i]]), each as two launch::permute_chunks passes

@@ -421,8 +421,9 @@ int axspmv_spmv(axspmv_plan *p, const double *d_x, double *d_y, void *stream);
 /* x_bar = A^T y_bar, run by the same kernel on a precomputed A^T in the same
  * format (plan created with AXSPMV_PLAN_TRANSPOSE).  CSR, K1, AXC, AXT COM
  * and AXT UNC plans without column slices reduce every row inside one wave
- * or a fixed fix-up order: no atomics, bit-identical results from call to
- * call.  RCT plans run the RCT plan of A^T, whose tiles add into LDS with
+ * (or, where x is large and its reads are scattered, one wave per part of x,
+ * the parts one after another) or a fixed fix-up order: no atomics,
+ * bit-identical results from call to call.  RCT plans run the RCT plan of A^T, whose tiles add into LDS with
  * atomics and, with several column slices, into x_bar with FP64 atomics, and
  * AXT plans in column slices add slice sums with FP64 atomics: the rounding
  * of x_bar then varies between calls (within the FP64 tolerance).  With

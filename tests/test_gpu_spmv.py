@@ -674,3 +674,67 @@ def test_rct_fused_clear_of_x_bar():
             assert rel_err(xb_ref, got[:nc] if shared else got[n:n + nc]) <= 1e-11
             if not shared:
                 assert np.array_equal(got[:n], b) and np.all(np.isnan(got[n + nc:]))
+
+
+@pytest.mark.parametrize("n,ncols,per,kw,launches", [
+    (701, 655360, 3000, {}, 2),                   # the fewest columns, long rows (over one pass of a wave)
+    (701, 655359, 3000, {}, 1),                   # one less
+    (300001, 700003, 5, dict(thw=1), 2),          # rows without entries, in one slice or in both
+    (400003, 700003, 5, dict(vtype=ax.F32), 2),
+    (250007, 1100001, 10, dict(thw=16), 4),
+    (150001, 3000001, 20, {}, 8),
+    (150001, 3000001, 10, {}, 4),                  # not two entries per row in 8 slices
+    (700003, 700003, 5, dict(flags=ax.PLAN_DETERMINISTIC), 2),
+    (700003, 700003, 5, dict(th=4, thw=64), 1),   # another layout
+    (700003, 700003, 5, dict(vtype=ax.F32, budget=256), 2),
+])
+def test_axt_one_slice_after_another(n, ncols, per, kw, launches):
+    """AXT UNC th == 1 on scattered columns of a large x: SpMV and adjoint in
+    column slices, SpMM and the value gradient on the planes in row order."""
+    m = _uneven(n, per, ncols, seed=per)
+    grads = kw.get("th", 1) == 1
+    p = ax.Plan(m, ax.FMT_AXT, **dict(kw, flags=kw.get("flags", 0) | (ax.PLAN_TRANSPOSE if grads else 0)))
+    assert p.info()["launches"] == launches
+    f32 = kw.get("vtype") == ax.F32
+    mv = ax.CsrMatrix(m.row, m.col, m.val.astype(np.float32).astype(np.float64), ncols=ncols) if f32 else m
+    x, w = ax.uniform(31, ncols), ax.uniform(32, n)
+    dx, dw = ax.DeviceBuffer.from_array(x), ax.DeviceBuffer.from_array(w)
+    ys = []
+    for _ in range(2):
+        dy = ax.DeviceBuffer.from_array(np.full(n + 1, np.nan))
+        p.spmv(dx, dy)
+        ys.append(dy.download(np.float64, n + 1))
+    assert np.array_equal(ys[0][:-1], ys[1][:-1]) and np.isnan(ys[0][-1])
+    assert rel_err(orc.ncsr(mv, x), ys[0][:-1]) <= TOL
+    if not grads:
+        return
+    dxb, dvb = ax.DeviceBuffer.from_array(np.full(ncols, np.nan)), ax.DeviceBuffer(8 * m.nnz)
+    p.adjoint(dw, dxb)
+    assert rel_err(orc.ncsr_t(mv, w, ncols), dxb.download(np.float64, ncols)) <= TOL
+    p.vbar(dw, dx, dvb)
+    assert np.array_equal(p.vbar_csr(dvb.download(np.float64, m.nnz)), orc.vbar(m, w, x))
+    k = 2
+    X = ax.uniform(33, ncols * k).reshape(ncols, k)
+    dX, dY = ax.DeviceBuffer.from_array(X), ax.DeviceBuffer(8 * n * k)
+    p.spmm(k, dX, dY)
+    assert rel_err(orc.spmm(mv, X), dY.download(np.float64, n * k).reshape(n, k)) <= TOL
+
+
+def test_axt_local_matrix_in_one_piece():
+    """A large x that rows read in bands, also with some entries far from
+    them, keeps the row order; a graph replays the slices."""
+    band = ax.banded(1 << 20, 3, 0.9, seed=3)
+    assert ax.Plan(band, ax.FMT_AXT).info()["launches"] == 1
+    far = np.random.default_rng(4).random(band.nnz)
+    for share, launches in ((0.2, 1), (0.9, 2)):
+        col = np.where(far < share, np.random.default_rng(5).integers(0, band.ncols, band.nnz), band.col).astype(np.uint32)
+        m = ax.CsrMatrix(band.row, col, band.val, ncols=band.ncols)
+        p = ax.Plan(m, ax.FMT_AXT)
+        assert p.info()["launches"] == launches
+        x = ax.uniform(34, m.ncols)
+        dx, dy = ax.DeviceBuffer.from_array(x), ax.DeviceBuffer(8 * m.nrows)
+        g = ax.Graph.of_plan(p, ax._lib.OP_SPMV, repeats=2, x=dx, y=dy)
+        for _ in range(3):
+            g.launch()
+            ax._lib.call("axspmv_device_sync")
+            assert rel_err(orc.ncsr(m, x), dy.download(np.float64, m.nrows)) <= TOL
