@@ -462,6 +462,8 @@ struct SpmmBatch {
                 ent.at(i + u * ROW, cc, rr);
                 c[u] = WIDE ? cc : cc * k * 8;
                 r[u] = rr * KT + (V == 2 ? (rr & 1) * GL : 0);
+            } else if constexpr (sizeof(VT) == 1) {
+                v[u] = 0;  // the table is read for every lane
             }
     }
 };
