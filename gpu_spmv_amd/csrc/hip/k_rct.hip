@@ -29,12 +29,6 @@
 #include "launch.hpp"
 #include "wave64.hpp"
 
-// Entries per lane per round (each of the two register sets holds this many,
-// as RCT_UNROLL / 2 pairs in the tile kernel).
-#ifndef RCT_UNROLL
-#define RCT_UNROLL 4
-#endif
-
 namespace {
 using axspmv::launch::RctArgs;
 
@@ -217,13 +211,27 @@ struct TileOf {
     }
 };
 
+// Pairs of a lane per round of the value-gradient sweep: 4 with column slices
+// (forward + adjoint, 2 / 3 / 4 pairs: 700,001-row power-law matrix 149.7 / 144.3 /
+// 142.2 us, FP32 values 139.0 / 134.7 / 132.3), else 3 (random, 300,007 rows 85.9 /
+// 82.1 / 79.9; permuted 60^3 stencil 73.6 / 70.8 / 68.6, but 80^3 renumbered 130.2 /
+// 128.9 / 131.6), and 2 for the 128-lane workgroups of small tiles, which hardly fill
+// one round (5,000-row power-law matrix 10.6 to 11.2 / 11.4 / 11.6).
+int vb_pairs(const RctArgs &a) { return a.S > 1 ? 4 : a.block <= 128 ? 2 : 3; }
+
 unsigned rct_grid(const RctArgs &a) { return tile_groups(a.nrb, a.S) + (a.nhb ? tile_groups(a.nhb, a.hs) : 0); }
 
 // VB: the same product on the plan of A^T, fused with the value gradient of
 // A: vb[e] = xr[row(e)] * x[col(e)] for every entry, in entry order (the
 // tile's xr values sit in LDS after its sums).  With x = r and xr = the
 // forward x, y = A^T r and vb holds r[i] * x[j] for every nonzero A(i, j).
-template <class VT, int KEY, bool VB, bool NT, bool HV = false>
+//
+// UP: pairs of a lane per round.  Two for the product alone (three and four:
+// 2^20-row power-law matrix 85.8 / 86.3 / 87.4 us, 48 banded matrices 90.0 /
+// 91.3 / 92.9).  The sweep with the value gradient has 8 bytes to store per
+// entry as well and a chain of one more load, so it takes more at a time:
+// see vb_pairs.
+template <class VT, int KEY, bool VB, bool NT, bool HV = false, int UP = 2>
 __global__ void __launch_bounds__(1024) rct_kernel(RctArgs a, const double *__restrict__ x, double *__restrict__ y,
                                                    const double *__restrict__ xr, double *__restrict__ vb,
                                                    const double *__restrict__ bvec, double *__restrict__ res) {
@@ -268,7 +276,6 @@ __global__ void __launch_bounds__(1024) rct_kernel(RctArgs a, const double *__re
     // two 8-byte stores; non-temporal, as nothing here reads vb again (the
     // permuted 128^3 stencil's forward + adjoint, renumbered: 485.8 ->
     // 478.8 us; the 2^20-row power-law matrix's: 233.0 -> 229.2 us).
-    constexpr int UP = (RCT_UNROLL + 1) / 2;
     struct PSet {
         uint32_t c[UP][2], r[UP][2];
         uint32_t at[UP][2];  // VB: the entries the two stores write
@@ -674,16 +681,25 @@ hipError_t rct(const RctArgs &a, const double *x, double *y, hipStream_t s, hipE
     // permuted 128^3 stencil's forward + adjoint, renumbered, 472.8 -> 467.7
     // us, one box
     // (24-bit keys are for streams that are loaded the ordinary way)
+#define AX_RCT_VB(VT, P, nt, UP)                                                                                  \
+    do {                                                                                                          \
+        if (nt && a.nt_stream)                                                                                    \
+            rct_kernel<VT, P, true, nt, false, UP><<<grid, a.block, lds, s>>>(a, x, y, xr, vbar, rb, res);        \
+        else                                                                                                      \
+            rct_kernel<VT, P, true, false, false, UP><<<grid, a.block, lds, s>>>(a, x, y, xr, vbar, rb, res);     \
+    } while (0)
 #define AX_RCT_LAUNCH(VT, P)                                                                              \
     do {                                                                                                  \
         constexpr bool nt = P != KEY_PACKED24;                                                            \
         if (P != KEY_DIAG && a.nhb)                                                                       \
             rct_kernel<VT, P == KEY_DIAG ? KEY_SPLIT : P, false, false, true><<<grid, a.block, lds, s>>>( \
                 a, x, y, xr, vbar, rb, res);                                                              \
-        else if (vb && nt && a.nt_stream)                                                                 \
-            rct_kernel<VT, P, true, nt><<<grid, a.block, lds, s>>>(a, x, y, xr, vbar, rb, res);           \
+        else if (vb && vb_pairs(a) == 2)                                                                  \
+            AX_RCT_VB(VT, P, nt, 2);                                                                      \
+        else if (vb && vb_pairs(a) == 3)                                                                  \
+            AX_RCT_VB(VT, P, nt, 3);                                                                      \
         else if (vb)                                                                                      \
-            rct_kernel<VT, P, true, false><<<grid, a.block, lds, s>>>(a, x, y, xr, vbar, rb, res);        \
+            AX_RCT_VB(VT, P, nt, 4);                                                                      \
         else if (nt && a.nt_stream)                                                                       \
             rct_kernel<VT, P, false, nt><<<grid, a.block, lds, s>>>(a, x, y, xr, vbar, rb, res);          \
         else                                                                                              \
@@ -707,6 +723,7 @@ hipError_t rct(const RctArgs &a, const double *x, double *y, hipStream_t s, hipE
     else
         with(double());
 #undef AX_RCT_LAUNCH
+#undef AX_RCT_VB
     hipError_t e = hipGetLastError();
     if (partials) {
         if (e == hipSuccess && mid) e = hipEventRecord(mid, s);

@@ -365,3 +365,31 @@ def test_axt_value_gradient_runs(thw, off):
 
     vbar(lambda d: p.vbar(dw, dx, d), lambda: w)
     vbar(lambda d: p.fwd_adj(dx, db, dy, dr, dxb, d), lambda: dr.download(np.float64, m.nrows))
+
+
+@pytest.mark.parametrize("off", [-1, 0, 1, 2])
+@pytest.mark.parametrize("block,slices", [(128, 1), (256, 1), (1024, 1), (128, 2), (512, 2)])
+def test_rct_sweep_rounds(block, slices, off):
+    """Tiles of the value-gradient sweep with entries around one, two and three
+    of its rounds (2, 3 or 4 pairs a lane), every other slice of another
+    length: v_bar bit for bit, x_bar against the oracle."""
+    pairs = 4 if slices > 1 else 2 if block <= 128 else 3
+    n, nc = 4000, 600
+    rng = np.random.default_rng(71)
+    for rounds in (1, 2, 3):
+        per = 2 * pairs * block * rounds + off
+        half = n // slices
+        flat = [np.sort(rng.choice(half * nc, per - k, replace=False)) + k * half * nc for k in range(slices)]
+        flat = np.concatenate(flat)
+        row = np.concatenate([[0], np.cumsum(np.bincount(flat // nc, minlength=n))]).astype(np.uint32)
+        m = ax.CsrMatrix(row, (flat % nc).astype(np.uint32), rng.standard_normal(flat.size), ncols=nc)
+        x, b = ax.uniform(72, nc), ax.uniform(73, n, stream=ax.VEC_STREAM + 1)
+        p = ax.Plan(m, ax.FMT_RCT, flags=ax.PLAN_TRANSPOSE, tile_rows=8192, slices=slices, block=block)
+        dx, db = ax.DeviceBuffer.from_array(x), ax.DeviceBuffer.from_array(b)
+        outs = [ax.DeviceBuffer.from_array(np.full(k, np.nan)) for k in (n, n, nc, m.nnz + 1)]
+        p.fwd_adj(dx, db, *outs)
+        r = outs[1].download(np.float64, n)
+        vbar = outs[3].download(np.float64, m.nnz + 1)
+        assert np.isnan(vbar[-1])
+        assert np.array_equal(p.vbar_csr(vbar[:-1]), orc.vbar(m, r, x))
+        assert rel_err(orc.ncsr_t(m, r, nc), outs[2].download(np.float64, nc)) <= TOL
