@@ -83,6 +83,7 @@ struct SpmmArgs {
     uint32_t nlong;
     uint32_t ncols;
     uint32_t xcd;  // 1: XCD i takes the i-th eighth of the rows
+    uint32_t far = 0;  // 1: short rows of scattered columns, one right-hand side per lane at k-tile 8
 };
 // kt (k-tile) in {8, 16, 32, 64}
 hipError_t spmm(const SpmmArgs &a, uint32_t k, uint32_t kt, const double *X, double *Y, hipStream_t s);

@@ -134,6 +134,8 @@ uint32_t spmm_by_eighths(const axspmv_csr *a) {
     return 8 * most <= uint64_t(a->nnz) + a->nnz / 8 ? 1 : 0;
 }
 
+bool narrow_bands(const axspmv_csr *a, uint32_t rows, uint64_t cols);
+
 // Row-contiguous layouts: record where each row starts (device array
 // `first`, uploaded here unless it is the CSR row pointer itself) for SpMM
 // and the value gradient.
@@ -156,7 +158,8 @@ int setup_rowwise(Plan &p, const axspmv_csr *a, const uint32_t *d_first, const v
     if (!lr) return AXSPMV_E_NOMEM;
     AX_TRY(p.upload(lr, longrows.data(), 4 * longrows.size(), s));
     p.spmm = launch::SpmmArgs{a->nrows, p.o.vtype, SPMM_LONG, p.d_first, p.d_rowptr, d_val, d_col, lr,
-                              uint32_t(longrows.size()), a->ncols, spmm_by_eighths(a)};
+                              uint32_t(longrows.size()), a->ncols, spmm_by_eighths(a),
+                              longrows.empty() && a->ncols > 65536 && !narrow_bands(a, 1024, 65536)};
     p.rowwise = true;
     return AXSPMV_OK;
 }
@@ -836,8 +839,9 @@ bool narrow_bands(const axspmv_csr *a, uint32_t rows, uint64_t cols) {
         if (b == e) continue;
         const auto mm = std::minmax_element(a->col + b, a->col + e);
         if (uint64_t(*mm.second) - *mm.first + 1 > cols) wide += e - b;
+        if (wide * 8 > a->nnz) return false;
     }
-    return wide * 8 <= a->nnz;
+    return true;
 }
 
 // The rows of an RCT plan for SpMM that get blocks of their own, in column

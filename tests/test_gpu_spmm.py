@@ -163,3 +163,18 @@ def test_heavy_rows_graph():
         g.launch()
         ax._lib.call("axspmv_device_sync")
         assert rel_err(ref, dY.download(np.float64, HEAVY.nrows * k).reshape(HEAVY.nrows, k)) <= TOL
+
+
+@pytest.mark.parametrize("vtype", [ax.F64, ax.F32])
+@pytest.mark.parametrize("fmt", [ax.FMT_AXT, ax.FMT_CSR, ax.FMT_AXC])
+def test_short_rows_of_scattered_columns(fmt, vtype):
+    """More than 65,536 columns read without locality by short rows only: one
+    right-hand side per lane at k-tile 8, whole and partial tiles."""
+    m = ax.random_sparse(66001, 0, 9, seed=14)
+    ref = m if vtype == ax.F64 else ax.CsrMatrix(m.row, m.col, m.val.astype(np.float32).astype(np.float64), ncols=m.ncols)
+    for k in (1, 7, 8, 16):
+        X = ax.uniform(15, m.ncols * k).reshape(m.ncols, k)
+        p = ax.Plan(m, fmt, vtype=vtype, ktile=8)
+        dX, dY = ax.DeviceBuffer.from_array(X), ax.DeviceBuffer.from_array(np.full(m.nrows * k, np.nan))
+        p.spmm(k, dX, dY)
+        assert rel_err(orc.spmm(ref, X), dY.download(np.float64, m.nrows * k).reshape(m.nrows, k)) <= 1e-12
