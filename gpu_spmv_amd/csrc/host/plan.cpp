@@ -677,7 +677,7 @@ int plan_axt(Plan &p, const axspmv_csr *a, hipStream_t s) {
     if (!p.d_fblocks) return AXSPMV_E_NOMEM;
     AX_TRY(p.upload(p.d_fblocks, fb.data(), sizeof(launch::Block) * fb.size(), s));
     AX_TRY(setup_rowwise(p, a, d_first, p.d_vplane, p.d_cplane, s));
-    if (!p.d_win) axt_add_slices(p, a, s);
+    if (!p.d_win && p.o.slices == 0) axt_add_slices(p, a, s);  // (1: one layout, as asked)
     return AXSPMV_OK;
 }
 

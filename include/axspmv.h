@@ -287,8 +287,16 @@ typedef struct axspmv_opts {
                            the matrix), each XCD gathering from one slice of
                            x; y is cleared, then the slices' row sums are
                            added with FP64 atomics (rounding order varies
-                           between runs).  SpMV and the adjoint only; 0 or 1
-                           = one layout; other AXT layouts reject S > 1. */
+                           between runs).  SpMV and the adjoint only.  1 =
+                           one layout, with the caller's thw.  0 = one
+                           layout, and where x is larger than 5 MB and the
+                           rows read it without locality (two entries per
+                           row and slice at least) the matrix once more in 2,
+                           4 or 8 column slices of 2 or 4 slots per tile, on
+                           which SpMV and the adjoint run one slice after
+                           another, without atomics: about twice the device
+                           memory, whatever thw is.  Other AXT layouts reject
+                           S > 1. */
 } axspmv_opts;
 
 #define AXSPMV_PLAN_TRANSPOSE 1u /* also build A^T (needed by the adjoint) */

@@ -738,3 +738,30 @@ def test_axt_local_matrix_in_one_piece():
             g.launch()
             ax._lib.call("axspmv_device_sync")
             assert rel_err(orc.ncsr(m, x), dy.download(np.float64, m.nrows)) <= TOL
+
+
+def _axt_slots(m, thw, slices=1):
+    """Value slots and tiles of AXT UNC th == 1 with thw slots per tile, in
+    column slices of ceil(ncols / slices) columns."""
+    C = -(-m.ncols // slices)
+    per = np.bincount(m.row_ids().astype(np.int64) * slices + m.col // C, minlength=m.nrows * slices)
+    tiles = int((-(-per // thw)).sum())
+    return tiles * thw, tiles, per.reshape(m.nrows, slices)
+
+
+@pytest.mark.parametrize("thw,vtype", [(1, ax.F64), (4, ax.F64), (4, ax.F32), (16, ax.F64)])
+def test_axt_slices_1_keeps_one_layout(thw, vtype):
+    """slices = 1 asks for one layout with the caller's thw, also where the
+    default takes column slices one after another."""
+    m = _uneven(400003, 5, 700003, seed=35)
+    assert ax.Plan(m, ax.FMT_AXT, thw=thw, vtype=vtype).info()["launches"] == 2
+    p = ax.Plan(m, ax.FMT_AXT, thw=thw, vtype=vtype, slices=1, flags=ax.PLAN_TRANSPOSE)
+    info = p.info()
+    assert info["launches"] == 1 and info["name"] == f"axt_unc_h1_thw{thw}"
+    assert info["slots"] == _axt_slots(m, thw)[0]
+    x, w = ax.uniform(36, m.ncols), ax.uniform(37, m.nrows)
+    mv = m if vtype == ax.F64 else ax.CsrMatrix(m.row, m.col, m.val.astype(np.float32).astype(np.float64), ncols=m.ncols)
+    assert rel_err(orc.ncsr(mv, x), ax.spmv_host(p, x)) <= TOL
+    dw, dxb = ax.DeviceBuffer.from_array(w), ax.DeviceBuffer(8 * m.ncols)
+    p.adjoint(dw, dxb)
+    assert rel_err(orc.ncsr_t(mv, w, m.ncols), dxb.download(np.float64, m.ncols)) <= TOL
