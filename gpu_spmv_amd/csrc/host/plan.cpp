@@ -499,9 +499,11 @@ int plan_axt_sliced(Plan &p, const axspmv_csr *a, bool one_by_one, hipStream_t s
     p.slices = S;
     p.stream_bytes = (vs + 4) * p.slots + 4 * nsec + 8ull * list.size();
     p.seg_nt = axt_stream_nt(a, p.stream_bytes);
+    if (one_by_one)  // the later slices read and write the rows of y they have entries in
+        for (size_t i = n; i < cnt.size(); ++i) p.stream_bytes += cnt[i] ? 16 : 0;
     p.launches = one_by_one ? S : 2;
     p.kind = Plan::AXT_UNC_H1_SLICED;
-    std::snprintf(p.name, sizeof p.name, "axt_unc_h1_thw%u_s%u%s", thw, S, det ? "_det" : "");
+    std::snprintf(p.name, sizeof p.name, "axt_unc_h1_thw%u_%s%u%s", thw, one_by_one ? "seq" : "s", S, det ? "_det" : "");
     return AXSPMV_OK;
 }
 
@@ -584,9 +586,12 @@ void axt_add_slices(Plan &p, const axspmv_csr *a, hipStream_t s) {
         return;
     }
     q->seg_nt = nt;
+    // the plan's info is of the layout that SpMV runs on
     p.device_bytes += q->device_bytes;
     p.stream_bytes = q->stream_bytes;
+    p.slots = q->slots;
     p.launches = S;
+    std::snprintf(p.name, sizeof p.name, "%s", q->name);
     p.by_slice = q.release();
 }
 
@@ -1512,7 +1517,7 @@ int plan_reordered(const axspmv_csr *a, const axspmv_opts *o, void *stream, axsp
     const bool direct = !p->to_b.L;
     p->stream_bytes = pi->stream_bytes + 2ull * (direct ? 20 : 40) * n;
     p->launches = pi->launches + (direct ? 2 : 4);
-    p->nblocks = pi->nblocks;
+    p->nblocks = pi->by_slice ? pi->by_slice->nblocks : pi->nblocks;
     p->staged_blocks = pi->staged_blocks;
     p->rowwise = pi->rowwise;
     *out = p.release();
@@ -1599,7 +1604,7 @@ extern "C" int axspmv_plan_get_info(const axspmv_plan *p, axspmv_plan_info *info
     info->alg_bytes = p->alg_bytes;
     info->beta = p->beta;
     info->launches = p->launches;
-    info->nblocks = p->nblocks;
+    info->nblocks = p->by_slice ? p->by_slice->nblocks : p->nblocks;
     info->staged_blocks = p->staged_blocks;
     return AXSPMV_OK;
 }

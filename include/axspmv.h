@@ -401,7 +401,10 @@ int axspmv_plan_create(const axspmv_csr *a, const axspmv_opts *o, void *stream,
 int axspmv_plan_destroy(axspmv_plan *p);
 
 typedef struct axspmv_plan_info {
-    char name[64];            /* kernel name, e.g. "axt_unc_h1_thw4"      */
+    char name[64];            /* kernel name, e.g. "axt_unc_h1_thw4"; the
+                                 default's column slices, one after another:
+                                 "axt_unc_h1_thw2_seq2" (slots, beta, bytes
+                                 and blocks are then the slices')           */
     uint32_t nrows, ncols, nnz, format;
     uint64_t slots;           /* value slots incl. padding                */
     uint64_t device_bytes;    /* bytes of matrix data held on the device  */

@@ -765,3 +765,24 @@ def test_axt_slices_1_keeps_one_layout(thw, vtype):
     dw, dxb = ax.DeviceBuffer.from_array(w), ax.DeviceBuffer(8 * m.ncols)
     p.adjoint(dw, dxb)
     assert rel_err(orc.ncsr_t(mv, w, m.ncols), dxb.download(np.float64, m.ncols)) <= TOL
+
+
+@pytest.mark.parametrize("n,per,ncols,kw,thw,slices", [
+    (400003, 5, 700003, {}, 2, 2),
+    (100001, 40, 1100001, {}, 4, 4),
+    (100001, 40, 1100001, dict(vtype=ax.F32), 4, 4),
+])
+def test_axt_one_slice_after_another_info(n, per, ncols, kw, thw, slices):
+    """The plan's info describes the layout that SpMV runs on: its name, slots
+    and padding, wave blocks, and the bytes of the later slices' reads and
+    writes of y."""
+    m = _uneven(n, per, ncols, seed=38)
+    i = ax.Plan(m, ax.FMT_AXT, **kw).info()
+    slots, tiles, per_slice = _axt_slots(m, thw, slices)
+    assert i["name"] == f"axt_unc_h1_thw{thw}_seq{slices}" and i["launches"] == slices
+    assert i["slots"] == slots and i["beta"] == m.nnz / slots
+    vs = 4 if kw.get("vtype") == ax.F32 else 8
+    later = int(np.count_nonzero(per_slice[:, 1:]))
+    assert i["stream_bytes"] == (vs + 4) * slots + 4 * tiles + 8 * i["nblocks"] + 16 * later + 8 * (n + ncols)
+    units = tiles * (thw // min(thw, 4))
+    assert units / 64 <= i["nblocks"] <= units
