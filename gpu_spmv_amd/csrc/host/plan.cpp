@@ -552,8 +552,11 @@ uint32_t axt_slices(const axspmv_csr *a) {
 }
 
 // The plan's SpMV in column slices (a copy of the matrix), where axt_slices
-// finds it worth while and a quarter of the free memory holds it.  The planes
-// in row order stay for the value gradient and SpMM.  Streams of more than 200
+// finds it worth while and a sixteenth of the card's memory holds it.  (Of all
+// its memory, not of what is free: the order of the additions then follows
+// from the matrix and the options.  Where the copy cannot be allocated all the
+// same the plan keeps row order, as a plan without the copy would have been
+// made.)  The planes in row order stay for the value gradient and SpMM.  Streams of more than 200
 // MB are loaded non-temporally (power-law, without / with, one matrix after
 // another and, in brackets, one again and again: 2^20 rows 177.9 / 163.1 us,
 // 900,000 151.2 / 136.8 (134.7 / 136.6), 750,000 124.8 / 112.0 (93.3 / 112.0)).
@@ -564,7 +567,7 @@ uint32_t axt_slices(const axspmv_csr *a) {
 void axt_add_slices(Plan &p, const axspmv_csr *a, hipStream_t s) {
     const uint32_t S = axt_slices(a);
     size_t avail = 0, total = 0;
-    if (S == 1 || hipMemGetInfo(&avail, &total) != hipSuccess || 4ull * 16 * (a->nnz + uint64_t(S) * a->nrows) > avail) return;
+    if (S == 1 || hipMemGetInfo(&avail, &total) != hipSuccess || 16ull * 16 * (a->nnz + uint64_t(S) * a->nrows) > total) return;
     auto q = std::make_unique<Plan>();
     q->o = p.o;
     const uint64_t vs = p.o.vtype == AXSPMV_F32 ? 4 : 8, cut = uint64_t(S) * a->nrows;  // rows of all slices

@@ -295,8 +295,10 @@ typedef struct axspmv_opts {
                            4 or 8 column slices of 2 or 4 slots per tile, on
                            which SpMV and the adjoint run one slice after
                            another, without atomics: about twice the device
-                           memory, whatever thw is.  Other AXT layouts reject
-                           S > 1. */
+                           memory, whatever thw is.  (One layout also where
+                           the copy would take more than a sixteenth of the
+                           card's memory or cannot be allocated; the plan's
+                           name tells.)  Other AXT layouts reject S > 1. */
 } axspmv_opts;
 
 #define AXSPMV_PLAN_TRANSPOSE 1u /* also build A^T (needed by the adjoint) */

@@ -786,3 +786,57 @@ def test_axt_one_slice_after_another_info(n, per, ncols, kw, thw, slices):
     assert i["stream_bytes"] == (vs + 4) * slots + 4 * tiles + 8 * i["nblocks"] + 16 * later + 8 * (n + ncols)
     units = tiles * (thw // min(thw, 4))
     assert units / 64 <= i["nblocks"] <= units
+
+
+def _free_bytes():
+    import ctypes
+    hip = ctypes.CDLL("libamdhip64.so")
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+class _Filled:
+    """Device memory taken up to about `left` bytes."""
+
+    def __init__(self, left):
+        self.left, self.bufs = left, []
+
+    def __enter__(self):
+        for piece in (16 << 30, 1 << 30, 64 << 20, 2 << 20):
+            while _free_bytes() >= self.left + piece:
+                self.bufs.append(ax.DeviceBuffer(piece))
+        return self
+
+    def __exit__(self, *a):
+        for b in self.bufs:
+            b.free()
+
+
+def test_axt_layout_does_not_depend_on_free_memory():
+    """The same matrix and options give the same layout, to the bit of its
+    products, on an almost full card; only where the slices cannot be
+    allocated at all does the plan keep row order, and its info says so."""
+    m = _uneven(400003, 5, 700003, seed=39)
+    x = ax.uniform(40, m.ncols)
+    dx, dy = ax.DeviceBuffer.from_array(x), ax.DeviceBuffer(8 * m.nrows)
+
+    def product():
+        p = ax.Plan(m, ax.FMT_AXT)
+        p.spmv(dx, dy)
+        return p.info(), dy.download(np.float64, m.nrows)
+
+    one = ax.Plan(m, ax.FMT_AXT, slices=1)
+    one.spmv(dx, dy)  # both kinds of plan have run: their code is on the device
+    row_order, info1 = dy.download(np.float64, m.nrows), one.info()
+    info, y = product()
+    del one
+    assert info["launches"] == 2
+    with _Filled(info["device_bytes"] + (64 << 20)):
+        info2, y2 = product()
+    assert info2 == info and np.array_equal(y, y2)
+    between = (info1["device_bytes"] + info["device_bytes"]) // 2
+    with _Filled(between):
+        info3, y3 = product()
+    assert info3 == info1 and np.array_equal(row_order, y3)
+    assert rel_err(orc.ncsr(m, x), y3) <= TOL
