@@ -8,6 +8,7 @@
 #include <cmath>
 #include <memory>
 #include <numeric>
+#include <string>
 
 #include "../hip/launch.hpp"
 #include "common.hpp"
@@ -564,10 +565,13 @@ uint32_t axt_slices(const axspmv_csr *a) {
 // streams (2^20 rows, 2 / 4 slots 163.0 / 168.6 us); else four, with half the
 // load instructions (FP64, 750,000 rows 124.8 / 120.7; FP32, 2^20 rows 167.7 /
 // 158.1; random rows of 6 61.7 / 65.2).
-void axt_add_slices(Plan &p, const axspmv_csr *a, hipStream_t s) {
+int axt_add_slices(Plan &p, const axspmv_csr *a, hipStream_t s) {
     const uint32_t S = axt_slices(a);
+    if (S == 1) return AXSPMV_OK;
     size_t avail = 0, total = 0;
-    if (S == 1 || hipMemGetInfo(&avail, &total) != hipSuccess || 16ull * 16 * (a->nnz + uint64_t(S) * a->nrows) > total) return;
+    const hipError_t e = hipMemGetInfo(&avail, &total);
+    if (e != hipSuccess) return hip_fail(e, "plan_create: hipMemGetInfo");
+    if (16ull * 16 * (a->nnz + uint64_t(S) * a->nrows) > total) return AXSPMV_OK;
     auto q = std::make_unique<Plan>();
     q->o = p.o;
     const uint64_t vs = p.o.vtype == AXSPMV_F32 ? 4 : 8, cut = uint64_t(S) * a->nrows;  // rows of all slices
@@ -579,15 +583,18 @@ void axt_add_slices(Plan &p, const axspmv_csr *a, hipStream_t s) {
     q->nrows = p.nrows;
     q->ncols = p.ncols;
     q->nnz = p.nnz;
+    const std::string last = axspmv_last_error();
     int rc = AXSPMV_E_NOMEM;
     try {
         rc = plan_axt_sliced(*q, a, true, s);
     } catch (const std::bad_alloc &) {
     }
-    if (rc) {  // no memory after all: row order
+    if (rc == AXSPMV_E_NOMEM || rc == AXSPMV_E_OVERFLOW) {  // no room for the copy: row order, and no error
         (void)hipGetLastError();
-        return;
+        fail(AXSPMV_OK, "%s", last.c_str());
+        return AXSPMV_OK;
     }
+    if (rc) return rc;
     q->seg_nt = nt;
     // the plan's info is of the layout that SpMV runs on
     p.device_bytes += q->device_bytes;
@@ -596,6 +603,7 @@ void axt_add_slices(Plan &p, const axspmv_csr *a, hipStream_t s) {
     p.launches = S;
     std::snprintf(p.name, sizeof p.name, "%s", q->name);
     p.by_slice = q.release();
+    return AXSPMV_OK;
 }
 
 int plan_axt(Plan &p, const axspmv_csr *a, hipStream_t s) {
@@ -685,7 +693,7 @@ int plan_axt(Plan &p, const axspmv_csr *a, hipStream_t s) {
     if (!p.d_fblocks) return AXSPMV_E_NOMEM;
     AX_TRY(p.upload(p.d_fblocks, fb.data(), sizeof(launch::Block) * fb.size(), s));
     AX_TRY(setup_rowwise(p, a, d_first, p.d_vplane, p.d_cplane, s));
-    if (!p.d_win && p.o.slices == 0) axt_add_slices(p, a, s);  // (1: one layout, as asked)
+    if (!p.d_win && p.o.slices == 0) AX_TRY(axt_add_slices(p, a, s));  // (1: one layout, as asked)
     return AXSPMV_OK;
 }
 

@@ -840,3 +840,23 @@ def test_axt_layout_does_not_depend_on_free_memory():
         info3, y3 = product()
     assert info3 == info1 and np.array_equal(row_order, y3)
     assert rel_err(orc.ncsr(m, x), y3) <= TOL
+
+
+def test_axt_row_order_for_want_of_memory_is_no_error():
+    """The plan that keeps row order because the slices cannot be allocated is
+    a success: the thread's last error stays what it was, and the runtime's
+    error does not come back from the next launch."""
+    m = _uneven(400003, 5, 700003, seed=41)
+    x = ax.uniform(42, m.ncols)
+    dx, dy = ax.DeviceBuffer.from_array(x), ax.DeviceBuffer(8 * m.nrows)
+    one, both = (ax.Plan(m, ax.FMT_AXT, **kw).info()["device_bytes"] for kw in (dict(slices=1), {}))
+    with pytest.raises(ax.AxspmvError):
+        ax.Plan(m, ax.FMT_AXT, thw=3)
+    last = ax._lib.load().axspmv_last_error()
+    with _Filled((one + both) // 2):
+        p = ax.Plan(m, ax.FMT_AXT)
+        assert p.info()["launches"] == 1
+        assert ax._lib.load().axspmv_last_error() == last
+        p.spmv(dx, dy)
+        ax._lib.call("axspmv_device_sync")
+    assert rel_err(orc.ncsr(m, x), dy.download(np.float64, m.nrows)) <= TOL
