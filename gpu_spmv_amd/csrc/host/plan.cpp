@@ -1028,10 +1028,23 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
     uint32_t R = 1;  // rows of the largest block: the LDS accumulator size
     for (uint32_t k = 0; k < nrb; ++k) R = std::max(R, rbs[k + 1] - rbs[k]);
     const uint32_t C = uint32_t(std::max<uint64_t>(1, ceil_div(a->ncols, S)));
-    // Heavy rows (plans that SpMM can use): blocks of their own, in column
-    // slices, their tiles after the others.
+    // Heavy rows: blocks of their own, in column slices, their tiles after the
+    // others.  Only in plans meant for SpMM (ktile or tile_rows given, tiles
+    // short enough): SpMV and forward + adjoint of a default plan pay the clear
+    // of the heavy rows, their adds and a residual pass of its own, and get
+    // little for it (power-law, without / with, SpMV: 70,000 rows 11.1 / 13.1
+    // us, 100,000 13.6 / 15.1, 200,000 21.5 / 22.5, 300,000 32.7 / 37.8; forward
+    // + adjoint 23.0 / 26.6, 32.3 / 34.0, 59.6 / 58.4, 75.9 / 81.0; from 215,000
+    // to 262,000 rows SpMV gains 6 to 12 % on changing matrices and loses 1 to 9
+    // on one).  Not beside column slices that the plan chose itself, which do
+    // the same for all rows (SpMM, k = 8, two slices: 270,000 rows 74.7 / 79.8
+    // us, 350,000 97.9 / 107.2, 500,000 142.1 / 148.8; k = 4 60.7 / 69.8, 79.7 /
+    // 91.4, 110.1 / 123.2).  Not in deterministic plans, which add no slice
+    // atomically.
     std::vector<uint32_t> hrows, hbs(1, 0), hmask;
-    if (!p.keep_pos && 64ull * R <= lds_max) hrows = heavy_rows(a);
+    if ((p.o.ktile || p.o.tile_rows) && (S == 1 || p.o.slices) && !(p.o.flags & AXSPMV_PLAN_DETERMINISTIC) && !p.keep_pos &&
+        64ull * R <= lds_max)
+        hrows = heavy_rows(a);
     // One slice per XCD, and blocks of few enough rows that their tiles reach
     // every CU: 100,000-row power-law matrix, k = 8, blocks as tall as the LDS
     // allows (64 tiles) 38 us, 256 tiles 26, 512 tiles 29.  4 slices lose where

@@ -324,8 +324,9 @@ typedef struct axspmv_opts {
                                     such an AXT plan (two slots per tile,
                                     slices of <= 2 MB of y_bar) and
                                     axspmv_adjoint runs on it.  The RCT
-                                    forward SpMV already adds its slices in
-                                    slice order (partials and a merge), but
+                                    forward SpMV keeps no heavy rows apart
+                                    (see axspmv_spmm) and adds its slices in
+                                    slice order where it stores partials, but
                                     its tiles sum their rows in LDS in no
                                     fixed order; its fused forward + adjoint
                                     keeps those LDS adds and FP64 slice adds
@@ -338,7 +339,9 @@ typedef struct axspmv_opts {
                                     nnz / 6) stores them in slice partials
                                     (slices x nrows doubles held by the
                                     plan) and a second kernel adds those in
-                                    slice order; other plans add. */
+                                    slice order; other plans, and those
+                                    that keep heavy rows apart (see
+                                    axspmv_spmm), add. */
 #define AXSPMV_PLAN_REORDER 64u /* square matrices: build the plan for
                                     B = Q A Q^T, Q the reverse Cuthill-McKee
                                     order of axspmv_csr_rcm, and run every
@@ -476,11 +479,13 @@ int axspmv_fwd_adj(axspmv_plan *p, const double *d_x, const double *d_b, double 
  * ktile sums in LDS, so tile_rows * ktile * 8 bytes must fit one workgroup's
  * LDS -- tile_rows <= 2560 at ktile 8 on 160 KB; the default ktile is cut
  * to fit; with several column slices Y is cleared, then atomically added
- * to; rows of 32 entries and more, where they are few but hold a good part
- * of a matrix of over 65,536 columns, get tiles of their own in plans whose
- * tile_rows SpMM can use, and their sums are added to Y atomically;
- * 1024-lane workgroups unless the plan sets block).  No reference
- * counterpart. */
+ * to; 1024-lane workgroups unless the plan sets block).  Heavy rows: a plan
+ * made with ktile or tile_rows set, tiles short enough for ktile 8, one
+ * column slice or as many as the caller asked for and no
+ * AXSPMV_PLAN_DETERMINISTIC gives the rows of 32 entries and more, where they
+ * are few but hold a good part of a matrix of over 65,536 columns, tiles of
+ * their own; their sums are added atomically, to Y and, by the plan's SpMV
+ * and forward + adjoint, to y.  No reference counterpart. */
 int axspmv_spmm(axspmv_plan *p, uint32_t k, const double *d_X, double *d_Y, void *stream);
 
 /* ---------------------------------------------------------- timing */
@@ -499,7 +504,7 @@ typedef struct axspmv_timing {
 #define AXSPMV_TIME_KERNEL 3u /* as REGION (SpMV only, iters <= 4096), with an
                                  event before every SpMV and one between its
                                  launches: main_ms is the mean time of its
-                                 main kernel.  Only RCT and AXT plans with
+                                 main kernel.  RCT and AXT plans with
                                  column slices launch a second kernel: the
                                  merge of slice partials after the main one
                                  or the clear of y before it; other paths

@@ -178,3 +178,40 @@ def test_short_rows_of_scattered_columns(fmt, vtype):
         dX, dY = ax.DeviceBuffer.from_array(X), ax.DeviceBuffer.from_array(np.full(m.nrows * k, np.nan))
         p.spmm(k, dX, dY)
         assert rel_err(orc.spmm(ref, X), dY.download(np.float64, m.nrows * k).reshape(m.nrows, k)) <= 1e-12
+
+
+# Heavy rows are for plans meant for SpMM.
+GRAPH = ax.powerlaw(100001, 2.0, 2048, 20.0, seed=31)
+
+
+@pytest.mark.parametrize("kw,heavy", [
+    (dict(), False), (dict(flags=ax.PLAN_TRANSPOSE), False), (dict(slices=4), False),
+    (dict(ktile=8), True), (dict(ktile=8, vtype=ax.F32), True), (dict(tile_rows=448), True),
+    (dict(ktile=8, flags=ax.PLAN_DETERMINISTIC), False), (dict(tile_rows=448, slices=4, flags=ax.PLAN_DETERMINISTIC), False)])
+def test_heavy_rows_by_intent(kw, heavy):
+    """Neither the default plan nor a deterministic one keeps heavy rows apart:
+    one launch per SpMV, with column slices partials and their merge."""
+    p = ax.Plan(GRAPH, ax.FMT_RCT, **kw)
+    info = p.info()
+    S = kw.get("slices", 1)
+    assert (info["nblocks"] > 1.05 * GRAPH.nrows / int(info["name"].split("_")[1][1:]) * S + S) == heavy, info
+    assert info["launches"] == (2 if heavy or S > 1 else 1)
+    assert heavy or not info["name"].endswith("_atomic")
+    mv = f32_values(GRAPH, kw)
+    x = ax.uniform(32, GRAPH.ncols)
+    assert rel_err(orc.ncsr(mv, x), ax.spmv_host(p, x)) <= TOL
+    X = ax.uniform(33, GRAPH.ncols * 5).reshape(GRAPH.ncols, 5)
+    assert rel_err(orc.spmm(mv, X), spmm(p, GRAPH, X)) <= TOL
+
+
+def test_heavy_rows_not_beside_automatic_slices():
+    """Column slices that the plan chooses itself replace heavy rows; slices
+    that the caller asks for do not."""
+    m = ax.powerlaw(270001, 2.0, 2048, 20.0, seed=34)
+    X = ax.uniform(35, m.ncols * 3).reshape(m.ncols, 3)
+    for kw, heavy in ((dict(ktile=8), False), (dict(ktile=8, tile_rows=2112), False), (dict(ktile=8, slices=2), True)):
+        p = ax.Plan(m, ax.FMT_RCT, **kw)
+        info = p.info()
+        assert info["name"].startswith("rct_r2112_s2"), info
+        assert (info["nblocks"] > 1.05 * m.nrows / 2112 * 2 + 2) == heavy, (kw, info)
+        assert rel_err(orc.spmm(m, X), spmm(p, m, X)) <= TOL
