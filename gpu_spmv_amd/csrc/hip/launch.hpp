@@ -103,7 +103,7 @@ struct RctArgs {
     uint32_t nrows, R, S, nrb, vtype, block, rbits, ncols;
     double *part;  // S > 1: S slice partials, pstride doubles apart (nullptr: atomic adds into y)
     size_t pstride;
-    uint32_t nt_stream = 0;  // 1: the tile kernel (SpMV, value-gradient sweep) streams with non-temporal loads
+    uint32_t nt_stream = 0;  // 1: the tile kernel (SpMV, value-gradient sweep) streams with non-temporal loads (nhb == 0)
     // narrow bands: a 16-bit key per entry (key16 != nullptr; key, col and
     // lrow unused) with the column as an offset of cbits16 bits from sbase
     // (runs of 128 entries) and row - column - dmin above it (dmin modulo

@@ -1327,9 +1327,10 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
     // 512-row tiles 92.6 -> 90.5, 1.5M banded rows, 5888-row tiles 102 -> 97).
     // A smaller stream stays cached between SpMVs, and non-temporal loads
     // give that up (the 2^20-row power-law matrix, 252 MB, back to back: 58 ->
-    // 89 us).
+    // 89 us).  Plans with heavy rows, which are for SpMM, have no such kernel:
+    // their SpMV loads the ordinary way.
     p.rct.pal = dpal;
-    p.rct.nt_stream = (vbytes + kbytes) * nnz > (256ull << 20) ? 1 : 0;
+    p.rct.nt_stream = !nhb && (vbytes + kbytes) * nnz > (256ull << 20) ? 1 : 0;
     p.rct.key16 = dk16;
     p.rct.key24 = dk24;
     p.rct.key8 = dk8;
