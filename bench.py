@@ -51,17 +51,20 @@ from gpu_spmv_amd.core import TIME_COLD, TIME_GRAPH, TIME_KERNEL, TIME_REGION  #
 
 PEAK_HBM_GBS = 8000.0
 FLAGSHIP = ("rct_auto", ax.FMT_RCT, dict())
-FLAGSHIP_AXT = ("axt_unc_h1_thw4", ax.FMT_AXT, dict(thw=4, th=1))
+# the reference's AXT UNC th = 1 layout in one piece (slices = 1; by itself, 0,
+# a plan of a large scattered matrix takes column slices: axt_unc_h1_auto)
+FLAGSHIP_AXT = ("axt_unc_h1_thw4", ax.FMT_AXT, dict(thw=4, th=1, slices=1))
 # the reference's AXT UNC th = 1 layout, one per column slice of 2 MB of x
 FLAGSHIP_AXT_SLICED = ("axt_unc_h1_thw2_s4", ax.FMT_AXT, dict(thw=2, slices=4))
 OTHERS = [
     FLAGSHIP_AXT,
     FLAGSHIP_AXT_SLICED,
+    ("axt_unc_h1_auto", ax.FMT_AXT, dict()),
     ("axt_unc_h1_thw2_s4_det", ax.FMT_AXT, dict(thw=2, slices=4, flags=ax.PLAN_DETERMINISTIC)),
     ("csr_naive", ax.FMT_CSR, dict(kernel=ax.KER_NAIVE)),
     ("csr_vector", ax.FMT_CSR, dict(kernel=ax.KER_STREAM)),
-    ("axt_unc_h1_thw8", ax.FMT_AXT, dict(thw=8, th=1)),
-    ("axt_unc_h1_thw16", ax.FMT_AXT, dict(thw=16, th=1)),
+    ("axt_unc_h1_thw8", ax.FMT_AXT, dict(thw=8, th=1, slices=1)),
+    ("axt_unc_h1_thw16", ax.FMT_AXT, dict(thw=16, th=1, slices=1)),
     ("axt_unc_h4_thw64", ax.FMT_AXT, dict(thw=64, th=4)),
     ("axt_unc_h8_thw64", ax.FMT_AXT, dict(thw=64, th=8)),
     ("axt_com_h1_thw64_bs256", ax.FMT_AXT, dict(mode=ax.AXT_COM, thw=64, th=1, bs=256)),
@@ -76,7 +79,7 @@ OTHERS = [
     ("rct_r16384_s2", ax.FMT_RCT, dict(tile_rows=16384, slices=2)),
     ("axt_unc_h1_thw4_ax", ax.FMT_AXT, dict(thw=4, flags=ax.PLAN_AX_LAYOUT)),
     ("rct_auto_f32val", ax.FMT_RCT, dict(vtype=ax.F32)),
-    ("axt_unc_h1_thw4_f32val", ax.FMT_AXT, dict(thw=4, vtype=ax.F32)),
+    ("axt_unc_h1_thw4_f32val", ax.FMT_AXT, dict(thw=4, slices=1, vtype=ax.F32)),
 ]
 # C3's rows with AXSPMV_PLAN_REORDER (the plan of B = Q A Q^T, Q the reverse
 # Cuthill-McKee order; x and y permuted inside the timed SpMV)

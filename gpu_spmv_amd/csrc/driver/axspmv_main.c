@@ -302,6 +302,7 @@ int main(int argc, char **argv) {
         o.mode = k->mode;
         if (k->thw) o.thw = k->thw;
         if (k->th) o.th = k->th;
+        if (k->format == AXSPMV_FMT_AXT) o.slices = 1; /* the kernel named, in one layout */
         if (k->bs) o.bs = cbs;
         if (k->format == AXSPMV_FMT_AXC || k->format == AXSPMV_FMT_CSR) o.hbs = k->hbs;
         if (k->chunk) o.chunk = k->chunk;

@@ -355,8 +355,12 @@ std::vector<axspmv_opts> default_candidates(uint32_t op, bool for_batch = false)
         for (uint32_t thw : {2u, 4u, 8u, 16u}) {
             o.th = 1;
             o.thw = thw;
+            // single plans: thw 4, the default, as the library lays it out (in
+            // column slices where those are faster), the others in one layout
+            o.slices = for_batch || thw == 4 ? 0 : 1;
             c.push_back(o);
         }
+        o.slices = 0;
         for (uint32_t th : {2u, 4u, 8u}) {
             o.th = th;
             o.thw = 64;

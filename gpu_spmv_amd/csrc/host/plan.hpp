@@ -78,8 +78,9 @@ struct axspmv_plan {
     axspmv_plan *by_slice = nullptr;
     // AXSPMV_PLAN_REORDER (kind REORDERED): the plan of B = Q A Q^T in
     // `inner`; the permutation into B's order (v~[k] = v[perm[k]]) and back
-    // (v[i] = v~[iperm[i]]), each as two launch::permute_chunks passes
-    // through a staging vector (pass 1: w1, b1; pass 2: b2; chunks of L);
+    // (v[i] = v~[iperm[i]]), each as one gather by idx (L == 0: up to 2^20
+    // entries) or as two launch::permute_chunks passes through a staging
+    // vector (pass 1: w1, b1; pass 2: b2; chunks of L);
     // nscratch vectors of nrows doubles (3, or 6 with a transposed plan; the
     // last one stages); bpos[e] = position in A of entry e of B's CSR
     axspmv_plan *inner = nullptr;

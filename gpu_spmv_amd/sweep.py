@@ -44,9 +44,10 @@ CANDIDATES = [
     ("k1_c64", L.FMT_K1, dict(chunk=64), False),
     ("axc_hbs4", L.FMT_AXC, dict(hbs=4), False),
     ("axc_hbs32", L.FMT_AXC, dict(hbs=32), False),
-    ("axt_unc_h1_thw4", L.FMT_AXT, dict(thw=4, th=1), False),
-    ("axt_unc_h1_thw8", L.FMT_AXT, dict(thw=8, th=1), False),
-    ("axt_unc_h1_thw16", L.FMT_AXT, dict(thw=16, th=1), False),
+    ("axt_unc_h1_auto", L.FMT_AXT, dict(), False),  # in column slices where x is large and scattered
+    ("axt_unc_h1_thw4", L.FMT_AXT, dict(thw=4, th=1, slices=1), False),
+    ("axt_unc_h1_thw8", L.FMT_AXT, dict(thw=8, th=1, slices=1), False),
+    ("axt_unc_h1_thw16", L.FMT_AXT, dict(thw=16, th=1, slices=1), False),
     ("axt_unc_h4_thw64", L.FMT_AXT, dict(thw=64, th=4), False),
     ("axt_unc_h8_thw64", L.FMT_AXT, dict(thw=64, th=8), False),
     ("axt_unc_h1_thw2_s4", L.FMT_AXT, dict(thw=2, slices=4), False),

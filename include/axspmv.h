@@ -654,7 +654,8 @@ int axspmv_graph_destroy(axspmv_graph *g);
  * the built-in set of axspmv_autotune_defaults; ncand then gives the room in
  * times_ms (which must hold the whole set).  No reference counterpart: the
  * reference sweeps block sizes by relaunching (jobLauncher.sh:145-176). */
-/* The built-in candidates: for SpMV AXT UNC th = 1 with thw 2..16 and th =
+/* The built-in candidates: for SpMV AXT UNC th = 1 with thw 2..16 (4 with
+ * slices = 0, the others with 1) and th =
  * 2..8 with thw 64 at two block budgets, AXT UNC th = 1 (thw 2) in 2, 4 and
  * 8 column slices, K1 (chunk 64), RCT (default, 256 and 1024 threads), and
  * RCT and AXT UNC th = 1 (thw 4) with AXSPMV_PLAN_REORDER (rejected, time
