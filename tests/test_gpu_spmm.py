@@ -215,3 +215,87 @@ def test_heavy_rows_not_beside_automatic_slices():
         assert info["name"].startswith("rct_r2112_s2"), info
         assert (info["nblocks"] > 1.05 * m.nrows / 2112 * 2 + 2) == heavy, (kw, info)
         assert rel_err(orc.spmm(m, X), spmm(p, m, X)) <= TOL
+
+
+@pytest.mark.parametrize("n,signs,kw,saved_bits", [
+    (300001, False, dict(tile_rows=1024), 8),                    # 72 MB: 24-bit keys
+    (450001, False, dict(tile_rows=1024, vtype=ax.F32), 8),
+    (100001, True, dict(tile_rows=448), 0),                      # values from a table, 32-bit keys
+    (200001, True, dict(tile_rows=1024), 8),                     # both (73 MB in 32-bit keys)
+    (100001, True, dict(tile_rows=448, flags=ax.PLAN_RCT_SPLIT), 0),
+], ids=["k24", "k24_f32", "table", "k24_table", "split_table"])
+def test_heavy_rows_with_short_keys_and_tables(n, signs, kw, saved_bits):
+    """Heavy rows, whose tiles lie after the ordinary ones, with every way of
+    storing a key and a value: SpMM, SpMV, forward + adjoint."""
+    if n == 200001:  # 25 entries a row, 600 in one of 12
+        rng = np.random.default_rng(n)
+        lens = np.where(np.arange(n) % 12 == 5, 600, 25)
+        row = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+        m = ax.CsrMatrix(row, rng.integers(0, n, int(row[-1])).astype(np.uint32), rng.standard_normal(int(row[-1])), ncols=n)
+    else:
+        m = ax.powerlaw(n, 2.0, 2048, 20.0, seed=n)
+    plain = ax.Plan(m, ax.FMT_RCT, **kw).info()
+    if signs:
+        m = ax.CsrMatrix(m.row, m.col, np.where(m.val < 0, -1.0, 1.0), ncols=m.ncols)
+    flags = kw.get("flags", 0)
+    p = ax.Plan(m, ax.FMT_RCT, **dict(kw, flags=flags | ax.PLAN_TRANSPOSE))
+    info = p.info()
+    wide = ax.Plan(m, ax.FMT_RCT, **dict(kw, flags=flags | ax.PLAN_RCT_WIDE_KEY)).info()
+    assert info["nblocks"] > 1.05 * n / kw["tile_rows"] + 1
+    assert abs(8 * (wide["stream_bytes"] - info["stream_bytes"]) / m.nnz - saved_bits) < 0.3
+    if signs:  # 8 bytes a value before, 1 now
+        assert info["stream_bytes"] < plain["stream_bytes"] - 6.5 * m.nnz
+    mv = f32_values(m, kw)
+    for k in (2, 5):
+        X = ax.uniform(130 + k, n * k).reshape(n, k)
+        assert rel_err(orc.spmm(mv, X), spmm(p, m, X)) <= TOL
+    x, b = ax.uniform(136, n), ax.uniform(137, n)
+    dx, db = ax.DeviceBuffer.from_array(x), ax.DeviceBuffer.from_array(b)
+    dy, dr, dxb = (ax.DeviceBuffer.from_array(np.full(n, np.nan)) for _ in range(3))
+    dv = ax.DeviceBuffer(8 * m.nnz)
+    p.fwd_adj(dx, db, dy, dr, dxb, dv)
+    y, r = dy.download(np.float64, n), dr.download(np.float64, n)
+    assert rel_err(orc.ncsr(mv, x), y) <= TOL and np.array_equal(r, y - b)
+    assert rel_err(orc.ncsr_t(mv, r, n), dxb.download(np.float64, n)) <= TOL
+    assert np.array_equal(p.vbar_csr(dv.download(np.float64, m.nnz)), r[m.row_ids()] * x[m.col])
+
+
+BIG, MID = (ax.powerlaw(n, 2.0, 2048, 20.0, seed=38) for n in (660001, 300001))
+NONFINITE = [("axt", EDGE, ax.FMT_AXT, {}), ("csr", EDGE, ax.FMT_CSR, {}), ("axc", EDGE, ax.FMT_AXC, dict(hbs=2)),
+             ("rct", EDGE, ax.FMT_RCT, dict(tile_rows=256)), ("rct_s4", EDGE, ax.FMT_RCT, dict(tile_rows=200, slices=4)),
+             ("k16", BAND, ax.FMT_RCT, dict(tile_rows=128)), ("heavy", HEAVY, ax.FMT_RCT, dict(tile_rows=1024)),
+             ("axt_seq", BIG, ax.FMT_AXT, {}), ("k24", BIG, ax.FMT_RCT, {}), ("k24_heavy", MID, ax.FMT_RCT, dict(tile_rows=1024))]
+
+
+@pytest.mark.parametrize("m,fmt,kw", [c[1:] for c in NONFINITE], ids=[c[0] for c in NONFINITE])
+def test_nonfinite_x_stays_in_its_rows_and_columns(m, fmt, kw):
+    """X[0] = inf and X[1] = nan in one right-hand side: only the rows holding
+    these columns become non-finite, and there only that right-hand side --
+    not through lanes past a row's or tile's end or past the last right-hand
+    side."""
+    p = ax.Plan(m, fmt, **kw)
+    if m is BIG or m is MID:  # the path is the one meant
+        info = p.info()
+        if fmt == ax.FMT_AXT:
+            assert "_seq" in info["name"]
+        else:
+            wide = ax.Plan(m, fmt, **dict(kw, flags=ax.PLAN_RCT_WIDE_KEY)).info()
+            assert info["stream_bytes"] < wide["stream_bytes"] - 0.9 * m.nnz
+            assert (info["nblocks"] > 1.05 * m.nrows / 1024 + 1) == bool(kw)
+
+    def check(ref, got):
+        fin = np.isfinite(ref)
+        assert fin.any() and not fin.all()
+        np.testing.assert_array_equal(got[~fin], ref[~fin])
+        assert rel_err(ref[fin], got[fin]) <= TOL
+
+    x = ax.uniform(140, m.ncols)
+    used = np.unique(m.col)[[0, -1]]
+    x[used] = np.inf, np.nan
+    check(orc.ncsr(m, x), ax.spmv_host(p, x))
+    if kw.get("tile_rows", 0) == 0 and fmt == ax.FMT_RCT:
+        return  # tiles too tall for SpMM
+    for k, j in ((3, 0), (8, 7), (6, 3)):
+        X = ax.uniform(141 + k, m.ncols * k).reshape(m.ncols, k)
+        X[used, j] = np.inf, np.nan
+        check(orc.spmm(m, X), spmm(p, m, X))
