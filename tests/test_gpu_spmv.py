@@ -790,9 +790,9 @@ def test_axt_one_slice_after_another_info(n, per, ncols, kw, thw, slices):
 
 def _free_bytes():
     import ctypes
-    hip = ctypes.CDLL("libamdhip64.so")
     free, total = ctypes.c_size_t(), ctypes.c_size_t()
-    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    # of the runtime that the library is linked to (torch brings another)
+    assert ax._lib.load().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
     return free.value
 
 
