@@ -32,10 +32,9 @@
 namespace {
 using axspmv::launch::RctArgs;
 
-// Entry e of a tile: value val[e] (VT double or float; uint8_t: the value's
-// index in a table of at most 256, for matrices of few different values); its
-// column and tile row stored one of
-// four ways (KEY):
+// Entry e of a tile: value val[e] (VT double or float; uint8_t or SmallRef: the
+// value's index in a table of at most 256, for matrices of few different
+// values); its column and tile row stored one of four ways (KEY):
 //  * KEY_SPLIT: col[e] and lrow[e];
 //  * KEY_PACKED: one word key[e] = offset << rbits | row, the column being
 //    (sbase[e >> 10] + offset) mod ncols: every run of 1024 entries has a
@@ -151,9 +150,15 @@ struct RctEntries {
     }
 };
 
+// uint8_t's form for small matrices: the tile kernel reads the table where it
+// lies, in the vector L1, and not from a copy in LDS, where a read waits behind
+// the LDS adds of the round before (see RctArgs::pal_lds).
+enum class SmallRef : uint8_t {};
+
 template <class VT>
-__device__ __forceinline__ double entry_value(VT v, const double *table) {
-    if constexpr (sizeof(VT) == 1) return table[v];
+__device__ __forceinline__ double entry_value(VT v, const double *table, const double *pal) {
+    if constexpr (std::is_same_v<VT, SmallRef>) return pal[uint32_t(v)];
+    else if constexpr (sizeof(VT) == 1) return table[v];
     else return double(v);
 }
 
@@ -241,8 +246,9 @@ __global__ void __launch_bounds__(1024) rct_kernel(RctArgs a, const double *__re
     const uint32_t tid = threadIdx.x, nt = blockDim.x;
     const uint32_t row0 = tile.row0, rows = tile.rows;
     double *xs = yl + a.R;  // VB: xr of the tile's rows
-    __shared__ double table[sizeof(VT) == 1 ? 256 : 1];
-    if constexpr (sizeof(VT) == 1)
+    constexpr bool TABLE = std::is_same_v<VT, uint8_t>;
+    __shared__ double table[TABLE ? 256 : 1];
+    if constexpr (TABLE)
         for (uint32_t k = tid; k < 256; k += nt) table[k] = a.pal[k];
     for (uint32_t k = tid; k < rows; k += nt) {
         yl[k] = 0.0;
@@ -320,8 +326,8 @@ __global__ void __launch_bounds__(1024) rct_kernel(RctArgs a, const double *__re
             }
 #pragma unroll
             for (int j = 0; j < UP; ++j) {
-                vv[j][0] = entry_value(S.v[j][0], table);
-                vv[j][1] = entry_value(S.v[j][1], table);
+                vv[j][0] = entry_value(S.v[j][0], table, a.pal);
+                vv[j][1] = entry_value(S.v[j][1], table, a.pal);
             }
         };
         auto add = [&](const PSet &S, const double (&xv)[UP][2], const double (&xl)[UP][2], const double (&vv)[UP][2]) {
@@ -688,11 +694,15 @@ hipError_t rct(const RctArgs &a, const double *x, double *y, hipStream_t s, hipE
         else                                                                                                      \
             rct_kernel<VT, P, true, false, false, UP><<<grid, a.block, lds, s>>>(a, x, y, xr, vbar, rb, res);     \
     } while (0)
-#define AX_RCT_LAUNCH(VT, P)                                                                              \
+    // (small matrices have neither 24-bit keys nor non-temporal loads, and
+    // their plans with heavy rows take the table in LDS)
+#define AX_RCT_LAUNCH(T, P)                                                                               \
     do {                                                                                                  \
-        constexpr bool nt = P != KEY_PACKED24;                                                            \
+        constexpr bool small = std::is_same_v<T, SmallRef>, nt = P != KEY_PACKED24 && !small;             \
+        using HVT = std::conditional_t<small, uint8_t, T>;                                                \
+        using VT = std::conditional_t<P == KEY_PACKED24, HVT, T>;                                         \
         if (P != KEY_DIAG && a.nhb)                                                                       \
-            rct_kernel<VT, P == KEY_DIAG ? KEY_SPLIT : P, false, false, true><<<grid, a.block, lds, s>>>( \
+            rct_kernel<HVT, P == KEY_DIAG ? KEY_SPLIT : P, false, false, true><<<grid, a.block, lds, s>>>( \
                 a, x, y, xr, vbar, rb, res);                                                              \
         else if (vb && vb_pairs(a) == 2)                                                                  \
             AX_RCT_VB(VT, P, nt, 2);                                                                      \
@@ -706,18 +716,20 @@ hipError_t rct(const RctArgs &a, const double *x, double *y, hipStream_t s, hipE
             rct_kernel<VT, P, false, false><<<grid, a.block, lds, s>>>(a, x, y, xr, vbar, rb, res);       \
     } while (0)
     auto with = [&](auto vt) {
-        using VT = decltype(vt);
+        using V = decltype(vt);
         if (km == KEY_DIAG)
-            AX_RCT_LAUNCH(VT, KEY_DIAG);
+            AX_RCT_LAUNCH(V, KEY_DIAG);
         else if (km == KEY_PACKED24)
-            AX_RCT_LAUNCH(VT, KEY_PACKED24);
+            AX_RCT_LAUNCH(V, KEY_PACKED24);
         else if (km == KEY_PACKED)
-            AX_RCT_LAUNCH(VT, KEY_PACKED);
+            AX_RCT_LAUNCH(V, KEY_PACKED);
         else
-            AX_RCT_LAUNCH(VT, KEY_SPLIT);
+            AX_RCT_LAUNCH(V, KEY_SPLIT);
     };
-    if (a.pal)
+    if (a.pal && a.pal_lds)
         with(uint8_t());
+    else if (a.pal)
+        with(SmallRef());
     else if (a.vtype == 1)
         with(float());
     else

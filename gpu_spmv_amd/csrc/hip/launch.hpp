@@ -117,6 +117,7 @@ struct RctArgs {
     // a matrix of at most 256 different values: val holds a byte per entry,
     // the index of its value in pal (256 doubles)
     const double *pal = nullptr;
+    uint32_t pal_lds = 0;  // 1: the tile kernel reads the table from a copy in LDS
     // rows of many entries kept apart (nhb > 0; not with key16 or partials):
     // nheavy rows listed in hrows (and marked in hmask, a bit per row; their
     // rows of the row blocks hold no entries), cut into nhb blocks (hb_start,

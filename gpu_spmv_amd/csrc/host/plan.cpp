@@ -895,8 +895,8 @@ std::vector<uint32_t> heavy_rows(const axspmv_csr *a) {
 // value instead of 8 (or 4), and a matrix of other values is told apart after
 // a few hundred of them.  SpMV, FP64, 12 / 5 B per entry, one box: 100^3
 // stencil renumbered 90 / 79 us, 90^3 in natural order 43 / 35, permuted 110^3
-// 179 / 141, the 1000^2 Laplacian 14.5 / 11.8, the 256^2 one launch-bound and
-// level.
+// 179 / 141, the 1000^2 Laplacian 14.5 / 11.8; below about 2M entries the gain
+// is gone (the 256^2 Laplacian by single calls 6.6 / 6.3, in a graph 3.2 / 3.3).
 bool value_table(const double *val, uint64_t n, bool f32, std::vector<double> &table, std::vector<uint8_t> &idx) {
     constexpr uint32_t SLOTS = 1024;  // open addressing over the values' bits
     std::vector<uint64_t> bits(SLOTS);
@@ -1330,6 +1330,14 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
     // 89 us).  Plans with heavy rows, which are for SpMM, have no such kernel:
     // their SpMV loads the ordinary way.
     p.rct.pal = dpal;
+    // The table's copy in LDS costs its fill and reads that queue behind the
+    // LDS adds; small matrices, whose stream is cached anyway, read it from the
+    // vector L1 (graph-timed, no table / copy in LDS / from L1: 256^2 Laplacian
+    // 3.18 / 3.54 / 3.31 us, 1000^2 14.7 / 11.6 / 12.3, +-1 on power-law
+    // patterns of 5,000 rows 6.2 / 7.3 / 6.3, of 50,000 7.2 / 7.6 / 7.3, of
+    // 100,000 (2.05M entries) 12.0 / 9.9 / 9.8, of 400,000 30.4 / 26.5 / 28.0,
+    // permuted 40^3 stencil (1.64M) 8.3 / 7.3 / 7.4).
+    p.rct.pal_lds = nnz >= (1u << 21);
     p.rct.nt_stream = !nhb && (vbytes + kbytes) * nnz > (256ull << 20) ? 1 : 0;
     p.rct.key16 = dk16;
     p.rct.key24 = dk24;

@@ -860,3 +860,28 @@ def test_axt_row_order_for_want_of_memory_is_no_error():
         p.spmv(dx, dy)
         ax._lib.call("axspmv_device_sync")
     assert rel_err(orc.ncsr(m, x), dy.download(np.float64, m.nrows)) <= TOL
+
+
+@pytest.mark.parametrize("vtype", [ax.F64, ax.F32])
+@pytest.mark.parametrize("nnz", [999, (1 << 21) - 1, 1 << 21, (1 << 21) + 1])
+def test_rct_value_table_in_lds_or_not(nnz, vtype):
+    """The tile kernel reads the values' table from memory below 2^21 entries
+    and from LDS from there on: product, forward + adjoint, value gradient."""
+    n, nc = max(nnz // 20, 50), max(nnz // 20, 40)
+    rng = np.random.default_rng(nnz)
+    row = np.concatenate([[0], np.sort(rng.integers(0, nnz + 1, n - 1)), [nnz]]).astype(np.uint32)
+    m = ax.CsrMatrix(row, rng.integers(0, nc, nnz).astype(np.uint32), rng.choice(rng.standard_normal(200), nnz), ncols=nc)
+    p = ax.Plan(m, ax.FMT_RCT, vtype=vtype, flags=ax.PLAN_TRANSPOSE)
+    vs = 8 if vtype == ax.F64 else 4
+    plain = ax.Plan(ax.CsrMatrix(m.row, m.col, rng.standard_normal(nnz), ncols=nc), ax.FMT_RCT, vtype=vtype)
+    assert plain.info()["stream_bytes"] - p.info()["stream_bytes"] == (vs - 1) * nnz
+    mv = m if vtype == ax.F64 else ax.CsrMatrix(m.row, m.col, m.val.astype(np.float32).astype(np.float64), ncols=nc)
+    x, b = ax.uniform(43, nc), ax.uniform(44, n)
+    assert rel_err(orc.ncsr(mv, x), ax.spmv_host(p, x)) <= TOL
+    dx, db = ax.DeviceBuffer.from_array(x), ax.DeviceBuffer.from_array(b)
+    dy, dr, dxb, dv = (ax.DeviceBuffer.from_array(np.full(s, np.nan)) for s in (n, n, nc, nnz))
+    p.fwd_adj(dx, db, dy, dr, dxb, dv)
+    r = dr.download(np.float64, n)
+    assert rel_err(orc.ncsr(mv, x) - b, r) <= TOL
+    assert rel_err(orc.ncsr_t(mv, r, nc), dxb.download(np.float64, nc)) <= TOL
+    assert np.array_equal(p.vbar_csr(dv.download(np.float64, nnz)), orc.vbar(m, r, x))
