@@ -22,8 +22,30 @@ namespace {
 using namespace axspmv::dev;
 using axspmv::launch::K1Item;
 
-// NT: val and col are streamed with non-temporal loads.
-template <class VT, bool NT>
+// NT: val and col are streamed with non-temporal loads.  MODE (launch::K1Mode):
+//
+//  * K1_LONG: steps 8 at a time, the values and columns of the next 8 in
+//    flight while the x gathers of these are waited for (a chunk is one chain
+//    of steps, and a small matrix has few chunks per SIMD to hide it behind).
+//    Steps past the end re-read the item's last one and add nothing.  Against
+//    K1_FAR's way: random rows of 4 to 40 entries, 20,001 rows 8.3 -> 7.2 us
+//    in a graph, 300,007 rows, FP32 values, 41.3 -> 37.4; 100,001-row
+//    power-law matrix 36.4 -> 28.5; 400,001 banded rows of 10 22.7 -> 18.4;
+//    permuted 90^3 stencil renumbered 84 -> 71.
+//  * K1_SHORT, rows of up to 6 entries on average: 4 at a time, none loaded
+//    past the end (8 at a time take 8 steps' loads and 66 to 80 registers for
+//    5 steps).  K1_FAR / K1_LONG / this: 700^2 Laplacian, FP32 values, in a
+//    graph 6.5 / 7.4 / 6.3 us, 1400^2 35.6 / 33.6 / 31.9, 400,001 banded rows of
+//    5 14.4 / 12.6 / 12.8, of 2.7 10.2 / 9.5 / 9.2.
+//  * K1_FAR, rows of up to 12 entries that gather without locality from an x
+//    larger than an L2: 4 at a time, the next 4 not before these are added.
+//    More loads in flight gain nothing there.  Random, this / K1_LONG: 540,001
+//    rows of 0 to 9 21.6 / 23.4 us, 700,001 30.8 / 34.0 (K1_SHORT 33.6),
+//    1,500,001 101 / 105; 700,001 of 0 to 16 46.1 / 50.9, of 4 to 16 65.2 / 65.2
+//    (in a graph 55.7 / 61.1), of 8 to 24 95.4 / 93.3, FP32 values in a graph
+//    75.4 / 80.9.
+using axspmv::launch::K1Mode;
+template <class VT, bool NT, K1Mode MODE>
 __global__ void __launch_bounds__(256) k1_kernel(const K1Item *__restrict__ items, uint32_t nitems, uint32_t chunk,
                                                  const VT *__restrict__ val, const uint32_t *__restrict__ col,
                                                  const uint32_t *__restrict__ permi, uint32_t nrows,
@@ -38,31 +60,48 @@ __global__ void __launch_bounds__(256) k1_kernel(const K1Item *__restrict__ item
     const uint32_t r = lane % chunk;
     const uint32_t gid = w.chunk * chunk + r;
     const uint64_t base = uint64_t(w.chp) + r;
-    // Steps U at a time: the values and columns of the next U steps are in
-    // flight while the x gathers of these are waited for (a chunk is one
-    // chain of steps, and a small matrix has few chunks per SIMD to hide it
-    // behind).  Steps past the end re-read the item's last one and add
-    // nothing.  Against 4 steps without prefetch: random rows of 4 to 40
-    // entries, 20,001 rows 14.6 -> 7.8 us, 300,007 rows, FP32 values, 41.3 ->
-    // 37.4 (their x gathers alone take 28); 50,000-row power-law matrix 34.6 ->
-    // 24.3; permuted 80^3 stencil renumbered 61.0 -> 53.6.
-    constexpr uint32_t U = 8;
     double acc = 0.0;
-    VT v[U];
-    uint32_t c[U];
-    auto half = [&](uint32_t j, uint32_t u0) {
+    if constexpr (MODE == K1Mode::K1_FAR) {
+        uint32_t j = w.j0;
+        for (; j + 4 <= w.j1; j += 4) {
+            const uint64_t q = base + uint64_t(j) * chunk;
+            VT v[4];
+            double xv[4];
 #pragma unroll
-        for (uint32_t u = u0; u < u0 + U / 2; ++u) {
-            const uint64_t q = base + uint64_t(min(j + u, w.j1 - 1)) * chunk;
+            for (uint32_t u = 0; u < 4; ++u) {
+                v[u] = stream_load<NT>(val + q + u * chunk);
+                xv[u] = xpad(x, stream_load<NT>(col + q + u * chunk));
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) acc = fma(double(v[u]), xv[u], acc);
+        }
+        for (; j < w.j1; ++j) {
+            const uint64_t q = base + uint64_t(j) * chunk;
+            acc = fma(double(stream_load<NT>(val + q)), xpad(x, stream_load<NT>(col + q)), acc);
+        }
+    } else if (w.j0 < w.j1) {
+        constexpr uint32_t U = MODE == K1Mode::K1_LONG ? 8 : 4;
+        VT v[U];
+        uint32_t c[U];
+        auto step = [&](uint32_t j, uint32_t u) {
+            const uint64_t q = base + uint64_t(j) * chunk;
             v[u] = stream_load<NT>(val + q);
             c[u] = stream_load<NT>(col + q);
-        }
-    };
-    auto fetch = [&](uint32_t j) {
-        half(j, 0);
-        if (j + U / 2 < w.j1) half(j, U / 2);
-    };
-    if (w.j0 < w.j1) {
+        };
+        auto half = [&](uint32_t j, uint32_t u0) {
+#pragma unroll
+            for (uint32_t u = u0; u < u0 + U / 2; ++u) step(min(j + u, w.j1 - 1), u);
+        };
+        auto fetch = [&](uint32_t j) {
+            if constexpr (MODE == K1Mode::K1_LONG) {
+                half(j, 0);
+                if (j + U / 2 < w.j1) half(j, U / 2);
+            } else {
+#pragma unroll
+                for (uint32_t u = 0; u < U; ++u)
+                    if (j + u < w.j1) step(j + u, u);
+            }
+        };
         fetch(w.j0);
         for (uint32_t j = w.j0; j < w.j1; j += U) {
             double xv[U], vv[U];
@@ -155,12 +194,15 @@ template <class VT>
 hipError_t k1_vt(const axspmv::launch::K1Args &a, const double *x, double *y, hipStream_t s) {
     const uint32_t per_wave = 64 / a.chunk;
     const uint32_t waves = (a.nitems + per_wave - 1) / per_wave;
-    if (waves && a.nt)
-        k1_kernel<VT, true><<<(waves + 3) / 4, 256, 0, s>>>(a.items, a.nitems, a.chunk, static_cast<const VT *>(a.val),
-                                                            a.col, a.permi, a.nrows, x, y, a.part);
-    else if (waves)
-        k1_kernel<VT, false><<<(waves + 3) / 4, 256, 0, s>>>(a.items, a.nitems, a.chunk, static_cast<const VT *>(a.val),
-                                                             a.col, a.permi, a.nrows, x, y, a.part);
+    auto run = [&](auto kernel) {
+        kernel<<<(waves + 3) / 4, 256, 0, s>>>(a.items, a.nitems, a.chunk, static_cast<const VT *>(a.val), a.col, a.permi,
+                                               a.nrows, x, y, a.part);
+    };
+    if (waves) switch (a.mode) {
+        case K1Mode::K1_LONG: a.nt ? run(k1_kernel<VT, true, K1Mode::K1_LONG>) : run(k1_kernel<VT, false, K1Mode::K1_LONG>); break;
+        case K1Mode::K1_SHORT: a.nt ? run(k1_kernel<VT, true, K1Mode::K1_SHORT>) : run(k1_kernel<VT, false, K1Mode::K1_SHORT>); break;
+        case K1Mode::K1_FAR: a.nt ? run(k1_kernel<VT, true, K1Mode::K1_FAR>) : run(k1_kernel<VT, false, K1Mode::K1_FAR>); break;
+    }
     if (a.nsplit) {
         const uint32_t th = a.nsplit * a.chunk;
         k1_fixup<<<(th + 255) / 256, 256, 0, s>>>(a.split, a.nsplit, a.chunk, a.permi, a.nrows, a.part, y);

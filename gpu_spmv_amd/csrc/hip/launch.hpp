@@ -184,6 +184,8 @@ hipError_t csr_vector(uint32_t nrows, const void *val, uint32_t vtype, const uin
 struct K1Item {
     uint32_t chunk, chp, j0, j1, slot;
 };
+// How a K1 item's steps are loaded (k_k1_axc.hip); the sums are the same.
+enum class K1Mode : uint32_t { K1_LONG, K1_SHORT, K1_FAR };
 struct K1Args {
     const K1Item *items;
     uint32_t nitems;
@@ -194,6 +196,7 @@ struct K1Args {
     const uint32_t *col, *permi;
     double *part;
     uint32_t nt = 0;  // 1: val and col streamed with non-temporal loads
+    K1Mode mode = K1Mode::K1_LONG;
 };
 hipError_t k1(const K1Args &a, const double *x, double *y, hipStream_t s);
 

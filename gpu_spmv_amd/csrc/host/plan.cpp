@@ -759,6 +759,13 @@ int plan_k1(Plan &p, const axspmv_csr *a, hipStream_t s) {
     // 128^3 stencil 740 -> 719.6 us, the same renumbered by reverse
     // Cuthill-McKee 209.2 -> 193.2 us.
     p.k1.nt = p.stream_bytes > (128ull << 20) ? 1 : 0;
+    // Short rows: fewer steps in flight (the kernel's comment has both sides).
+    // x of more than 4 MB, an L2, is where scattered gathers leave it.
+    const uint64_t n = a->nrows;
+    if (a->nnz <= 12 * n && a->ncols > (4u << 20) / 8 && scattered(a))
+        p.k1.mode = launch::K1Mode::K1_FAR;
+    else if (a->nnz <= 6 * n)
+        p.k1.mode = launch::K1Mode::K1_SHORT;
     p.launches = split.empty() ? 1 : 2;
     p.nblocks = uint32_t(items.size());
     p.kind = Plan::K1;

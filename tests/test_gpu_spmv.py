@@ -885,3 +885,26 @@ def test_rct_value_table_in_lds_or_not(nnz, vtype):
     assert rel_err(orc.ncsr(mv, x) - b, r) <= TOL
     assert rel_err(orc.ncsr_t(mv, r, nc), dxb.download(np.float64, nc)) <= TOL
     assert np.array_equal(p.vbar_csr(dv.download(np.float64, nnz)), orc.vbar(m, r, x))
+
+
+@pytest.mark.parametrize("vtype", [ax.F64, ax.F32])
+@pytest.mark.parametrize("chunk,reorder", [(64, 1), (64, 0), (16, 1), (1, 1)])
+@pytest.mark.parametrize("most,ncols", [(3, 600), (11, 600), (24, 600), (48, 600), (3, 700001), (23, 700001), (48, 700001)],
+                         ids=["short3", "short11", "short24", "long", "far3", "far23", "long_far"])
+def test_k1_step_loads(most, ncols, chunk, reorder, vtype):
+    """Every way of loading a K1 item's steps, at step counts around its
+    groups of 4 and 8, with empty rows and a few rows split over several
+    items; the same order of terms in all of them."""
+    n = 3001
+    rng = np.random.default_rng(most + ncols)
+    lens = rng.integers(0, most + 1, n)
+    lens[[5, 2000]] = 300, 65
+    row = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    m = ax.CsrMatrix(row, rng.integers(0, ncols, int(row[-1])).astype(np.uint32), rng.standard_normal(int(row[-1])), ncols=ncols)
+    x = ax.uniform(45, ncols)
+    x[m.col[row[1000]]] = np.inf
+    ref = (orc.ncsr_f32val if vtype == ax.F32 else orc.ncsr)(m, x)
+    y = ax.spmv_host(ax.Plan(m, ax.FMT_K1, chunk=chunk, reorder=reorder, vtype=vtype), x)
+    fin = np.isfinite(ref)
+    np.testing.assert_array_equal(y[~fin], ref[~fin])
+    assert rel_err(ref[fin], y[fin]) <= TOL
