@@ -22,13 +22,13 @@ __global__ void __launch_bounds__(256) csr_naive_kernel(uint32_t nrows, const VT
     y[r] = acc;
 }
 
-// NT: val and col are streamed with non-temporal loads.
-template <class VT, int G, bool NT>
+// NT: val and col are streamed with non-temporal loads.  R: rows of a group at
+// once (rows_per_group).
+template <class VT, int G, bool NT, uint32_t R>
 __global__ void __launch_bounds__(256) csr_vector_kernel(uint32_t nrows, const VT *__restrict__ val,
                                                          const uint32_t *__restrict__ col,
                                                          const uint32_t *__restrict__ row, uint32_t long_len,
                                                          const double *__restrict__ x, double *__restrict__ y) {
-    constexpr uint32_t R = rows_per_group(G);
     const size_t gl = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (gl / G * R >= nrows) return;  // whole groups leave together (G divides 64)
     const uint32_t r = uint32_t(gl / G) * R, g = uint32_t(gl % G);
@@ -78,18 +78,23 @@ template <class VT, bool NT>
 hipError_t csr_vector_vt(uint32_t nrows, const VT *val, const uint32_t *col, const uint32_t *row, uint32_t lanes,
                          uint32_t long_len, const uint32_t *longrows, uint32_t nlong, const double *x, double *y,
                          hipStream_t s) {
-    const uint32_t rows = rows_per_group(lanes);
+    const uint32_t rows = rows_per_group(lanes, nrows);
     const unsigned grid = unsigned(((uint64_t(nrows) + rows - 1) / rows * lanes + 255) / 256);
     switch (lanes) {
 #define AX_G_CASE(G) \
-    case G: csr_vector_kernel<VT, G, NT><<<grid, 256, 0, s>>>(nrows, val, col, row, long_len, x, y); break;
+    case G: csr_vector_kernel<VT, G, NT, 1><<<grid, 256, 0, s>>>(nrows, val, col, row, long_len, x, y); break;
         AX_G_CASE(1)
         AX_G_CASE(2)
         AX_G_CASE(4)
         AX_G_CASE(8)
         AX_G_CASE(16)
-        AX_G_CASE(32)
         AX_G_CASE(64)
+        case 32:
+            if (rows == 2)
+                csr_vector_kernel<VT, 32, NT, 2><<<grid, 256, 0, s>>>(nrows, val, col, row, long_len, x, y);
+            else
+                csr_vector_kernel<VT, 32, NT, 1><<<grid, 256, 0, s>>>(nrows, val, col, row, long_len, x, y);
+            break;
 #undef AX_G_CASE
         default: return hipErrorInvalidValue;
     }

@@ -138,12 +138,11 @@ __global__ void __launch_bounds__(256) k1_fixup(const uint32_t *__restrict__ spl
 
 // AXC: G lanes per row; rows listed in `longrows` are skipped here and done
 // by axc_long (one wave per row).
-template <class VT, int G, bool NT>
+template <class VT, int G, bool NT, uint32_t R>
 __global__ void __launch_bounds__(256) axc_kernel(uint32_t nrows, const uint32_t *__restrict__ brp,
                                                   const VT *__restrict__ vp, const uint32_t *__restrict__ mapx,
                                                   uint32_t long_slots, const double *__restrict__ x,
                                                   double *__restrict__ y) {
-    constexpr uint32_t R = rows_per_group(G);
     const size_t gl = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (gl / G * R >= nrows) return;  // whole groups leave together (G divides 64)
     const uint32_t r = uint32_t(gl / G) * R, g = uint32_t(gl % G);
@@ -213,18 +212,23 @@ hipError_t k1_vt(const axspmv::launch::K1Args &a, const double *x, double *y, hi
 template <class VT, bool NT>
 hipError_t axc_vt(const axspmv::launch::AxcArgs &a, const double *x, double *y, hipStream_t s) {
     const VT *vp = static_cast<const VT *>(a.vplane);
-    const uint32_t rows = rows_per_group(a.hbs);
+    const uint32_t rows = rows_per_group(a.hbs, a.nrows);
     const unsigned grid = unsigned(((uint64_t(a.nrows) + rows - 1) / rows * a.hbs + 255) / 256);
     if (a.nrows) switch (a.hbs) {
 #define AX_G(G) \
-    case G: axc_kernel<VT, G, NT><<<grid, 256, 0, s>>>(a.nrows, a.brp, vp, a.mapx, a.long_slots, x, y); break;
+    case G: axc_kernel<VT, G, NT, 1><<<grid, 256, 0, s>>>(a.nrows, a.brp, vp, a.mapx, a.long_slots, x, y); break;
         AX_G(1)
         AX_G(2)
         AX_G(4)
         AX_G(8)
         AX_G(16)
-        AX_G(32)
         AX_G(64)
+        case 32:
+            if (rows == 2)
+                axc_kernel<VT, 32, NT, 2><<<grid, 256, 0, s>>>(a.nrows, a.brp, vp, a.mapx, a.long_slots, x, y);
+            else
+                axc_kernel<VT, 32, NT, 1><<<grid, 256, 0, s>>>(a.nrows, a.brp, vp, a.mapx, a.long_slots, x, y);
+            break;
 #undef AX_G
         default: return hipErrorInvalidValue;
     }

@@ -73,8 +73,13 @@ __device__ __forceinline__ double strided_dot(const VT *__restrict__ val, const 
 // and the waves' own cost shows (the 80^3 stencil in natural order, CSR / AXC
 // 67.3 -> 52.6 / 71.7 -> 56.1 us; four rows take 48.5 / 50.9 there but lose 4 %
 // on random rows of 20 to 46 entries); with 64 lanes two lost 8 % on rows of
-// 60 to 90 entries, with fewer a group has four terms in flight already.
-__host__ __device__ constexpr uint32_t rows_per_group(uint32_t G) { return G == 32 ? 2 : 1; }
+// 60 to 90 entries, with fewer a group has four terms in flight already.  One
+// on matrices of under 32,768 rows, where the second row halves the waves of a
+// chip that two rows a wave fill once or twice (CSR vector, graph-timed, one /
+// two rows: banded rows of 38 entries, 5,001 rows 2.49 / 2.90 us, 10,001 2.79 /
+// 3.17, 20,001 3.84 / 4.04, 30,001 4.85 / 4.86, 60,001 9.64 / 8.56; random rows
+// of 20 to 46, 10,001 rows 3.31 / 3.61, 100,001 21.4 / 20.9).
+inline uint32_t rows_per_group(uint32_t G, uint32_t nrows) { return G == 32 && nrows >= 32768 ? 2 : 1; }
 
 // R rows at once: acc[i] = the sum of val[j] x[col[j]] over j = b[i] + g, b[i] +
 // g + stride, ... < e[i], term by term with the R rows' loads in flight

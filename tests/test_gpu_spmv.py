@@ -908,3 +908,25 @@ def test_k1_step_loads(most, ncols, chunk, reorder, vtype):
     fin = np.isfinite(ref)
     np.testing.assert_array_equal(y[~fin], ref[~fin])
     assert rel_err(ref[fin], y[fin]) <= TOL
+
+
+@pytest.mark.parametrize("fmt,kw", [(ax.FMT_CSR, dict(kernel=ax.KER_STREAM, hbs=32)), (ax.FMT_AXC, dict(hbs=32)),
+                                    (ax.FMT_AXC, dict(hbs=32, vtype=ax.F32))], ids=["csr", "axc", "axc_f32"])
+@pytest.mark.parametrize("nrows", [32767, 32768, 32769])
+@pytest.mark.parametrize("last", [0, 33, 5000])
+def test_one_or_two_rows_per_group(fmt, kw, nrows, last):
+    """32 lanes per row: one row at once below 32,768 rows, two from there on;
+    an odd last row, empty rows, long rows next to short ones."""
+    rng = np.random.default_rng(nrows + last)
+    lens = rng.integers(0, 70, nrows)
+    lens[[0, 1, 100]] = 4000, 0, 4000
+    lens[-1] = last
+    row = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    nc = 9000
+    m = ax.CsrMatrix(row, rng.integers(0, nc, int(row[-1])).astype(np.uint32), rng.standard_normal(int(row[-1])), ncols=nc)
+    x = ax.uniform(46, nc)
+    ref = (orc.ncsr_f32val if kw.get("vtype") == ax.F32 else orc.ncsr)(m, x)
+    dx, dy = ax.DeviceBuffer.from_array(x), ax.DeviceBuffer.from_array(np.full(nrows + 1, np.nan))
+    ax.Plan(m, fmt, **kw).spmv(dx, dy)
+    y = dy.download(np.float64, nrows + 1)
+    assert np.isnan(y[-1]) and rel_err(ref, y[:-1]) <= TOL
