@@ -542,10 +542,16 @@ bool scattered(const axspmv_csr *a) {
 // 750,000 129.6 / 120.7 (121.0 / 92.6), 2^20 209.5 / 163.0, 3M 920 / 550;
 // permuted 100^3 stencil 270 / 194; random, 10^6 rows of 6 74.4 / 61.6.  Below
 // two entries: 2M rows of 2 72.7 / 81.8; 4M of 5, 4 slices 350 / 328, 8 slices
-// 350 (so 2).
+// 350 (so 2).  Few entries read few lines of x twice, whatever the slices, and
+// a launch each is all that those add (20,001 rows of 20 of 700,001 columns 7.3
+// / 10.1 us, 3,001 of 300 of 5M 18.6 / 36.5, 150,001 of 9 of 3M 25.0 / 31.1):
+// none under 1.4M.  Up to about 2.5M, matrices of more columns than rows still
+// lose a little (300,001 of 5 of 700,001 18.4 / 18.8, 150,001 of 20 of 3M 50.9 /
+// 56.3; 100,001 of 40 of 700,001 35.2 / 31.5); plans there keep the layout, and
+// the order of additions, that they had.
 uint32_t axt_slices(const axspmv_csr *a) {
     constexpr uint64_t SLICE = (4ull << 20) / 8;
-    if (a->ncols < 5 * SLICE / 4 || !a->nnz) return 1;
+    if (a->ncols < 5 * SLICE / 4 || a->nnz < 1400000) return 1;
     uint32_t S = 2;
     while (S < 8 && ceil_div(a->ncols, S) > SLICE) S *= 2;
     while (S > 1 && a->nnz < 2ull * S * a->nrows) S /= 2;

@@ -290,8 +290,9 @@ typedef struct axspmv_opts {
                            between runs).  SpMV and the adjoint only.  1 =
                            one layout, with the caller's thw.  0 = one
                            layout, and where x is larger than 5 MB and the
-                           rows read it without locality (two entries per
-                           row and slice at least) the matrix once more in 2,
+                           rows read it without locality (1.4M entries, and
+                           two per row and slice, at least) the matrix once
+                           more in 2,
                            4 or 8 column slices of 2 or 4 slots per tile, on
                            which SpMV and the adjoint run one slice after
                            another, without atomics: about twice the device

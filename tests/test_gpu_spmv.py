@@ -930,3 +930,18 @@ def test_one_or_two_rows_per_group(fmt, kw, nrows, last):
     ax.Plan(m, fmt, **kw).spmv(dx, dy)
     y = dy.download(np.float64, nrows + 1)
     assert np.isnan(y[-1]) and rel_err(ref, y[:-1]) <= TOL
+
+
+@pytest.mark.parametrize("n,ncols,per,launches", [
+    (20001, 700001, 20, 1), (3001, 5000001, 300, 1), (46666, 700001, 30, 1),   # 1,399,980 entries at most
+    (46667, 700001, 30, 2), (46667, 1500001, 30, 4)])
+def test_axt_few_entries_in_one_piece(n, ncols, per, launches):
+    """Few entries of a wide matrix are not cut into column slices: a launch
+    per slice would be all that they add."""
+    rng = np.random.default_rng(n)
+    row = (np.arange(n + 1) * per).astype(np.uint32)
+    m = ax.CsrMatrix(row, rng.integers(0, ncols, n * per).astype(np.uint32), rng.standard_normal(n * per), ncols=ncols)
+    p = ax.Plan(m, ax.FMT_AXT)
+    assert p.info()["launches"] == launches
+    x = ax.uniform(47, ncols)
+    assert rel_err(orc.ncsr(m, x), ax.spmv_host(p, x)) <= TOL
