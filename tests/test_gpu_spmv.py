@@ -945,3 +945,20 @@ def test_axt_few_entries_in_one_piece(n, ncols, per, launches):
     assert p.info()["launches"] == launches
     x = ax.uniform(47, ncols)
     assert rel_err(orc.ncsr(m, x), ax.spmv_host(p, x)) <= TOL
+
+
+@pytest.mark.parametrize("n", [4000, 4001, (1 << 19) - 1, (1 << 19) + 1])
+def test_rct_merge_of_odd_rows(n):
+    """The merge of slice partials, one row per lane or two, with the residual
+    and the clear of x_bar."""
+    m = _uneven(n, 3, 5001, seed=n)
+    p = ax.Plan(m, ax.FMT_RCT, flags=ax.PLAN_TRANSPOSE, slices=4, tile_rows=8192)
+    assert not p.info()["name"].endswith("_atomic")
+    x, b = ax.uniform(48, 5001), ax.uniform(49, n)
+    dx, db = ax.DeviceBuffer.from_array(x), ax.DeviceBuffer.from_array(b)
+    dy, dr, dxb, dv = (ax.DeviceBuffer.from_array(np.full(s + 1, np.nan)) for s in (n, n, 5001, m.nnz))
+    p.fwd_adj(dx, db, dy, dr, dxb, dv)
+    y, r, xb = (d.download(np.float64, s + 1) for d, s in ((dy, n), (dr, n), (dxb, 5001)))
+    assert np.isnan(y[-1]) and np.isnan(r[-1]) and np.isnan(xb[-1])
+    assert rel_err(orc.ncsr(m, x), y[:-1]) <= TOL and np.array_equal(r[:-1], y[:-1] - b)
+    assert rel_err(orc.ncsr_t(m, r[:-1], 5001), xb[:-1]) <= TOL
