@@ -188,9 +188,9 @@ hipError_t run_kt(const axspmv::launch::SpmmArgs &a, uint32_t k, const double *X
 // Two right-hand sides per lane where every 16-byte access is aligned: k
 // even, X and Y 16-byte aligned.  X rows by 32-bit byte offsets where X is
 // under 4 GB.  Not at k-tile 8 where X rows are read without locality and
-// every row is short (a.far: X of 8 right-hand sides over 4 MB): groups of 4
-// lanes then keep 16 rows of a wave waiting for the slowest line, against 8.
-// One / two per lane, k = 8: permuted 66^3 stencil 133 / 149 us, 110^3 731 / 808,
+// every row is short (a.far: the k-tile's part of X, 64 bytes a row whatever k
+// is, over 4 MB): groups of 4 lanes then keep 16 rows of a wave waiting for the
+// slowest line, against 8.  One / two per lane, k = 8: permuted 66^3 stencil 133 / 149 us, 110^3 731 / 808,
 // 300,007 random rows 115 / 130; but natural 66^3 53.1 / 51.7, 200,000-row
 // power-law matrix (long rows) 98.6 / 92.4, permuted 40^3 (X of 4 MB) 17.7 / 16.9.
 template <class VT, int KT>

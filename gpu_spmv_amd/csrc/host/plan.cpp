@@ -1212,10 +1212,12 @@ int plan_rct(Plan &p, const axspmv_csr *a, hipStream_t s) {
     // comes from the caches and the third load costs more than the bytes (FP64
     // power-law matrix, 32 / 24 bits: 50,000 rows 9.3 / 9.5 us; random rows,
     // 150,001, FP32 15.0 / 15.8); between, the bytes count, most of all where
-    // they let the stream stay in the Infinity Cache (power-law, 400,000 rows
-    // 40.1 / 37.9 us; 2^20 rows 86.8 / 85.8, run again and again 59.8 / 54.7,
-    // FP32 78.3 / 74.9; random, 450,007 rows, FP32 38.5 / 33.3); above, with
-    // non-temporal loads, it is level or slightly behind (1.4M rows 160.0 / 161.0).
+    // they let the stream stay in the Infinity Cache (plans and vectors in
+    // turn: power-law, 400,003 rows 42.6 / 42.5 us, 600,000 52.4 / 51.6, 2^20 rows
+    // 86.8 / 85.9, FP32 78.0 / 75.1, forward + adjoint 212.8 / 209.5; random,
+    // 450,007 rows, FP32 45.6 / 44.1; SpMM, k = 8, 150.4 / 149.5; 2^20 rows run
+    // again and again 63.2 / 57.2); above, with non-temporal loads, it is level
+    // or slightly behind (1.4M rows 160.0 / 161.0).
     const uint64_t stream32 = nnz * (4 + vbytes);
     std::vector<uint32_t> sbase24;
     bool key24 = packed && !diag && rbits < 24 && !(p.o.flags & AXSPMV_PLAN_RCT_WIDE_KEY) &&
