@@ -40,10 +40,10 @@ using axspmv::launch::K1Item;
 //  * K1_FAR, rows of up to 12 entries that gather without locality from an x
 //    larger than an L2: 4 at a time, the next 4 not before these are added.
 //    More loads in flight gain nothing there.  Random, this / K1_LONG: 540,001
-//    rows of 0 to 9 21.6 / 23.4 us, 700,001 30.8 / 34.0 (K1_SHORT 33.6),
-//    1,500,001 101 / 105; 700,001 of 0 to 16 46.1 / 50.9, of 4 to 16 65.2 / 65.2
-//    (in a graph 55.7 / 61.1), of 8 to 24 95.4 / 93.3, FP32 values in a graph
-//    75.4 / 80.9.
+//    rows of 0 to 9 21.6 / 23.4 us, 700,001 30.7 / 34.0 (K1_SHORT 33.6), of 0 to
+//    16 45.1 / 50.9, 900,001 of 4 to 12 74.4 / 79.4, 1,200,001 of 9 to 13 146.8 /
+//    155.0, 600,001 of 10 to 14 66.2 / 62.4 (in a graph 52.9 / 55.4), 700,001 of 8
+//    to 24 95.4 / 93.3, FP32 values in a graph 75.4 / 80.9.
 using axspmv::launch::K1Mode;
 template <class VT, bool NT, K1Mode MODE>
 __global__ void __launch_bounds__(256) k1_kernel(const K1Item *__restrict__ items, uint32_t nitems, uint32_t chunk,
@@ -68,10 +68,9 @@ __global__ void __launch_bounds__(256) k1_kernel(const K1Item *__restrict__ item
             VT v[4];
             double xv[4];
 #pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) {
-                v[u] = stream_load<NT>(val + q + u * chunk);
-                xv[u] = xpad(x, stream_load<NT>(col + q + u * chunk));
-            }
+            for (uint32_t u = 0; u < 4; ++u) v[u] = stream_load<NT>(val + q + u * chunk);
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) xv[u] = xpad(x, stream_load<NT>(col + q + u * chunk));
 #pragma unroll
             for (uint32_t u = 0; u < 4; ++u) acc = fma(double(v[u]), xv[u], acc);
         }
